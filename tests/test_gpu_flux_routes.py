@@ -1,0 +1,71 @@
+"""The form-factor flux integrals take one of several kernels by their number
+(teams of 64, 16 or 8 lanes per integral, or one lane per integral with rows
+grouped by photon energy).  Every route runs the same dqagse arithmetic, so a
+point's luminosity must not depend on how many points were asked for with it:
+1e-11 relative between routes (the integrand may differ by rounding, which
+the contraction of these Pb-Pb points amplifies by less than 1e3), and 1e-9
+against the oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CFG = dict(flux_point=0, breakup_mode=2, nm=3, ny=3)
+NMAX = 1500  # 3000 rows: one lane per integral, last group of 64 rows partly filled
+
+
+@pytest.fixture(scope="module")
+def data(gpu):
+    import torch
+    rng = np.random.default_rng(77)
+    M = np.exp(rng.uniform(np.log(2.0), np.log(60.0), NMAX))
+    Y = rng.uniform(-3.5, 3.5, NMAX)
+    c = gpu.Context(**CFG)
+    t = lambda x: torch.as_tensor(x, device="cuda")
+    L = c.lumi_points(t(M), t(Y)).cpu().numpy()
+    return c, M, Y, L, c.info.qags_evals
+
+
+# one point; row groups of 64 and their neighbours; both sides of every change of route
+@pytest.mark.parametrize("n", [1, 14, 15, 31, 32, 33, 175, 176, 702, 703, 1499])
+def test_route_does_not_change_a_point(gpu, data, n):
+    import torch
+    c, M, Y, L, _ = data
+    t = lambda x: torch.as_tensor(x, device="cuda")
+    got = c.lumi_points(t(M[:n]), t(Y[:n])).cpu().numpy()
+    assert c.info.qags_bad == 0
+    assert np.max(np.abs(got - L[:n]) / np.abs(L[:n])) <= 1e-11
+
+
+def test_evaluation_counts_add_up(gpu, data):
+    """Every QAGS decision is the same on every route: the integrand
+    evaluations of the parts sum to those of the whole."""
+    import torch
+    c, M, Y, _, evals = data
+    t = lambda x: torch.as_tensor(x, device="cuda")
+    total = 0
+    for a, b in ((0, 14), (14, 189), (189, 500), (500, 1500)):
+        c.lumi_points(t(M[a:b].copy()), t(Y[a:b].copy()))
+        total += c.info.qags_evals
+    assert total == evals
+
+
+def test_points_against_oracle(data, oracle_ctx):
+    _, M, Y, L, _ = data
+    o = oracle_ctx(**CFG)
+    for i in (0, 1, 700, NMAX - 1):
+        assert abs(L[i] / o.lumi(M[i], Y[i]) - 1) <= 1e-9
+
+
+@pytest.mark.parametrize("n", [1, 2048, 2049, 24576, 24577, 98304, 98305])
+def test_flux_form_routes(gpu, data, n):
+    """Bit for bit: the per-point routes evaluate every node alike."""
+    import torch
+    c = data[0]
+    rng = np.random.default_rng(5)
+    b = torch.as_tensor(rng.uniform(0.3, 16.0, 98305), device="cuda")
+    k = torch.as_tensor(10 ** rng.uniform(-2.0, 2.5, 98305), device="cuda")
+    full, ier = c.flux_form(b, k)
+    got, ier_n = c.flux_form(b[:n].clone(), k[:n].clone())
+    assert torch.equal(got.view(torch.int64), full[:n].view(torch.int64))
+    assert torch.equal(ier_n, ier[:n])

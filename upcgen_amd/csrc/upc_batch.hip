@@ -5,10 +5,11 @@
 // UpcCrossSection::init + prepareTwoPhotonLumi (src/UpcCrossSection.cpp:
 // 116-137, 463-592).  Every job keeps its own context (tables: G_AA, form
 // factor, breakup), and the grid work of all jobs is concatenated:
-//   points [sum npts], flux rows [sum nrows][120], QAGS tasks [sum tasks].
+//   points [sum npts], flux rows [sum nrows][120].
 // One kernel per stage serves all jobs (a job table in HBM maps a point,
 // row or block to its job), so the QAGS integrals of every job share one
-// persistent launch and its task cursor, and the contraction is one launch.
+// persistent launch and its cursor (rows sorted by job, then by photon
+// energy), and the contraction is one launch.
 // The sequence is captured once into a hipGraph and replayed; buffers are
 // cleared by kernels (no memset nodes).  The launch shapes (QAGS workgroups
 // per CU, contraction waves per block) are chosen by timing the candidates
@@ -41,7 +42,12 @@ int mfma_read_counts(void* st, unsigned long long* h_out, hipStream_t s);
 
 constexpr int kLumiWaveChoices[3] = {2, 4, 8};
 constexpr int kMfmaTileChoices[3] = {1, 2, 4};  // column tiles per A-fragment load (MFMA form)
-constexpr int kQagsBlockChoices[3] = {1, 2, 3};  // workgroups of 256 per CU (3 fit its LDS)
+constexpr int kQagsBlockChoices[3] = {1, 2, 3};  // workgroups of 256 per CU; the last choice fills the CU
+static int qags_blocks_per_cu(int choice) { return choice == 2 ? kQagsRowsBlocksPerCu : kQagsBlockChoices[choice]; }
+
+// Buckets of the row sort: per job, 64 per octave of k.
+constexpr int kBatchPerOctave = 64;
+constexpr int kBatchBuckets = kRowOctaves * kBatchPerOctave;
 
 __device__ __forceinline__ int find_job(const int* __restrict__ start, int njobs, long idx)
 {
@@ -76,61 +82,89 @@ __global__ void k_batch_points(const BatchJob* __restrict__ jobs, const int* __r
   pts[4 * idx + 3] = dy;
 }
 
-__global__ void k_batch_rows(const BatchJob* __restrict__ jobs, const int* __restrict__ row0, int njobs, long total,
-                             double* __restrict__ row_k, double* __restrict__ row_logd, int* __restrict__ row_cnt)
+// Clears the batch's counters, its jobs' failure counts and the row histogram.
+__global__ void k_batch_clear(unsigned long long* __restrict__ counters, unsigned long long* __restrict__ job_failed,
+                              int njobs, int* __restrict__ hist, int nhist)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < 8) counters[i] = 0;
+  if (i < njobs) job_failed[i] = 0;
+  if (i < nhist) hist[i] = 0;
+}
+
+__device__ __forceinline__ int batch_bucket(int job, double k)
+{
+  return job * kBatchBuckets + row_bucket(k, kBatchPerOctave);
+}
+
+__global__ __launch_bounds__(256) void k_batch_rows(const BatchJob* __restrict__ jobs, const int* __restrict__ row0,
+                                                    int njobs, long total, double* __restrict__ row_k,
+                                                    double* __restrict__ row_logd, int* __restrict__ row_cnt,
+                                                    int* __restrict__ hist, unsigned long long* __restrict__ ntasks)
 {
   const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= total) return;
-  const BatchJob& J = jobs[find_job(row0, njobs, r)];
-  row_setup(J.v.pts, J.v.npts, (int)(r - J.row0), J.v.fp, &row_k[r], &row_logd[r], &row_cnt[r]);
+  int cnt = 0;
+  if (r < total) {
+    const int jb = find_job(row0, njobs, r);
+    const BatchJob& J = jobs[jb];
+    double k;
+    row_setup(J.v.pts, J.v.npts, (int)(r - J.row0), J.v.fp, &k, &row_logd[r], &cnt);
+    row_k[r] = k;
+    row_cnt[r] = cnt;
+    if (cnt > 0) atomicAdd(&hist[batch_bucket(jb, k)], 1);
+  }
+  for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
+  if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(ntasks, (unsigned long long)cnt);
 }
 
 __global__ void k_batch_point_rows(const BatchJob* __restrict__ jobs, const int* __restrict__ row0, int njobs,
                                    long total_rows, const double* __restrict__ row_k,
                                    const double* __restrict__ row_logd, const int* __restrict__ row_cnt,
-                                   const long long* __restrict__ row_off, double* __restrict__ flux,
-                                   TaskRec* __restrict__ recs)
+                                   double* __restrict__ flux, unsigned long long* __restrict__ off,
+                                   int* __restrict__ perm)
 {
   const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (gid >= total_rows * kNB1) return;
   const long r = gid / kNB1;
-  const BatchJob& J = jobs[find_job(row0, njobs, r)];
-  point_row_node(r, (int)(gid % kNB1), J.v.fp, row_k, row_logd, row_cnt, row_off, flux, recs);
+  const int j = (int)(gid % kNB1);
+  const int jb = find_job(row0, njobs, r);
+  if (j == 0 && row_cnt[r] > 0) perm[atomicAdd(&off[batch_bucket(jb, row_k[r])], 1ull)] = (int)r;
+  point_row_node(r, j, jobs[jb].v.fp, row_k, row_logd, row_cnt, flux);
 }
 
-// QAGS task source over all jobs: task records of the concatenated flux rows.
-struct BatchTask {
-  static constexpr bool kSharedFF = false;  // each job has its nucleus' table (FluxTask::ff)
-  const TaskRec* __restrict__ recs;
+// Flux rows of all jobs for the QAGS kernels; as a task source, task t = row
+// * 120 + node (its flux slot).
+struct BatchRows {
+  static constexpr bool kManyJobs = true;
+  const double* __restrict__ row_k;
+  const double* __restrict__ row_logd;
+  const int* __restrict__ row_cnt;
+  const int* __restrict__ perm;
   const BatchJob* __restrict__ jobs;
   const int* __restrict__ row0;
   int njobs;
   unsigned long long* __restrict__ job_failed;  // [njobs] integrals with ier != 0
-  __device__ void get(long long t, FluxTask* ft) const
+  __device__ int job_of(int r) const { return find_job(row0, njobs, r); }
+  __device__ RowJob params(int job) const
   {
-    const TaskRec rec = recs[t];
-    const int jb = find_job(row0, njobs, rec.out / kNB1);
-    const BatchJob& J = jobs[jb];
-    ft->b = rec.b;
-    ft->k = rec.k;
-    ft->out = rec.out;
-    ft->ff = J.ff;
-    ft->g1 = J.v.fp.g1;
-    ft->factor = J.v.fp.factor;
-    ft->A = J.v.fp.A;
-    ft->slot = jb;
-  }
-  __device__ void out(long long t, int job, FluxOut* fo) const
-  {
-    const TaskRec rec = recs[t];
     const BatchJob& J = jobs[job];
-    fo->k = rec.k;
-    fo->out = rec.out;
-    fo->factor = J.v.fp.factor;
-    fo->A = J.v.fp.A;
+    return RowJob{J.ff, J.v.fp.bmin, J.v.fp.g1, J.v.fp.factor, J.v.fp.A};
   }
   __device__ void failed(int job) const { atomicAdd(&job_failed[job], 1ull); }
-  __device__ const double4* any_ff() const { return jobs[0].ff; }
+  __device__ void get(long long t, FluxTask* ft) const
+  {
+    const long long r = t / kNB1;
+    const int jb = job_of((int)r);
+    const RowJob P = params(jb);
+    ft->b = row_node_b(P.bmin, row_logd[r], (int)(t - r * kNB1));
+    ft->k = row_k[r];
+    ft->out = t;
+    ft->ff = P.ff;
+    ft->g1 = P.g1;
+    ft->factor = P.factor;
+    ft->A = P.A;
+    ft->slot = jb;
+  }
 };
 
 // Contraction job resolver: blk0[j] = first block of job j for this wave count.
@@ -167,14 +201,15 @@ struct upc_batch {
   double* d_row_k = nullptr;
   double* d_row_logd = nullptr;
   int* d_row_cnt = nullptr;
-  long long* d_row_off = nullptr;
+  int* d_perm = nullptr;         // rows with QAGS nodes, by job and photon energy
+  int* d_hist = nullptr;         // [njobs][kBatchBuckets] rows per bucket
+  long long* d_off = nullptr;    // their offsets in d_perm
   long long* d_part = nullptr;
   double* d_flux = nullptr;
-  long long ntasks = 0;          // QAGS tasks of every job (counted at creation)
+  long long ntasks = 0;          // QAGS integrals of every job (counted at creation)
   long long work_bytes = 0;      // device memory of the buffers below
-  TaskRec* d_tasks = nullptr;
   long long* d_overflow = nullptr;
-  unsigned long long* d_counters = nullptr;  // [0] evals [1] bad [2] overflow n [4] tasks [5] cursor
+  unsigned long long* d_counters = nullptr;  // [0] evals [1] bad [2] overflow n [4] tasks [5] cursor [6] rows in d_perm
   unsigned long long* d_job_failed = nullptr;  // [njobs] QAGS integrals with ier != 0 per job
   int qags_choice = 2, lumi_choice = 1;  // indices into the candidate lists
   int form = UPC_FORM_FP64;              // contraction form of every job
@@ -206,7 +241,7 @@ void free_batch(upc_batch* b)
   if (b->graph) (void)hipGraphDestroy(b->graph);
   if (b->cap_stream) (void)hipStreamDestroy(b->cap_stream);
   void* ptrs[] = {b->d_jobs, b->d_pt0, b->d_row0, b->d_blk0[0], b->d_blk0[1], b->d_blk0[2], b->d_pts,
-                  b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_row_off, b->d_part, b->d_flux, b->d_tasks,
+                  b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_perm, b->d_hist, b->d_off, b->d_part, b->d_flux,
                   b->d_overflow, b->d_counters, b->d_job_failed};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
@@ -228,29 +263,52 @@ int contract_mfma(upc_batch* b, int tile_group, hipStream_t s)
   return 0;
 }
 
+// Points, row geometry and the row histogram of every job, from cleared counters.
+void enqueue_rows(upc_batch* b, hipStream_t s)
+{
+  const int nj = (int)b->jobs.size(), nhist = nj * kBatchBuckets;
+  hipLaunchKernelGGL(k_batch_clear, dim3(nblk(nhist, 256)), dim3(256), 0, s, b->d_counters, b->d_job_failed, nj,
+                     b->d_hist, nhist);
+  hipLaunchKernelGGL(k_batch_points, dim3(nblk(b->npts, 256)), dim3(256), 0, s, b->d_jobs, b->d_pt0, nj,
+                     b->npts, b->d_pts);
+  hipLaunchKernelGGL(k_batch_rows, dim3(nblk(b->nrows, 256)), dim3(256), 0, s, b->d_jobs, b->d_row0, nj,
+                     b->nrows, b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_hist, b->d_counters + 4);
+}
+
+BatchRows batch_rows(const upc_batch* b)
+{
+  return BatchRows{b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_perm, b->d_jobs, b->d_row0, (int)b->jobs.size(),
+                   b->d_job_failed};
+}
+
+void launch_qags(upc_batch* b, int choice, hipStream_t s)
+{
+  hipLaunchKernelGGL((k_flux_qags_rows<kQagsCap, BatchRows>), dim3(b->ncu * qags_blocks_per_cu(choice)),
+                     dim3(kQagsBlock), 0, s, batch_rows(b), b->d_counters + 6, b->d_counters + 5, b->d_flux,
+                     b->d_counters, b->d_overflow, kQagsCap);
+}
+
+void launch_qags_wave(upc_batch* b, hipStream_t s)
+{
+  hipLaunchKernelGGL((k_flux_qags_wave<BatchRows>), dim3(kQagsWaveBlocks), dim3(64), 0, s, batch_rows(b),
+                     b->d_overflow, b->d_counters, b->d_flux, (int*)nullptr);
+}
+
 // The whole grid computation of every job (no host synchronisation).
 int enqueue(upc_batch* b, hipStream_t s)
 {
   const int nj = (int)b->jobs.size();
-  hipLaunchKernelGGL(k_batch_zero, dim3(1), dim3(64), 0, s, b->d_counters, 8);
-  hipLaunchKernelGGL(k_batch_zero, dim3(nblk(nj, 256)), dim3(256), 0, s, b->d_job_failed, nj);
-  hipLaunchKernelGGL(k_batch_points, dim3(nblk(b->npts, 256)), dim3(256), 0, s, b->d_jobs, b->d_pt0, nj,
-                     b->npts, b->d_pts);
-  hipLaunchKernelGGL(k_batch_rows, dim3(nblk(b->nrows, 256)), dim3(256), 0, s, b->d_jobs, b->d_row0, nj,
-                     b->nrows, b->d_row_k, b->d_row_logd, b->d_row_cnt);
-  hipLaunchKernelGGL(k_scan_part<>, dim3(b->nparts), dim3(kScanBlock), 0, s, b->d_row_cnt, b->nrows, b->d_part);
-  hipLaunchKernelGGL(k_scan_top<>, dim3(1), dim3(kScanBlock), 0, s, b->d_part, b->nparts, b->d_counters + 4);
-  hipLaunchKernelGGL(k_scan_apply<>, dim3(b->nparts), dim3(kScanBlock), 0, s, b->d_row_cnt, b->nrows, b->d_part,
-                     b->d_row_off);
+  const long nhist = (long)nj * kBatchBuckets;
+  enqueue_rows(b, s);
+  hipLaunchKernelGGL(k_scan_part<>, dim3(b->nparts), dim3(kScanBlock), 0, s, b->d_hist, nhist, b->d_part);
+  hipLaunchKernelGGL(k_scan_top<>, dim3(1), dim3(kScanBlock), 0, s, b->d_part, b->nparts, b->d_counters + 6);
+  hipLaunchKernelGGL(k_scan_apply<>, dim3(b->nparts), dim3(kScanBlock), 0, s, b->d_hist, nhist, b->d_part,
+                     b->d_off);
   hipLaunchKernelGGL(k_batch_point_rows, dim3(nblk(b->nrows * kNB1, 256)), dim3(256), 0, s, b->d_jobs, b->d_row0,
-                     nj, b->nrows, b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_row_off, b->d_flux, b->d_tasks);
-  BatchTask ts{b->d_tasks, b->d_jobs, b->d_row0, nj, b->d_job_failed};
-  const int qblocks = b->ncu * kQagsBlockChoices[b->qags_choice];
-  hipLaunchKernelGGL((k_flux_qags<kQagsCap, BatchTask>), dim3(qblocks), dim3(kQagsBlock), 0, s, ts,
-                     b->d_counters + 4, b->d_counters + 5, b->d_flux, (int*)nullptr, b->d_counters, b->d_overflow,
-                     kQagsCap);
-  hipLaunchKernelGGL((k_flux_qags_wave<BatchTask>), dim3(kQagsWaveBlocks), dim3(64), 0, s, ts, b->d_overflow,
-                     b->d_counters, b->d_flux, (int*)nullptr);
+                     nj, b->nrows, b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_flux,
+                     (unsigned long long*)b->d_off, b->d_perm);
+  launch_qags(b, b->qags_choice, s);
+  launch_qags_wave(b, s);
   if (b->form != UPC_FORM_FP64) return contract_mfma(b, kMfmaTileChoices[b->mfma_choice], s);
   const int li = b->lumi_choice, w = kLumiWaveChoices[li];
   BatchLumi jr{b->d_jobs, b->d_blk0[li], nj};
@@ -305,7 +363,7 @@ int upc_batch_create(const upc_config* cfgs, int njobs, void* stream, upc_batch*
   }
   b->npts = np;
   b->nrows = nr;
-  b->nparts = nblk(nr, kScanBlock);
+  b->nparts = nblk((long)njobs * kBatchBuckets, kScanBlock);
   for (int i = 0; i < 3; ++i) b->lumi_blocks[i] = (int)blocks[i];
 #define BA(ptr, n)                                                  \
   do {                                                              \
@@ -321,7 +379,9 @@ int upc_batch_create(const upc_config* cfgs, int njobs, void* stream, upc_batch*
     BA(b->d_row_k, nr);
     BA(b->d_row_logd, nr);
     BA(b->d_row_cnt, nr);
-    BA(b->d_row_off, nr);
+    BA(b->d_perm, nr);
+    BA(b->d_hist, (size_t)njobs * kBatchBuckets);
+    BA(b->d_off, (size_t)njobs * kBatchBuckets);
     BA(b->d_part, b->nparts);
     BA(b->d_flux, nr * kNB1);
     BA(b->d_counters, 8);
@@ -373,27 +433,18 @@ int upc_batch_create(const upc_config* cfgs, int njobs, void* stream, upc_batch*
     free_batch(b);
     return rc;
   }
-  // The QAGS task buffers (records, overflow list) are sized by
-  // the batch's task count, which the row kernels and the scan give once here.
+  // The overflow list is sized by the batch's integral count, which the row
+  // kernels give once here.
   auto size_tasks = [&]() -> int {
-    const int nj = (int)b->jobs.size();
-    hipLaunchKernelGGL(k_batch_zero, dim3(1), dim3(64), 0, s, b->d_counters, 8);
-    hipLaunchKernelGGL(k_batch_points, dim3(nblk(b->npts, 256)), dim3(256), 0, s, b->d_jobs, b->d_pt0, nj,
-                       b->npts, b->d_pts);
-    hipLaunchKernelGGL(k_batch_rows, dim3(nblk(b->nrows, 256)), dim3(256), 0, s, b->d_jobs, b->d_row0, nj,
-                       b->nrows, b->d_row_k, b->d_row_logd, b->d_row_cnt);
-    hipLaunchKernelGGL(k_scan_part<>, dim3(b->nparts), dim3(kScanBlock), 0, s, b->d_row_cnt, b->nrows,
-                       b->d_part);
-    hipLaunchKernelGGL(k_scan_top<>, dim3(1), dim3(kScanBlock), 0, s, b->d_part, b->nparts, b->d_counters + 4);
+    enqueue_rows(b, s);
     UPC_HIP(hipGetLastError());
     unsigned long long total = 0;
     UPC_HIP(hipMemcpyAsync(&total, b->d_counters + 4, sizeof(total), hipMemcpyDeviceToHost, s));
     UPC_HIP(hipStreamSynchronize(s));
     b->ntasks = (long long)total;
     const size_t n = total > 0 ? (size_t)total : 1;
-    UPC_HIP(hipMalloc(&b->d_tasks, sizeof(TaskRec) * n));
     UPC_HIP(hipMalloc(&b->d_overflow, sizeof(long long) * n));
-    b->work_bytes += (long long)((sizeof(TaskRec) + sizeof(long long)) * n);
+    b->work_bytes += (long long)(sizeof(long long) * n);
     return 0;
   };
   if (int rc = size_tasks()) {
@@ -508,16 +559,12 @@ int upc_batch_autotune(upc_batch* b, void* stream, upc_tune* h_out)
   UPC_HIP(hipEventCreate(&e0));
   UPC_HIP(hipEventCreate(&e1));
   const int nj = (int)b->jobs.size();
-  BatchTask ts{b->d_tasks, b->d_jobs, b->d_row0, nj, b->d_job_failed};
   for (int i = 0; i < 3; ++i) {
-    // QAGS alone: clear the counters except the task total, then time
+    // QAGS alone: clear the counters except the integral and row totals, then time
     hipLaunchKernelGGL(k_batch_zero, dim3(1), dim3(64), 0, s, b->d_counters, 4);
     hipLaunchKernelGGL(k_batch_zero, dim3(1), dim3(64), 0, s, b->d_counters + 5, 1);
     UPC_HIP(hipEventRecord(e0, s));
-    const int qblocks = b->ncu * kQagsBlockChoices[i];
-    hipLaunchKernelGGL((k_flux_qags<kQagsCap, BatchTask>), dim3(qblocks), dim3(kQagsBlock), 0, s, ts,
-                       b->d_counters + 4, b->d_counters + 5, b->d_flux, (int*)nullptr, b->d_counters, b->d_overflow,
-                       kQagsCap);
+    launch_qags(b, i, s);
     UPC_HIP(hipEventRecord(e1, s));
     UPC_HIP(hipEventSynchronize(e1));
     float ms = 0;
@@ -526,8 +573,7 @@ int upc_batch_autotune(upc_batch* b, void* stream, upc_tune* h_out)
     t.qags_ms[i] = ms;
   }
   // restore the overflow results (the timed passes re-ran every task)
-  hipLaunchKernelGGL((k_flux_qags_wave<BatchTask>), dim3(kQagsWaveBlocks), dim3(64), 0, s, ts, b->d_overflow,
-                     b->d_counters, b->d_flux, (int*)nullptr);
+  launch_qags_wave(b, s);
   for (int i = 0; i < 3 && b->form != UPC_FORM_FP64; ++i) {
     // the MFMA form's tile shape: column tiles per A-fragment load (results identical)
     UPC_HIP(hipEventRecord(e0, s));

@@ -30,6 +30,15 @@ __device__ __forceinline__ double row_node(double bmin, double logd, int j, doub
   return (*bh + *bl) / 2.;
 }
 
+// The same node for the QAGS kernels, the contraction that the compiler makes
+// of row_node's sum spelled out: every kernel that integrates a node sees the
+// same b.
+__device__ __forceinline__ double row_node_b(double bmin, double logd, int j)
+{
+  const double bl = bmin * exp(j * logd);
+  return fma(bmin, exp((j + 1.) * logd), bl) / 2.;
+}
+
 // Position guess on a row's log-spaced nodes b_j = (bmin e^{j logd} +
 // bmin e^{(j+1) logd}) / 2 = c0 e^{j logd}: the first j with b_j >= v, from
 // one float log2 (right up to +-1 where v lies within rounding of a node).
@@ -109,6 +118,11 @@ __device__ __forceinline__ double flux_point(double b, double k, double g1, doub
   return factor * k / g / g * (K1 * K1 + K0 * K0 / g / g);
 }
 
+// QAGS nodes of one flux row are at most 97: node j has b_j >= bmin e^{j logd}
+// with bmin = 0.05 R and logd >= ln(5R / bmin) / 120, so b_j <= 2R needs
+// j <= 120 ln 40 / ln 100 = 96.09.
+constexpr int kMaxQagsNodesPerRow = 98;
+
 // Geometry of flux row r of a grid of npts points (src/UpcCrossSection.cpp:
 // 224-233): photon energy, log step of the b grid, and the number of its
 // nodes with b <= 2R (form-factor QAGS nodes; 0 for the point flux).
@@ -142,7 +156,19 @@ __device__ __forceinline__ void row_setup(const double* __restrict__ pts, int np
   }
   *k_out = k;
   *logd_out = logd;
-  *cnt_out = cnt;
+  *cnt_out = cnt < kMaxQagsNodesPerRow ? cnt : kMaxQagsNodesPerRow;  // more only where k is NaN
+}
+
+// Bucket of a row in the photon energy order of the QAGS kernel: `per_octave`
+// buckets per factor of two of k over 40 octaves about 1 GeV, the end buckets
+// taking what lies outside (NaN in the first).
+constexpr int kRowOctaves = 40;
+
+__device__ __forceinline__ int row_bucket(double k, int per_octave)
+{
+  const float v = (__log2f((float)k) + 0.5f * kRowOctaves) * per_octave;
+  const int n = kRowOctaves * per_octave;
+  return v > 0.f ? (v < (float)(n - 1) ? (int)v : n - 1) : 0;
 }
 
 // fluxFormIntegrand (src/UpcCrossSection.cpp:181-191):
@@ -211,30 +237,15 @@ struct FluxFormIntegrand {
   __device__ __forceinline__ double operator()(double q) const { return flux_integrand<0>(ff, b, w2g2, q); }
 };
 
-// One form-factor QAGS task of a flux row: its node (b, k) and the flux slot
-// (row * 120 + node) the integral fills.
-struct TaskRec {
-  double b, k;
-  long long out;
-};
-
-// Node j of flux row r: the point-charge flux (b > 2R or FLUX_POINT 1), or a
-// QAGS task record at the row's task offset.
+// Node j of flux row r: the point-charge flux (b > 2R or FLUX_POINT 1).  The
+// form-factor nodes j < row_cnt[r] are left to the QAGS kernel.
 __device__ __forceinline__ void point_row_node(long long r, int j, const FluxParams& fp,
                                                const double* __restrict__ row_k, const double* __restrict__ row_logd,
-                                               const int* __restrict__ row_cnt,
-                                               const long long* __restrict__ row_off, double* __restrict__ flux,
-                                               TaskRec* __restrict__ recs)
+                                               const int* __restrict__ row_cnt, double* __restrict__ flux)
 {
+  if (j < row_cnt[r]) return;
   double bl, bh;
   const double b = row_node(fp.bmin, row_logd[r], j, &bl, &bh);
-  if (j < row_cnt[r]) {
-    TaskRec* t = recs + row_off[r] + j;
-    t->b = b;
-    t->k = row_k[r];
-    t->out = r * kNB1 + j;
-    return;
-  }
   flux[r * kNB1 + j] = flux_point(b, row_k[r], fp.g1, fp.factor);
 }
 
@@ -256,45 +267,22 @@ struct FluxOut {
   int A;
 };
 
-// Task sources of the QAGS kernel: get(t) describes task t; out(t, job)
-// gives its output fields again (job: FluxTask::slot of the same task).
-struct GridTask {  // flux-row nodes of one context
-  static constexpr bool kSharedFF = true;  // one form-factor table for every task (ff)
-  const TaskRec* __restrict__ recs;
-  FluxParams fp;
-  const double4* ff;
-  __device__ void get(long long t, FluxTask* ft) const
-  {
-    const TaskRec rec = recs[t];
-    ft->b = rec.b;
-    ft->k = rec.k;
-    ft->out = rec.out;
-    ft->ff = ff;
-    ft->g1 = fp.g1;
-    ft->factor = fp.factor;
-    ft->A = fp.A;
-    ft->slot = 0;
-  }
-  __device__ void out(long long t, int, FluxOut* fo) const
-  {
-    const TaskRec rec = recs[t];
-    fo->k = rec.k;
-    fo->out = rec.out;
-    fo->factor = fp.factor;
-    fo->A = fp.A;
-  }
-  // An integral of job `job` that ended with ier != 0 (counted in the launch's stats).
-  __device__ void failed(int) const {}
-  __device__ const double4* any_ff() const { return ff; }
-};
-
-struct PointTask {  // arbitrary (b, k) points of one context
-  static constexpr bool kSharedFF = true;
+// Task sources of the per-point QAGS kernel and of the 1000-interval kernel:
+// get(t) describes task t.  Per-point tasks: an arbitrary (b, k).
+struct PointTask {
   const double* __restrict__ b;
   const double* __restrict__ k;
   const int* __restrict__ idx;  // compacted indices of points needing QAGS
   FluxParams fp;
   const double4* ff;
+  const unsigned long long* __restrict__ count;  // compacted points
+  __device__ long long ids() const { return (long long)*count; }
+  __device__ bool team(long long id, FluxTask* ft) const
+  {
+    get(id, ft);
+    return true;
+  }
+  __device__ long long overflow_id(long long id) const { return id; }
   __device__ void get(long long t, FluxTask* ft) const
   {
     const int i = idx[t];
@@ -307,7 +295,7 @@ struct PointTask {  // arbitrary (b, k) points of one context
     ft->A = fp.A;
     ft->slot = 0;
   }
-  __device__ void out(long long t, int, FluxOut* fo) const
+  __device__ void out(long long t, FluxOut* fo) const
   {
     const int i = idx[t];
     fo->k = k[i];
@@ -316,11 +304,58 @@ struct PointTask {  // arbitrary (b, k) points of one context
     fo->A = fp.A;
   }
   __device__ void failed(int) const {}
-  __device__ const double4* any_ff() const { return ff; }
+};
+
+// What the integrals of one configuration share.
+struct RowJob {
+  const double4* ff;
+  double bmin, g1, factor;
+  int A;
+};
+
+// Flux rows of one context for k_flux_qags_rows; as a task source, task
+// t = row * 120 + node (its flux slot).
+struct GridRows {
+  static constexpr bool kManyJobs = false;
+  const double* __restrict__ row_k;
+  const double* __restrict__ row_logd;
+  const int* __restrict__ row_cnt;
+  const int* __restrict__ perm;  // rows with form-factor nodes, ordered by k
+  RowJob job;
+  long long nrows;
+  // team work ids: (row, node), kMaxQagsNodesPerRow slots per row
+  __device__ long long ids() const { return nrows * kMaxQagsNodesPerRow; }
+  __device__ long long overflow_id(long long id) const
+  {
+    const long long r = id / kMaxQagsNodesPerRow;
+    return r * kNB1 + (id - r * kMaxQagsNodesPerRow);
+  }
+  __device__ bool team(long long id, FluxTask* ft) const
+  {
+    const long long r = id / kMaxQagsNodesPerRow;
+    if ((int)(id - r * kMaxQagsNodesPerRow) >= row_cnt[r]) return false;
+    get(overflow_id(id), ft);
+    return true;
+  }
+  __device__ int job_of(int) const { return 0; }
+  __device__ RowJob params(int) const { return job; }
+  __device__ void failed(int) const {}
+  __device__ void get(long long t, FluxTask* ft) const
+  {
+    const long long r = t / kNB1;
+    ft->b = row_node_b(job.bmin, row_logd[r], (int)(t - r * kNB1));
+    ft->k = row_k[r];
+    ft->out = t;
+    ft->ff = job.ff;
+    ft->g1 = job.g1;
+    ft->factor = job.factor;
+    ft->A = job.A;
+    ft->slot = 0;
+  }
 };
 
 // ---------------------------------------------------------------------------
-// Form-factor flux: persistent QAGS kernel.
+// Form-factor flux at arbitrary points: persistent QAGS kernel.
 //
 // Each lane owns one integral at a time (the dqagse state machine of
 // upc_qags.h, its interval lists in private memory) and takes a new task
@@ -382,7 +417,6 @@ struct SweepItem {
   FluxNode n;
 };
 
-template <bool SHARED_FF>
 __device__ __forceinline__ void sweep_fetch(QagsWaveLds& W, int lane, int r0, int end, const double4* ff, double b,
                                             double w2g2, SweepItem* it)
 {
@@ -393,13 +427,11 @@ __device__ __forceinline__ void sweep_fetch(QagsWaveLds& W, int lane, int r0, in
   const int code = it->act ? raw : lane << 5;
   const int owner = code >> 5, e = code & 31;
   const double bo = __shfl(b, owner), wo = __shfl(w2g2, owner);
-  const double4* ffo = ff;
-  if (!SHARED_FF) ffo = (const double4*)__shfl((long long)ff, owner);
   it->slot = owner * 21 + e;
   const double qv = W.v[it->slot];
   const double q = it->act ? qv : 0.0;
   it->x = flux_j1_arg(bo, q);
-  flux_prelude(ffo, wo, q, &it->n);
+  flux_prelude(ff, wo, q, &it->n);
 }
 
 template <int BR>
@@ -415,7 +447,7 @@ __device__ __forceinline__ void sweep_finish(QagsWaveLds& W, const SweepItem& it
 // the other waves' fetches and bookkeeping, whose waits then overlap them
 // (2 % on the QAGS phase).  A remainder of at most 64 items takes one sweep
 // of its own.
-template <int BR, bool SHARED_FF>
+template <int BR>
 __device__ __forceinline__ void qags_sweeps(QagsWaveLds& W, int lane, int beg, int end, const double4* ff,
                                             double b, double w2g2)
 {
@@ -423,8 +455,8 @@ __device__ __forceinline__ void qags_sweeps(QagsWaveLds& W, int lane, int beg, i
 #pragma unroll 1
   for (; r0 + 64 < end; r0 += 128) {
     SweepItem ia, ib;
-    sweep_fetch<SHARED_FF>(W, lane, r0, end, ff, b, w2g2, &ia);
-    sweep_fetch<SHARED_FF>(W, lane, r0 + 64, end, ff, b, w2g2, &ib);
+    sweep_fetch(W, lane, r0, end, ff, b, w2g2, &ia);
+    sweep_fetch(W, lane, r0 + 64, end, ff, b, w2g2, &ib);
     __builtin_amdgcn_s_setprio(2);
     sweep_finish<BR>(W, ia);
     sweep_finish<BR>(W, ib);
@@ -432,7 +464,7 @@ __device__ __forceinline__ void qags_sweeps(QagsWaveLds& W, int lane, int beg, i
   }
   if (r0 < end) {
     SweepItem ia;
-    sweep_fetch<SHARED_FF>(W, lane, r0, end, ff, b, w2g2, &ia);
+    sweep_fetch(W, lane, r0, end, ff, b, w2g2, &ia);
     sweep_finish<BR>(W, ia);
   }
 }
@@ -466,7 +498,6 @@ __device__ __forceinline__ int wave_prefix5(int x, int* total)
 // nodes are the first ns of its nodes in abscissa order: the lane's items
 // are two runs, [ps, ps + ns) among the small items and the rest among the
 // large ones, placed by one prefix sum over the lanes.
-template <bool SHARED_FF>
 __device__ __forceinline__ QK21Out qk21_wave(QagsWaveLds& W, int lane, bool mine, double qa, double qb,
                                              const double4* ff, double b, double w2g2)
 {
@@ -500,8 +531,8 @@ __device__ __forceinline__ QK21Out qk21_wave(QagsWaveLds& W, int lane, bool mine
     }
   }
   wave_lds_sync();
-  qags_sweeps<1, SHARED_FF>(W, lane, 0, S, ff, b, w2g2);
-  qags_sweeps<2, SHARED_FF>(W, lane, S, ntot, ff, b, w2g2);
+  qags_sweeps<1>(W, lane, 0, S, ff, b, w2g2);
+  qags_sweeps<2>(W, lane, S, ntot, ff, b, w2g2);
   wave_lds_sync();
   QK21Out o{};
   if (mine) o = qk21_stored(col, 1, qa, qb);
@@ -523,11 +554,8 @@ void k_flux_qags(TS ts, const unsigned long long* __restrict__ ntasks_p, unsigne
   const long long ntasks = (long long)*ntasks_p;
   const int lane = threadIdx.x & 63;
   long long task = -1;  // -1: needs a task; LLONG_MAX: exhausted
-  // Live across the steps of a task: b, (k/g)^2, the form-factor table and the
-  // job; the output fields (k, slot, factor, A) are read again when it ends.
-  const double4* ft_ff = ts.any_ff();  // a valid table for the sweeps' idle lanes before the first task
+  // Live across the steps of a task: b and (k/g)^2; the output fields (k, slot, factor, A) are read again when it ends.
   double ft_b = 0.0, w2g2 = 0.0;
-  int ft_job = 0;
   unsigned my_evals = 0, my_bad = 0;  // 32-bit per lane; evaluations flushed before they could wrap
   while (true) {
     bool need = task < 0;
@@ -544,8 +572,6 @@ void k_flux_qags(TS ts, const unsigned long long* __restrict__ ntasks_p, unsigne
           FluxTask ft;
           ts.get(t, &ft);
           ft_b = ft.b;
-          ft_ff = ft.ff;
-          ft_job = ft.slot;
           w2g2 = ft.k * ft.k / ft.g1 / ft.g1;
           q.start();
         } else {
@@ -557,22 +583,19 @@ void k_flux_qags(TS ts, const unsigned long long* __restrict__ ntasks_p, unsigne
     if (__ballot(task != LLONG_MAX) == 0) break;
     const bool live = task != LLONG_MAX;
     const int np = live ? q.passes() : 0;
-    const double4* ff;
-    if constexpr (TS::kSharedFF) ff = ts.ff;
-    else ff = ft_ff;
     double qa = 0.0, qb = 0.0;
     if (live) q.interval(0, &qa, &qb);
-    const QK21Out o = qk21_wave<TS::kSharedFF>(W, lane, live, qa, qb, ff, ft_b, w2g2);
+    const QK21Out o = qk21_wave(W, lane, live, qa, qb, ts.ff, ft_b, w2g2);
     QK21Out o2{};
     if (__ballot(np == 2) != 0) {
       if (np == 2) q.interval(1, &qa, &qb);
-      o2 = qk21_wave<TS::kSharedFF>(W, lane, np == 2, qa, qb, ff, ft_b, w2g2);
+      o2 = qk21_wave(W, lane, np == 2, qa, qb, ts.ff, ft_b, w2g2);
     }
     if (!live) continue;
     const int st = q.consume(o, o2);
     if (st == kQagsDone) {
       FluxOut fo;
-      ts.out(task, ft_job, &fo);
+      ts.out(task, &fo);
       const double Q = q.result / fo.A;
       flux[fo.out] = fo.factor * Q * Q / fo.k;
       const int status = q.status();
@@ -583,7 +606,6 @@ void k_flux_qags(TS ts, const unsigned long long* __restrict__ ntasks_p, unsigne
         my_evals = 0;
       }
       my_bad += status != 0;
-      if (status != 0) ts.failed(ft_job);
       task = -1;
     } else if (st == kQagsOverflow) {
       const unsigned long long slot = atomicAdd(&stats[2], 1ull);
@@ -599,6 +621,249 @@ void k_flux_qags(TS ts, const unsigned long long* __restrict__ ntasks_p, unsigne
   if (lane == 0) {
     atomicAdd(&stats[0], evals);
     atomicAdd(&stats[1], bad);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Form-factor flux of whole flux rows.
+//
+// A wavefront takes 64 rows that are neighbours in photon energy k (rows are
+// bucket-sorted by k) and one node index j, one integral per lane.  b_j and
+// (k/g)^2 then differ by a fraction of a percent over the lanes, so nearly
+// every dqagse decision is the same for all of them: on the 1001 x 121 Pb-Pb
+// grid 99 % of the QK21 passes are on one interval for the whole wavefront,
+// 99.7 % of the lane steps are in use although a lane that ends early waits
+// for the others, and J1's branch (x = b q / hc <= 8 or not) is mixed in 0.5 %
+// of the node evaluations (101 x 41: 92 %, 91 %, 4 %).  So each lane
+// evaluates its own nodes directly, in QK21's summation order, with J1's
+// branch taken by the whole wavefront; the spline records of one node lie
+// side by side over the lanes.  A pass keeps its 20 off-centre values in LDS
+// (10,240 B per wavefront) for the mean deviation.
+//
+// Against the per-point kernel above over the same integrals (1001 x 121
+// Pb-Pb): 14.2 -> 10.4 ms, 158 -> 124 VALU instructions per integrand value,
+// no task records (24 B each) written and read.  Bound: VALU issue (80 % of
+// the time at 3 waves per SIMD, no spills).  Two nodes per trip spill 44 VGPRs
+// (10.2 ms, slower on small grids); 4 waves per SIMD spill 66 (10.1 ms, same).
+//
+// Work ids are (group of 64 rows, j), taken from a global cursor; ids whose
+// group has no node j end at once.  nrows_p: rows in rs.perm.  stats as in
+// k_flux_qags; overflow receives flux slots (row * 120 + node).
+// ---------------------------------------------------------------------------
+constexpr int kQagsRowsWaves = 3;        // waves per SIMD (register and LDS budget)
+constexpr int kQagsRowsBlocksPerCu = 3;  // resident workgroups of kQagsBlock per CU
+
+// One QK21 pass on [qa, qb] for every active lane: qk21_stored's sums in its
+// order, the integrand evaluated on the way.  fv: the lane's column of the
+// wavefront's table (stride 64).
+__device__ __forceinline__ QK21Out qk21_rows(double* fv, double qa, double qb, const double4* __restrict__ ff,
+                                             double b, double w2g2)
+{
+  const double centr = 0.5 * (qa + qb), hlgth = 0.5 * (qb - qa);
+  double resg = 0.0, resk = 0.0, rabs = 0.0, fc = 0.0, f1 = 0.0;
+#pragma unroll 1
+  for (int e = 0; e < 21; ++e) {  // the centre, the Gauss pairs, the Kronrod-only pairs (left, right)
+    const double f = flux_integrand<0>(ff, b, w2g2, qk21_abscissa(e, centr, hlgth));
+    if (e == 0) {
+      fc = f;
+      resk = kWgk[10] * fc;
+      rabs = fabs(resk);
+      continue;
+    }
+    fv[(e - 1) * 64] = f;
+    if (e & 1) {
+      f1 = f;
+      continue;
+    }
+    const double fsum = f1 + f;
+    const int p = (e >> 1) - 1;
+    const int j = p < 5 ? 2 * p + 1 : 2 * (p - 5);
+    if (p < 5) resg = resg + kWg[p] * fsum;
+    resk = resk + kWgk[j] * fsum;
+    rabs = rabs + kWgk[j] * (fabs(f1) + fabs(f));
+  }
+  return qk21_tail([&](int j, int side) { return fv[(qk21_node(j, side) - 1) * 64]; }, resg, resk, rabs, fc, hlgth);
+}
+
+template <int CAP, class RS>
+__global__ __launch_bounds__(kQagsBlock) __attribute__((amdgpu_waves_per_eu(kQagsRowsWaves, kQagsRowsWaves)))
+void k_flux_qags_rows(RS rs, const unsigned long long* __restrict__ nrows_p, unsigned long long* __restrict__ cursor,
+                      double* __restrict__ flux, unsigned long long* __restrict__ stats,
+                      long long* __restrict__ overflow, int fast_cap)
+{
+  __shared__ double lds[kQagsBlock / 64][20 * 64];
+  const int lane = threadIdx.x & 63;
+  double* fv = lds[threadIdx.x >> 6] + lane;
+  typename QagsSmallStore<CAP>::Arrays lists;
+  Qags<QagsSmallStore<CAP>> q;
+  q.s.a = &lists;
+  q.s.lim = fast_cap < CAP ? fast_cap : CAP;
+  const long long nrows = (long long)*nrows_p;
+  const unsigned long long nids = (unsigned long long)((nrows + 63) / 64) * kMaxQagsNodesPerRow;
+  unsigned my_evals = 0, my_bad = 0;  // 32-bit per lane; evaluations flushed before they could wrap
+  while (true) {
+    unsigned long long id = 0;
+    if (lane == 0) id = atomicAdd(cursor, 1ull);
+    id = __shfl(id, 0);
+    if (id >= nids) break;
+    const long long g = (long long)(id / kMaxQagsNodesPerRow);
+    const int j = (int)(id - (unsigned long long)g * kMaxQagsNodesPerRow);
+    const long long pos = g * 64 + lane;
+    int r = 0, job = 0;
+    bool act = false;
+    if (pos < nrows) {
+      r = rs.perm[pos];
+      act = j < rs.row_cnt[r];
+      if (RS::kManyJobs && act) job = rs.job_of(r);
+    }
+    unsigned long long todo = __ballot(act);
+    while (todo) {
+      // one configuration at a time (a group straddles two only where their rows meet)
+      int jb = 0;
+      bool live = act;
+      if (RS::kManyJobs) {
+        jb = __builtin_amdgcn_readlane(job, __ffsll((long long)todo) - 1);
+        live = act && job == jb;
+        todo &= ~__ballot(live);
+      } else {
+        todo = 0;
+      }
+      const RowJob P = rs.params(jb);
+      double b = 0.0, w2g2 = 0.0;
+      if (live) {
+        b = row_node_b(P.bmin, rs.row_logd[r], j);
+        const double k = rs.row_k[r];
+        w2g2 = k * k / P.g1 / P.g1;
+        q.start();
+      }
+      while (__ballot(live) != 0) {
+        if (!live) continue;
+        QK21Out o{}, o2{};
+#pragma unroll 1
+        for (int pass = 0; pass < q.passes(); ++pass) {
+          double qa, qb;
+          q.interval(pass, &qa, &qb);
+          o = o2;
+          o2 = qk21_rows(fv, qa, qb, P.ff, b, w2g2);
+        }
+        if (q.phase == 0) o = o2;
+        const int st = q.consume(o, o2);
+        if (st == kQagsRunning) continue;
+        live = false;
+        const long long slot = (long long)r * kNB1 + j;
+        if (st == kQagsDone) {
+          const double Q = q.result / P.A;
+          flux[slot] = P.factor * Q * Q / rs.row_k[r];
+          my_evals += (unsigned)q.neval();
+          if (my_evals >= 0x80000000u) {
+            atomicAdd(&stats[0], (unsigned long long)my_evals);
+            my_evals = 0;
+          }
+          if (q.status() != 0) {
+            my_bad++;
+            rs.failed(jb);
+          }
+        } else {
+          overflow[atomicAdd(&stats[2], 1ull)] = slot;
+        }
+      }
+    }
+  }
+  unsigned long long evals = my_evals, bad = my_bad;
+  for (int o = 32; o > 0; o >>= 1) {
+    evals += __shfl_down(evals, o);
+    bad += __shfl_down(bad, o);
+  }
+  if (lane == 0) {
+    atomicAdd(&stats[0], evals);
+    atomicAdd(&stats[1], bad);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Form-factor flux, few integrals: G lanes per integral.
+//
+// With one integral per lane an integral takes some 300 integrand values one
+// after another, 0.4 ms whatever the count, and a launch of fewer integrals
+// than the chip has lanes leaves SIMDs idle for that long.  Here a team of G
+// lanes evaluates the 42 nodes of a dqagse step together (all of them at once
+// for G = 64), lane pairs sum the two passes in QK21's order, and every lane
+// of the team runs the same bookkeeping on lists in LDS.  The values and
+// their order are those of the other kernels.
+//
+// TS::ids(): work ids, one team each; TS::team(id, &task): false where the id
+// holds no integral.  overflow receives what TS::get takes.
+// ---------------------------------------------------------------------------
+template <int CAP>
+struct QagsTeamLds {
+  double v[42];
+  typename QagsSmallStore<CAP>::Arrays lists;
+};
+
+template <int G, int CAP, class TS>
+__global__ __launch_bounds__(kQagsBlock) void k_flux_qags_team(TS ts, double* __restrict__ flux,
+                                                               int* __restrict__ ier_out,
+                                                               unsigned long long* __restrict__ stats,
+                                                               long long* __restrict__ overflow, int fast_cap)
+{
+  constexpr int kTeams = kQagsBlock / G;
+  __shared__ QagsTeamLds<CAP> lds[kTeams];
+  __shared__ unsigned blk_evals, blk_bad;
+  if (threadIdx.x == 0) blk_evals = blk_bad = 0;
+  __syncthreads();
+  const int tl = threadIdx.x % G, lane0 = (threadIdx.x & 63) - tl;
+  QagsTeamLds<CAP>& W = lds[threadIdx.x / G];
+  const long long id = (long long)blockIdx.x * kTeams + threadIdx.x / G;
+  Qags<QagsSmallStore<CAP>> q;
+  q.s.a = &W.lists;
+  q.s.lim = fast_cap < CAP ? fast_cap : CAP;
+  FluxTask ft{};
+  bool live = id < ts.ids() && ts.team(id, &ft);
+  const double w2g2 = ft.k * ft.k / ft.g1 / ft.g1;
+  if (live) q.start();
+  while (live) {
+    const int np = q.passes();
+#pragma unroll 1
+    for (int n = tl; n < 21 * np; n += G) {
+      const int pass = n >= 21;
+      double qa, qb;
+      q.interval(pass, &qa, &qb);
+      W.v[n] = flux_integrand<0>(ft.ff, ft.b, w2g2, qk21_abscissa(n - 21 * pass, 0.5 * (qa + qb), 0.5 * (qb - qa)));
+    }
+    wave_lds_sync();
+    QK21Out o, o2;
+    {
+      const int pass = np == 2 ? tl & 1 : 0;
+      double qa, qb;
+      q.interval(pass, &qa, &qb);
+      const QK21Out t = qk21_stored(W.v + 21 * pass, 1, qa, qb);
+      o = QK21Out{__shfl(t.result, lane0), __shfl(t.abserr, lane0), __shfl(t.resabs, lane0), __shfl(t.resasc, lane0)};
+      o2 = QK21Out{__shfl(t.result, lane0 + 1), __shfl(t.abserr, lane0 + 1), 0.0, __shfl(t.resasc, lane0 + 1)};
+    }
+    wave_lds_sync();
+    const int st = q.consume(o, o2);
+    wave_lds_sync();
+    if (st == kQagsRunning) continue;
+    live = false;
+    if (tl) continue;
+    if (st == kQagsDone) {
+      const double Q = q.result / ft.A;
+      flux[ft.out] = ft.factor * Q * Q / ft.k;
+      const int status = q.status();
+      if (ier_out) ier_out[ft.out] = status;
+      atomicAdd(&blk_evals, (unsigned)q.neval());
+      if (status != 0) {
+        atomicAdd(&blk_bad, 1u);
+        ts.failed(ft.slot);
+      }
+    } else {
+      overflow[atomicAdd(&stats[2], 1ull)] = ts.overflow_id(id);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (blk_evals) atomicAdd(&stats[0], (unsigned long long)blk_evals);
+    if (blk_bad) atomicAdd(&stats[1], (unsigned long long)blk_bad);
   }
 }
 

@@ -10,8 +10,10 @@
 // -ymax, lower bin edges) the k2 of bin (im, iy >= 1) is the k1 of its mirror
 // bin (im, ny - iy) up to one rounding of y, so only the iy = 0 column gets
 // own k2 rows: rows [npts, npts + nm).  Otherwise rows [npts, 2 npts) hold the
-// k2 rows.  flux[r*120 + j].  Nodes with b <= 2R (form-factor flux) become
-// QAGS tasks; the rest take the point-charge flux.
+// k2 rows.  flux[r*120 + j].  Nodes with b <= 2R (form-factor flux) are left
+// to the QAGS kernel, which takes the rows in order of k (counting sort:
+// histogram in k_rows, offsets in k_row_offsets, ranks in
+// k_flux_point_rows); the rest take the point-charge flux.
 #include "upc_internal.h"
 #include "upc_qags.h"
 #include "upc_flux.h"
@@ -24,10 +26,14 @@ namespace upc {
 // ---------------------------------------------------------------------------
 // Grid points: lower bin edges (src/UpcCrossSection.cpp:540-550)
 // ---------------------------------------------------------------------------
+//
+// The points kernels also clear the counters and the row histogram of the
+// flux launch that follows (clear[0 .. nclear)).
 __global__ void k_grid_points(int nm, double mmin, double mmax, int ny, double ymin, double ymax,
-                              double* __restrict__ pts)
+                              double* __restrict__ pts, int* __restrict__ clear, int nclear)
 {
   const long bin = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  for (long i = bin; i < nclear; i += (long)gridDim.x * blockDim.x) clear[i] = 0;
   if (bin >= (long)nm * ny) return;
   const int im = (int)(bin / ny), iy = (int)(bin % ny);
   const double dy = (ymax - ymin) / ny;
@@ -38,32 +44,76 @@ __global__ void k_grid_points(int nm, double mmin, double mmax, int ny, double y
   pts[4 * bin + 3] = dy;
 }
 
-// Row geometry and the number of form-factor (QAGS) nodes of each row.
-// need (may be null): rows with need[r] == 0 get no QAGS tasks (their
-// form-factor nodes are left unset).
-__global__ void k_rows(const double* __restrict__ pts, int npts, int nrows, FluxParams fp,
-                       double* __restrict__ row_k, double* __restrict__ row_logd, int* __restrict__ row_cnt,
-                       const unsigned char* __restrict__ need)
+// Row geometry, the number of form-factor (QAGS) nodes of each row, the
+// histogram of the rows that have some over the k buckets, and the total of
+// those nodes.
+// need (may be null): rows with need[r] == 0 get no QAGS nodes.
+__global__ __launch_bounds__(256) void k_rows(const double* __restrict__ pts, int npts, int nrows, FluxParams fp,
+                                              double* __restrict__ row_k, double* __restrict__ row_logd,
+                                              int* __restrict__ row_cnt, const unsigned char* __restrict__ need,
+                                              int* __restrict__ hist, unsigned long long* __restrict__ total)
 {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= nrows) return;
-  row_setup(pts, npts, r, fp, &row_k[r], &row_logd[r], &row_cnt[r]);
-  if (need && !need[r]) row_cnt[r] = 0;
+  int cnt = 0;
+  if (r < nrows) {
+    double k;
+    row_setup(pts, npts, r, fp, &k, &row_logd[r], &cnt);
+    if (need && !need[r]) cnt = 0;
+    row_k[r] = k;
+    row_cnt[r] = cnt;
+    if (cnt > 0) atomicAdd(&hist[row_bucket(k, kRowsPerOctave)], 1);
+  }
+  if (fp.isPoint) return;
+  for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
+  if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(total, (unsigned long long)cnt);
 }
 
-// Point-charge flux for nodes with b > 2R (or FLUX_POINT 1); QAGS task ids
-// for the others.
+// Exclusive prefix sums of the kRowBuckets row counts (in place), their total
+// in *nrows.  One block: 10 buckets per thread, wave scans.
+__global__ __launch_bounds__(1024) void k_row_offsets(int* __restrict__ hist, unsigned long long* __restrict__ nrows)
+{
+  constexpr int kPer = kRowBuckets / 1024;
+  __shared__ int wsum[16];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  int v[kPer], s = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    v[i] = hist[t * kPer + i];
+    s += v[i];
+  }
+  int inc = s;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(inc, o);
+    if (lane >= o) inc += u;
+  }
+  if (lane == 63) wsum[wv] = inc;
+  __syncthreads();
+  int base = inc - s;
+  for (int w = 0; w < wv; ++w) base += wsum[w];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    hist[t * kPer + i] = base;
+    base += v[i];
+  }
+  if (t == 1023) *nrows = (unsigned long long)base;
+}
+
+// Point-charge flux of the nodes with b > 2R (or FLUX_POINT 1), and the rank
+// of each row that has form-factor nodes in the order of k (off: the bucket
+// offsets, advanced here; perm may be null: no order needed).
 // row_need (may be null): rows that no needed bin reads are skipped.
 __global__ void k_flux_point_rows(int nrows, FluxParams fp, const double* __restrict__ row_k,
                                   const double* __restrict__ row_logd, const int* __restrict__ row_cnt,
-                                  const long long* __restrict__ row_off, double* __restrict__ flux,
-                                  TaskRec* __restrict__ recs, const unsigned char* __restrict__ row_need)
+                                  double* __restrict__ flux, int* __restrict__ off, int* __restrict__ perm,
+                                  const unsigned char* __restrict__ row_need)
 {
   const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (gid >= (long)nrows * kNB1) return;
   const long r = gid / kNB1;
   if (row_need && !row_need[r]) return;
-  point_row_node(r, (int)(gid % kNB1), fp, row_k, row_logd, row_cnt, row_off, flux, recs);
+  const int j = (int)(gid % kNB1);
+  if (perm && j == 0 && row_cnt[r] > 0) perm[atomicAdd(&off[row_bucket(row_k[r], kRowsPerOctave)], 1)] = (int)r;
+  point_row_node(r, j, fp, row_k, row_logd, row_cnt, flux);
 }
 
 // ---------------------------------------------------------------------------
@@ -71,55 +121,90 @@ __global__ void k_flux_point_rows(int nrows, FluxParams fp, const double* __rest
 // ---------------------------------------------------------------------------
 static inline int nblk(long n, int bs) { return (int)((n + bs - 1) / bs); }
 
-static int qags_persistent_blocks()
+static int qags_persistent_blocks(int per_cu)
 {
   int dev = 0, ncu = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   if (ncu <= 0) ncu = 256;
-  return ncu * kQagsBlocksPerCu;  // as many workgroups as stay resident
+  return ncu * per_cu;  // as many workgroups as stay resident
 }
 
-// QAGS nodes of one flux row are at most 97: node j has b_j >= bmin e^{j logd}
-// with bmin = 0.05 R and logd >= ln(5R / bmin) / 120, so b_j <= 2R needs
-// j <= 120 ln 40 / ln 100 = 96.09.
-constexpr int kMaxQagsNodesPerRow = 98;
+// Lanes per integral for a launch of about n form-factor integrals (1: one
+// per lane, k_flux_qags_rows or k_flux_qags).  Wider teams shorten an
+// integral's serial chain but spend more issue slots on it (sums and
+// bookkeeping run on every lane), so the width falls as the count fills the
+// chip.  Whole calls, ms (lumi_points up to 3200 points, the contraction's
+// 0.1 included; flux_form 5000 to 100000):
+//   integrals     64      16       8       1 lane each
+//        140   0.145   0.172   0.196   0.609
+//       4620   0.211   0.194   0.211   0.641
+//      28000   0.521   0.311   0.301   0.630
+//     112000   1.61    0.751   0.648   0.667
+//     448000   5.99    2.60    2.13    1.10
+//   5000 pts   0.136   0.119   0.147   0.464
+//  50000 pts   0.748   0.393   0.331   0.478
+// 100000 pts   1.41    0.707   0.568   0.573
+constexpr int kQagsNodesPerRow = 70;  // form-factor nodes of a typical row
 
-// Work buffers for npts points and their flux rows (at most 2 npts); task
-// records, offsets and overflow lists are 64-bit.  The point-charge flux has
-// no QAGS tasks, so its task buffers stay minimal; the per-point form-factor
-// call needs `tasks` of them (its point indices).
-static int ensure_work(upc_ctx* c, size_t npts, size_t rows, size_t tasks = 0)
+static int qags_team(long long n) { return n <= 2048 ? 64 : (n <= 24576 ? 16 : (n <= 98304 ? 8 : 1)); }
+
+template <class TS>
+static void launch_qags_team(int team, const TS& ts, long long ids, double* flux, int* ier,
+                             unsigned long long* counters, long long* overflow, int cap, hipStream_t s)
+{
+  const dim3 grid((unsigned)((ids * team + kQagsBlock - 1) / kQagsBlock)), block(kQagsBlock);
+  if (team == 64)
+    hipLaunchKernelGGL((k_flux_qags_team<64, kQagsCap, TS>), grid, block, 0, s, ts, flux, ier, counters, overflow, cap);
+  else if (team == 16)
+    hipLaunchKernelGGL((k_flux_qags_team<16, kQagsCap, TS>), grid, block, 0, s, ts, flux, ier, counters, overflow, cap);
+  else
+    hipLaunchKernelGGL((k_flux_qags_team<8, kQagsCap, TS>), grid, block, 0, s, ts, flux, ier, counters, overflow, cap);
+}
+
+// Work buffers for npts points and their flux rows (at most 2 npts).  The
+// point-charge flux has no QAGS integrals, so its overflow list stays minimal;
+// the per-point form-factor call needs `points_ff` point indices and as many
+// overflow entries.
+static int ensure_work(upc_ctx* c, size_t npts, size_t rows, size_t points_ff = 0)
 {
   LumiWork& w = c->work;
-  const size_t need_tasks = std::max<size_t>(
-      {tasks, c->cfg.flux_point ? (size_t)1 : rows * kMaxQagsNodesPerRow, (size_t)1});
-  if (rows <= w.rows_cap && npts <= w.points_cap && need_tasks <= w.tasks_cap) return 0;
+  const size_t need_over = std::max<size_t>(
+      {points_ff, c->cfg.flux_point ? (size_t)1 : rows * kMaxQagsNodesPerRow, (size_t)1});
+  if (rows <= w.rows_cap && npts <= w.points_cap && need_over <= w.over_cap && points_ff <= w.idx_cap) return 0;
   rows = std::max(rows, w.rows_cap);
   npts = std::max(npts, w.points_cap);
-  const size_t ntask = std::max(need_tasks, w.tasks_cap);
+  const size_t nover = std::max(need_over, w.over_cap), nidx = std::max({points_ff, w.idx_cap, (size_t)1});
   free_work(c);
   UPC_HIP(hipMalloc(&w.d_row_k, sizeof(double) * rows));
   UPC_HIP(hipMalloc(&w.d_row_logd, sizeof(double) * rows));
   UPC_HIP(hipMalloc(&w.d_row_cnt, sizeof(int) * rows));
-  UPC_HIP(hipMalloc(&w.d_row_off, sizeof(long long) * rows));
+  UPC_HIP(hipMalloc(&w.d_perm, sizeof(int) * rows));
   UPC_HIP(hipMalloc(&w.d_flux, sizeof(double) * rows * kNB1));
-  UPC_HIP(hipMalloc(&w.d_tasks, sizeof(TaskRec) * ntask));
-  UPC_HIP(hipMalloc(&w.d_overflow, sizeof(long long) * ntask));
-  UPC_HIP(hipMalloc(&w.d_counters, sizeof(unsigned long long) * 8));
+  UPC_HIP(hipMalloc(&w.d_idx, sizeof(int) * nidx));
+  UPC_HIP(hipMalloc(&w.d_overflow, sizeof(long long) * nover));
+  UPC_HIP(hipMalloc(&w.d_counters, sizeof(unsigned long long) * 8 + sizeof(int) * kRowBuckets));
+  w.d_hist = (int*)(w.d_counters + 8);
   UPC_HIP(hipMalloc(&w.d_points, sizeof(double) * 4 * npts));
-  UPC_HIP(hipMalloc(&w.d_part, sizeof(long long) * ((rows + 1023) / 1024 + 1)));
   w.rows_cap = rows;
-  w.tasks_cap = ntask;
+  w.over_cap = nover;
+  w.idx_cap = nidx;
   w.points_cap = npts;
   return 0;
+}
+
+// What the points kernels clear before a flux launch: the counters and, where
+// rows are sorted, the histogram behind them.
+static int flux_clear_ints(const upc_ctx* c)
+{
+  return (int)(sizeof(unsigned long long) * 8 / sizeof(int)) + (c->cfg.flux_point ? 0 : kRowBuckets);
 }
 
 void free_work(upc_ctx* c)
 {
   LumiWork& w = c->work;
-  void* ptrs[] = {w.d_row_k, w.d_row_logd, w.d_row_cnt, w.d_row_off, w.d_flux,
-                  w.d_tasks, w.d_overflow, w.d_counters, w.d_points, w.d_part};
+  void* ptrs[] = {w.d_row_k, w.d_row_logd, w.d_row_cnt, w.d_perm, w.d_flux,
+                  w.d_idx, w.d_overflow, w.d_counters, w.d_points};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   w = LumiWork{};
@@ -141,27 +226,31 @@ static int run_flux(upc_ctx* c, int npts, int mirror_ny, hipStream_t s, const un
   LumiWork& w = c->work;
   const FluxParams fp = flux_params(c, mirror_ny);
   const int nrows = flux_rows(npts, mirror_ny);
+  // a restricted grid has few rows of many: only the sort knows how many
+  const int team = row_need ? 1 : qags_team((long long)nrows * kQagsNodesPerRow);
+  const bool sorted = !c->cfg.flux_point && team == 1;
   {
   PhaseScope ph(c, s, UPC_PHASE_FLUX);
-  UPC_HIP(hipMemsetAsync(w.d_counters, 0, sizeof(unsigned long long) * 8, s));
   hipLaunchKernelGGL(k_rows, dim3(nblk(nrows, 256)), dim3(256), 0, s, w.d_points, npts, nrows, fp, w.d_row_k,
-                     w.d_row_logd, w.d_row_cnt, row_need);
-  const int nparts = nblk(nrows, kScanBlock);
-  hipLaunchKernelGGL(k_scan_part<>, dim3(nparts), dim3(kScanBlock), 0, s, w.d_row_cnt, (long)nrows, w.d_part);
-  hipLaunchKernelGGL(k_scan_top<>, dim3(1), dim3(kScanBlock), 0, s, w.d_part, nparts, w.d_counters + 4);
-  hipLaunchKernelGGL(k_scan_apply<>, dim3(nparts), dim3(kScanBlock), 0, s, w.d_row_cnt, (long)nrows, w.d_part,
-                     w.d_row_off);
+                     w.d_row_logd, w.d_row_cnt, row_need, w.d_hist, w.d_counters + 4);
+  if (sorted)
+    hipLaunchKernelGGL(k_row_offsets, dim3(1), dim3(1024), 0, s, w.d_hist, w.d_counters + 6);
   hipLaunchKernelGGL(k_flux_point_rows, dim3(nblk((long)nrows * kNB1, 256)), dim3(256), 0, s, nrows, fp,
-                     w.d_row_k, w.d_row_logd, w.d_row_cnt, w.d_row_off, w.d_flux, (TaskRec*)w.d_tasks, row_need);
+                     w.d_row_k, w.d_row_logd, w.d_row_cnt, w.d_flux, w.d_hist, sorted ? w.d_perm : nullptr, row_need);
   UPC_HIP(hipGetLastError());
   }
   if (!c->cfg.flux_point) {
     PhaseScope ph(c, s, UPC_PHASE_QAGS);
-    GridTask ts{(const TaskRec*)w.d_tasks, fp, c->d_ff};
-    hipLaunchKernelGGL((k_flux_qags<kQagsCap, GridTask>), dim3(qags_persistent_blocks()), dim3(kQagsBlock), 0, s,
-                       ts, w.d_counters + 4, w.d_counters + 5, w.d_flux, (int*)nullptr, w.d_counters,
-                       w.d_overflow, c->qags_cap);
-    hipLaunchKernelGGL((k_flux_qags_wave<GridTask>), dim3(kQagsWaveBlocks), dim3(64), 0, s, ts, w.d_overflow,
+    const GridRows rs{w.d_row_k, w.d_row_logd, w.d_row_cnt, w.d_perm,
+                      RowJob{c->d_ff, fp.bmin, fp.g1, fp.factor, fp.A}, nrows};
+    if (team > 1)
+      launch_qags_team(team, rs, (long long)nrows * kMaxQagsNodesPerRow, w.d_flux, nullptr, w.d_counters,
+                       w.d_overflow, c->qags_cap, s);
+    else
+      hipLaunchKernelGGL((k_flux_qags_rows<kQagsCap, GridRows>), dim3(qags_persistent_blocks(kQagsRowsBlocksPerCu)),
+                         dim3(kQagsBlock), 0, s, rs, w.d_counters + 6, w.d_counters + 5, w.d_flux, w.d_counters,
+                         w.d_overflow, c->qags_cap);
+    hipLaunchKernelGGL((k_flux_qags_wave<GridRows>), dim3(kQagsWaveBlocks), dim3(64), 0, s, rs, w.d_overflow,
                        w.d_counters, w.d_flux, (int*)nullptr);
     UPC_HIP(hipGetLastError());
   }
@@ -183,15 +272,16 @@ int make_grid_points(upc_ctx* c, hipStream_t s)
   int rc = ensure_work(c, (size_t)npts, (size_t)flux_rows((int)npts, grid_mirror_ny(c, true)));
   if (rc) return rc;
   hipLaunchKernelGGL(k_grid_points, dim3(nblk(npts, 256)), dim3(256), 0, s, g.nm, g.mmin, g.mmax, g.ny,
-                     g.ymin, g.ymax, c->work.d_points);
+                     g.ymin, g.ymax, c->work.d_points, (int*)c->work.d_counters, flux_clear_ints(c));
   UPC_HIP(hipGetLastError());
   return 0;
 }
 
 __global__ void k_copy_points(const double* __restrict__ M, const double* __restrict__ Y, int n,
-                              double* __restrict__ pts)
+                              double* __restrict__ pts, int* __restrict__ clear, int nclear)
 {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  for (long l = i; l < nclear; l += (long)gridDim.x * blockDim.x) clear[l] = 0;
   if (i >= n) return;
   pts[4 * i] = M[i];
   pts[4 * i + 1] = Y[i];
@@ -206,7 +296,7 @@ int prepare_flux(upc_ctx* c, const double* d_pts, int npts, FluxParams* fp, hipS
   if (rc) return rc;
   if (d_pts) {
     hipLaunchKernelGGL(k_copy_points, dim3(nblk(npts, 256)), dim3(256), 0, s, d_pts, d_pts + npts, npts,
-                       c->work.d_points);
+                       c->work.d_points, (int*)c->work.d_counters, flux_clear_ints(c));
   }
   rc = run_flux(c, npts, mirror_ny, s);
   if (rc) return rc;
@@ -461,8 +551,8 @@ __global__ void k_zero_u64(unsigned long long* __restrict__ p, int n)
 }
 
 // The per-point form-factor flux on the buffers in w: classify (point flux
-// beyond 2R, QAGS tasks inside), the persistent QAGS kernel, then the
-// 1000-interval kernel for the tasks that outgrew the fast list.  Counters are cleared by a kernel, so the sequence may be captured.
+// beyond 2R, QAGS tasks inside), the QAGS kernel for that many points, then
+// the 1000-interval kernel for the tasks that outgrew the fast list.  Counters are cleared by a kernel, so the sequence may be captured.
 int enqueue_flux_form(upc_ctx* c, const double* d_b, const double* d_k, int n, double* d_out, int* d_ier,
                       const FluxFormBufs& w, hipStream_t s)
 {
@@ -470,9 +560,13 @@ int enqueue_flux_form(upc_ctx* c, const double* d_b, const double* d_k, int n, d
   hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, w.counters, 8);
   hipLaunchKernelGGL(k_flux_form_classify, dim3(nblk(n, 256)), dim3(256), 0, s, d_b, d_k, n, fp, d_out, d_ier,
                      w.idx, w.counters);
-  PointTask ts{d_b, d_k, w.idx, fp, c->d_ff};
-  hipLaunchKernelGGL((k_flux_qags<kQagsCap, PointTask>), dim3(qags_persistent_blocks()), dim3(kQagsBlock), 0, s,
-                     ts, w.counters + 4, w.counters + 5, d_out, d_ier, w.counters, w.overflow, c->qags_cap);
+  PointTask ts{d_b, d_k, w.idx, fp, c->d_ff, w.counters + 4};
+  const int team = qags_team(n);
+  if (team > 1)
+    launch_qags_team(team, ts, n, d_out, d_ier, w.counters, w.overflow, c->qags_cap, s);
+  else
+    hipLaunchKernelGGL((k_flux_qags<kQagsCap, PointTask>), dim3(qags_persistent_blocks(kQagsBlocksPerCu)),
+                     dim3(kQagsBlock), 0, s, ts, w.counters + 4, w.counters + 5, d_out, d_ier, w.counters, w.overflow, c->qags_cap);
   hipLaunchKernelGGL((k_flux_qags_wave<PointTask>), dim3(kQagsWaveBlocks), dim3(64), 0, s, ts, w.overflow,
                      w.counters, d_out, d_ier);
   UPC_HIP(hipGetLastError());
@@ -483,11 +577,10 @@ int launch_flux_form(upc_ctx* c, const double* d_b, const double* d_k, int n, do
                      hipStream_t s)
 {
   if (n <= 0) return 0;
-  // the per-point QAGS keeps its n point indices in the task buffer
   int rc = ensure_work(c, 1, 1, (size_t)n);
   if (rc) return rc;
   LumiWork& w = c->work;
-  const FluxFormBufs bufs{(int*)w.d_tasks, w.d_overflow, w.d_counters};
+  const FluxFormBufs bufs{w.d_idx, w.d_overflow, w.d_counters};
   rc = enqueue_flux_form(c, d_b, d_k, n, d_out, d_ier, bufs, s);
   if (rc) return rc;
   return read_stats(c, s);

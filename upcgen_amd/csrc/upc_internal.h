@@ -38,19 +38,25 @@ constexpr int kMaxEE = 1024;  // calcBreakupProb energy table capacity (referenc
 constexpr int kBkGuard = 96;
 constexpr int kNBkUsed = 20000 + kBkGuard;
 
+// Rows are bucketed by photon energy at 256 buckets per octave (0.3 %): on the
+// 1001 x 121 grid a group of 64 rows spans three buckets.
+constexpr int kRowsPerOctave = 256;
+constexpr int kRowBuckets = 40 * kRowsPerOctave;
+
 struct LumiWork {
   size_t rows_cap = 0;
   double* d_row_k = nullptr;      // photon energy of each flux row
   double* d_row_logd = nullptr;   // log step of the row's b grid
   int* d_row_cnt = nullptr;       // number of QAGS nodes in the row
-  long long* d_row_off = nullptr; // exclusive scan of d_row_cnt
+  int* d_perm = nullptr;          // rows with QAGS nodes, ordered by photon energy
   double* d_flux = nullptr;       // [rows][120]
-  size_t tasks_cap = 0;
-  void* d_tasks = nullptr;        // QAGS task records (b, k, flux slot); per-point calls: point indices
-  unsigned long long* d_counters = nullptr;  // [0] task cursor, [1] qags bad, [2] evals, [3] overflow n
+  size_t idx_cap = 0, over_cap = 0;
+  int* d_idx = nullptr;           // per-point calls: point indices
+  // [0] evals [1] qags bad [2] overflow n [4] integrals [5] cursor [6] rows in d_perm
+  unsigned long long* d_counters = nullptr;
+  int* d_hist = nullptr;          // [kRowBuckets] behind d_counters: rows per k bucket, then their offsets
   long long* d_overflow = nullptr;  // tasks that exceeded the fast workspace
   double* d_points = nullptr;     // (M, Y, dm, dy) per point
-  long long* d_part = nullptr;    // per-block partial sums of the row-count scan
   size_t points_cap = 0;
 };
 
