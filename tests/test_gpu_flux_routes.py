@@ -1,6 +1,6 @@
 """The form-factor flux integrals take one of several kernels by their number
-(teams of 64, 16 or 8 lanes per integral, or one lane per integral with rows
-grouped by photon energy).  Every route runs the same dqagse arithmetic, so a
+(teams of 64, 16 or 8 lanes per integral, one lane per integral with rows
+grouped by photon energy, or that with shared integrand factors).  Every route runs the same dqagse arithmetic, so a
 point's luminosity must not depend on how many points were asked for with it:
 1e-11 relative between routes (the integrand may differ by rounding, which
 the contraction of these Pb-Pb points amplifies by less than 1e3), and 1e-9
@@ -48,6 +48,38 @@ def test_evaluation_counts_add_up(gpu, data):
         c.lumi_points(t(M[a:b].copy()), t(Y[a:b].copy()))
         total += c.info.qags_evals
     assert total == evals
+
+
+# the fewest rows that share factors, one group and one row more, and more
+# than one launch's groups (262,144 rows)
+@pytest.mark.parametrize("n", [4096, 4129, 131105])
+def test_shared_factors_do_not_change_a_point(gpu, data, n):
+    import torch
+    c = data[0]
+    rng = np.random.default_rng(n)
+    M = np.exp(rng.uniform(np.log(2.0), np.log(60.0), n))
+    Y = rng.uniform(-3.5, 3.5, n)
+    t = lambda x: torch.as_tensor(x, device="cuda")
+    L = c.lumi_points(t(M), t(Y)).cpu().numpy()
+    assert c.info.qags_bad == 0
+    idx = rng.choice(n, 700, replace=False)
+    one = c.lumi_points(t(M[idx]), t(Y[idx])).cpu().numpy()
+    assert np.max(np.abs(L[idx] - one) / np.abs(one)) <= 1e-11
+
+
+def test_shared_factors_evaluation_counts(gpu, data):
+    import torch
+    c = data[0]
+    rng = np.random.default_rng(3)
+    M = np.exp(rng.uniform(np.log(2.0), np.log(60.0), 6150))
+    Y = rng.uniform(-3.5, 3.5, 6150)
+    t = lambda x: torch.as_tensor(x, device="cuda")
+    c.lumi_points(t(M), t(Y))  # 12,300 rows share factors, 2,460 do not
+    whole, total = c.info.qags_evals, 0
+    for a in range(0, 6150, 1230):
+        c.lumi_points(t(M[a:a + 1230].copy()), t(Y[a:a + 1230].copy()))
+        total += c.info.qags_evals
+    assert total == whole
 
 
 def test_points_against_oracle(data, oracle_ctx):

@@ -22,7 +22,7 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libupcgen_amd.so")
 EXE = os.path.join(HERE, "upcgen")
 
-HIP_SOURCES = ["upc_capi.hip", "upc_tables.hip", "upc_flux_lumi.hip", "upc_xsec.hip", "upc_mfma.hip",
+HIP_SOURCES = ["upc_capi.hip", "upc_tables.hip", "upc_flux_lumi.hip", "upc_flux_rows.hip", "upc_lumi.hip", "upc_xsec.hip", "upc_mfma.hip",
                "upc_surrogate.hip", "upc_events.hip", "upc_batch.hip", "upc_noalloc.hip"]
 CXX_SOURCES = ["UpcCrossSection.cpp", "UpcGenerator.cpp"]
 
@@ -32,6 +32,15 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", f"-I{os.path.join(ROOT, 'include')}", f"
 # Packed-FP32 VALU forms are disabled for every HIP translation unit.
 HIPFLAGS = COMMON + [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                      "-munsafe-fp-atomics", "-Wno-unused-command-line-argument"]
+# The QAGS kernels run at their register budget: without this the compiler lifts
+# address and constant computations out of their long loops and spills them
+# (k_flux_qags_team 164 -> 122 VGPRs, k_flux_qags_table 60 -> 0 spilled).
+QAGS_FLAGS = ["-mllvm", "-disable-machine-licm"]
+QAGS_SOURCES = {"upc_flux_lumi.hip", "upc_batch.hip", "upc_noalloc.hip"}
+
+
+def _hip_flags(src: str) -> list:
+    return HIPFLAGS + (QAGS_FLAGS if src in QAGS_SOURCES else [])
 
 
 def _run(cmd):
@@ -45,7 +54,7 @@ def _compile(src: str) -> str:
     path = os.path.join(CSRC, src)
     obj = os.path.join(BUILD, os.path.splitext(src)[0] + ".o")
     # host-only C++ of the facade is compiled as HIP too: it calls the HIP runtime
-    flags = HIPFLAGS
+    flags = _hip_flags(src)
     extra = ["-x", "hip"]
     _run([HIPCC] + flags + extra + ["-c", path, "-o", obj])
     return obj
@@ -86,7 +95,7 @@ def resources(name_filter: str = "") -> list:
     with tempfile.TemporaryDirectory() as tmp:
         for src in HIP_SOURCES:
             asm = os.path.join(tmp, src + ".s")
-            _run([HIPCC] + HIPFLAGS + ["--cuda-device-only", "-S", "-x", "hip", os.path.join(CSRC, src), "-o", asm])
+            _run([HIPCC] + _hip_flags(src) + ["--cuda-device-only", "-S", "-x", "hip", os.path.join(CSRC, src), "-o", asm])
             text = open(asm).read()
             for m in re.finditer(r"\n  - \.agpr_count:(.*?)(?=\n  - \.|\n\.end_amdgpu_metadata)", text, re.S):
                 block = m.group(0)

@@ -1,5 +1,5 @@
 """Generate upc_coeffs.h: Chebyshev / power-series coefficients for the device
-Bessel functions J1, K0, K1 used by the photon-flux kernels.
+Bessel functions J0, J1, K0, K1 used by the photon-flux kernels.
 
 The functions are defined by the mathematics (DLMF 10.2, 10.17, 10.25, 10.31,
 10.40); the coefficients are computed here with mpmath at 50 digits and
@@ -92,10 +92,15 @@ def main():
     out.append("// J1(x)/x = sum c_k T_k(x^2/32 - 1), 0 <= x <= 8")
     out.append(emit("kJ1Small", j1s))
 
+    # J0 likewise (J1' = J0 - J1/x).
+    j0s = cheb_coeffs(lambda u: mp.besselj(0, mp.sqrt(32 * (u + 1))), -1, 1, atol=mp.mpf("1e-17"))
+    out.append("// J0(x) = sum c_k T_k(x^2/32 - 1), 0 <= x <= 8")
+    out.append(emit("kJ0Small", j0s))
+
     # Hankel modulus/phase form for x >= 8, s = 64/x^2 in (0, 1] -> v = 2 s - 1.
-    def pq(x):
-        chi = x - 3 * mp.pi / 4
-        j, y = mp.besselj(1, x), mp.bessely(1, x)
+    def pq(x, nu=1):
+        chi = x - (2 * nu + 1) * mp.pi / 4
+        j, y = mp.besselj(nu, x), mp.bessely(nu, x)
         f = mp.sqrt(mp.pi * x / 2)
         P = f * (j * mp.cos(chi) + y * mp.sin(chi))
         Q = f * (y * mp.cos(chi) - j * mp.sin(chi))
@@ -126,6 +131,25 @@ def main():
     out.append("// P = sum p_k v^k, Q = (8/x) sum q_k v^k, v = 128/x^2 - 1")
     out.append(emit("kJ1P", cheb_to_mono(pc)))
     out.append(emit("kJ1Q", cheb_to_mono(qc)))
+
+    def P0_of_v(v):
+        s = (v + 1) / 2
+        return mp.mpf(1) if s == 0 else pq(8 / mp.sqrt(s), 0)[0]
+
+    def Q0_of_v(v):
+        s = (v + 1) / 2
+        if s == 0:
+            return -mp.mpf(1) / 64
+        x = 8 / mp.sqrt(s)
+        return pq(x, 0)[1] * x / 8
+
+    pc = cheb_coeffs(P0_of_v, -1, 1, atol=mp.mpf("1e-17"))
+    qc = cheb_coeffs(Q0_of_v, -1, 1, atol=mp.mpf("1e-17"))
+    n = max(len(pc), len(qc))
+    pc, qc = pc + [mp.mpf(0)] * (n - len(pc)), qc + [mp.mpf(0)] * (n - len(qc))
+    out.append("// J0(x) = (P (sin x + cos x) - Q (sin x - cos x)) / sqrt(pi x), x >= 8, P, Q in v as for J1")
+    out.append(emit("kJ0P", cheb_to_mono(pc)))
+    out.append(emit("kJ0Q", cheb_to_mono(qc)))
 
     # sin r = r + r^3 S(r^2), cos r = 1 - r^2/2 + r^4 C(r^2) on |r| <= pi/4
     # (after reduction by pi/2); absolute errors 1.4e-17 and 9e-19.

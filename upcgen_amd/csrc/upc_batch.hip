@@ -7,14 +7,15 @@
 // factor, breakup), and the grid work of all jobs is concatenated:
 //   points [sum npts], flux rows [sum nrows][120].
 // One kernel per stage serves all jobs (a job table in HBM maps a point,
-// row or block to its job), so the QAGS integrals of every job share one
-// persistent launch and its cursor (rows sorted by job, then by photon
-// energy), and the contraction is one launch.
+// row, group of rows or block to its job), so the QAGS integrals of all jobs
+// share two persistent launch sequences (rows sorted by job, then by photon
+// energy; jobs with many rows, jobs with few), and the contraction is one
+// launch.
 // The sequence is captured once into a hipGraph and replayed; buffers are
 // cleared by kernels (no memset nodes).  The launch shapes (QAGS workgroups
 // per CU, contraction waves per block) are chosen by timing the candidates
 // on the batch itself.
-#include "upc_flux.h"
+#include "upc_batch_job.h"
 
 #include <algorithm>
 #include <climits>
@@ -23,14 +24,6 @@
 struct upc_batch;
 
 namespace upc {
-
-struct BatchJob {
-  LumiView v;          // pts, row_logd, flux point at this job's slice
-  const double4* ff;
-  int nm, ny;
-  double mmin, mmax, ymin, ymax;
-  int pt0, row0;       // first point and row of the job in the batch arrays
-};
 
 // upc_mfma.hip: the MFMA contraction of one view, on a state of the batch's own
 void* mfma_state_create(double h);
@@ -43,22 +36,6 @@ int mfma_read_counts(void* st, unsigned long long* h_out, hipStream_t s);
 constexpr int kLumiWaveChoices[3] = {2, 4, 8};
 constexpr int kMfmaTileChoices[3] = {1, 2, 4};  // column tiles per A-fragment load (MFMA form)
 constexpr int kQagsBlockChoices[3] = {1, 2, 3};  // workgroups of 256 per CU; the last choice fills the CU
-static int qags_blocks_per_cu(int choice) { return choice == 2 ? kQagsRowsBlocksPerCu : kQagsBlockChoices[choice]; }
-
-// Buckets of the row sort: per job, 64 per octave of k.
-constexpr int kBatchPerOctave = 64;
-constexpr int kBatchBuckets = kRowOctaves * kBatchPerOctave;
-
-__device__ __forceinline__ int find_job(const int* __restrict__ start, int njobs, long idx)
-{
-  int lo = 0, hi = njobs - 1;  // largest j with start[j] <= idx
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (start[mid] <= idx) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
 
 __global__ void k_batch_zero(unsigned long long* __restrict__ p, int n)
 {
@@ -82,19 +59,19 @@ __global__ void k_batch_points(const BatchJob* __restrict__ jobs, const int* __r
   pts[4 * idx + 3] = dy;
 }
 
-// Clears the batch's counters, its jobs' failure counts and the row histogram.
-__global__ void k_batch_clear(unsigned long long* __restrict__ counters, unsigned long long* __restrict__ job_failed,
-                              int njobs, int* __restrict__ hist, int nhist)
+// Clears the batch's counters and cursors, its jobs' failure counts and the row histogram.
+__global__ void k_batch_clear(unsigned long long* __restrict__ counters, int ncounters,
+                              unsigned long long* __restrict__ job_failed, int njobs, int* __restrict__ hist, long nhist)
 {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < 8) counters[i] = 0;
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < ncounters) counters[i] = 0;
   if (i < njobs) job_failed[i] = 0;
   if (i < nhist) hist[i] = 0;
 }
 
-__device__ __forceinline__ int batch_bucket(int job, double k)
+__device__ __forceinline__ size_t batch_bucket(int job, double k)
 {
-  return job * kBatchBuckets + row_bucket(k, kBatchPerOctave);
+  return (size_t)job * kRowBuckets + row_bucket(k);
 }
 
 __global__ __launch_bounds__(256) void k_batch_rows(const BatchJob* __restrict__ jobs, const int* __restrict__ row0,
@@ -120,7 +97,7 @@ __global__ __launch_bounds__(256) void k_batch_rows(const BatchJob* __restrict__
 __global__ void k_batch_point_rows(const BatchJob* __restrict__ jobs, const int* __restrict__ row0, int njobs,
                                    long total_rows, const double* __restrict__ row_k,
                                    const double* __restrict__ row_logd, const int* __restrict__ row_cnt,
-                                   double* __restrict__ flux, unsigned long long* __restrict__ off,
+                                   double* __restrict__ flux, int* __restrict__ off,
                                    int* __restrict__ perm)
 {
   const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -128,58 +105,9 @@ __global__ void k_batch_point_rows(const BatchJob* __restrict__ jobs, const int*
   const long r = gid / kNB1;
   const int j = (int)(gid % kNB1);
   const int jb = find_job(row0, njobs, r);
-  if (j == 0 && row_cnt[r] > 0) perm[atomicAdd(&off[batch_bucket(jb, row_k[r])], 1ull)] = (int)r;
+  if (j == 0 && row_cnt[r] > 0) perm[atomicAdd(&off[batch_bucket(jb, row_k[r])], 1)] = (int)r;
   point_row_node(r, j, jobs[jb].v.fp, row_k, row_logd, row_cnt, flux);
 }
-
-// Flux rows of all jobs for the QAGS kernels; as a task source, task t = row
-// * 120 + node (its flux slot).
-struct BatchRows {
-  static constexpr bool kManyJobs = true;
-  const double* __restrict__ row_k;
-  const double* __restrict__ row_logd;
-  const int* __restrict__ row_cnt;
-  const int* __restrict__ perm;
-  const BatchJob* __restrict__ jobs;
-  const int* __restrict__ row0;
-  int njobs;
-  unsigned long long* __restrict__ job_failed;  // [njobs] integrals with ier != 0
-  __device__ int job_of(int r) const { return find_job(row0, njobs, r); }
-  __device__ RowJob params(int job) const
-  {
-    const BatchJob& J = jobs[job];
-    return RowJob{J.ff, J.v.fp.bmin, J.v.fp.g1, J.v.fp.factor, J.v.fp.A};
-  }
-  __device__ void failed(int job) const { atomicAdd(&job_failed[job], 1ull); }
-  __device__ void get(long long t, FluxTask* ft) const
-  {
-    const long long r = t / kNB1;
-    const int jb = job_of((int)r);
-    const RowJob P = params(jb);
-    ft->b = row_node_b(P.bmin, row_logd[r], (int)(t - r * kNB1));
-    ft->k = row_k[r];
-    ft->out = t;
-    ft->ff = P.ff;
-    ft->g1 = P.g1;
-    ft->factor = P.factor;
-    ft->A = P.A;
-    ft->slot = jb;
-  }
-};
-
-// Contraction job resolver: blk0[j] = first block of job j for this wave count.
-struct BatchLumi {
-  static constexpr int kWavesPerEu = 4;  // register budget of k_lumi_fp64 (waves per SIMD)
-  const BatchJob* __restrict__ jobs;
-  const int* __restrict__ blk0;
-  int njobs;
-  __device__ void get(int blk, int waves, LumiView* out, int* p0) const
-  {
-    const int j = find_job(blk0, njobs, blk);
-    *out = jobs[j].v;
-    *p0 = (blk - blk0[j]) * waves;
-  }
-};
 
 }  // namespace upc
 
@@ -191,7 +119,7 @@ struct upc_batch {
   std::vector<upc_ctx*> ctx;
   std::vector<BatchJob> jobs;  // host copy (pointers into the batch buffers)
   long npts = 0, nrows = 0;
-  int nparts = 0;
+  long long share_groups = 0, groups = 0;  // groups of rows: of the jobs that share factors (first), in all
   int lumi_blocks[3] = {0, 0, 0};
   BatchJob* d_jobs = nullptr;
   int* d_pt0 = nullptr;
@@ -202,14 +130,17 @@ struct upc_batch {
   double* d_row_logd = nullptr;
   int* d_row_cnt = nullptr;
   int* d_perm = nullptr;         // rows with QAGS nodes, by job and photon energy
-  int* d_hist = nullptr;         // [njobs][kBatchBuckets] rows per bucket
-  long long* d_off = nullptr;    // their offsets in d_perm
-  long long* d_part = nullptr;
+  int* d_hist = nullptr;         // [njobs][kRowBuckets] rows per k bucket, then their offsets in d_perm
+  int* d_group_job = nullptr;    // job of each group of 64 positions in d_perm
+  int* d_nsorted = nullptr;      // [njobs] rows in d_perm
   double* d_flux = nullptr;
   long long ntasks = 0;          // QAGS integrals of every job (counted at creation)
   long long work_bytes = 0;      // device memory of the buffers below
   long long* d_overflow = nullptr;
-  unsigned long long* d_counters = nullptr;  // [0] evals [1] bad [2] overflow n [4] tasks [5] cursor [6] rows in d_perm
+  double* d_h = nullptr;         // integrand factors of one launch's groups of rows
+  int ncursors = 0;
+  // [0] evals [1] bad [2] overflow n [4] tasks, [8..] work cursors of the row QAGS launches
+  unsigned long long* d_counters = nullptr;
   unsigned long long* d_job_failed = nullptr;  // [njobs] QAGS integrals with ier != 0 per job
   int qags_choice = 2, lumi_choice = 1;  // indices into the candidate lists
   int form = UPC_FORM_FP64;              // contraction form of every job
@@ -241,8 +172,8 @@ void free_batch(upc_batch* b)
   if (b->graph) (void)hipGraphDestroy(b->graph);
   if (b->cap_stream) (void)hipStreamDestroy(b->cap_stream);
   void* ptrs[] = {b->d_jobs, b->d_pt0, b->d_row0, b->d_blk0[0], b->d_blk0[1], b->d_blk0[2], b->d_pts,
-                  b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_perm, b->d_hist, b->d_off, b->d_part, b->d_flux,
-                  b->d_overflow, b->d_counters, b->d_job_failed};
+                  b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_perm, b->d_hist, b->d_group_job, b->d_nsorted, b->d_flux,
+                  b->d_overflow, b->d_counters, b->d_job_failed, b->d_h};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   for (upc_ctx* c : b->ctx) upc_ctx_destroy(c);
@@ -266,31 +197,35 @@ int contract_mfma(upc_batch* b, int tile_group, hipStream_t s)
 // Points, row geometry and the row histogram of every job, from cleared counters.
 void enqueue_rows(upc_batch* b, hipStream_t s)
 {
-  const int nj = (int)b->jobs.size(), nhist = nj * kBatchBuckets;
-  hipLaunchKernelGGL(k_batch_clear, dim3(nblk(nhist, 256)), dim3(256), 0, s, b->d_counters, b->d_job_failed, nj,
-                     b->d_hist, nhist);
+  const int nj = (int)b->jobs.size();
+  const long nhist = (long)nj * kRowBuckets;
+  hipLaunchKernelGGL(k_batch_clear, dim3(nblk(nhist, 256)), dim3(256), 0, s, b->d_counters, 8 + b->ncursors,
+                     b->d_job_failed, nj, b->d_hist, nhist);
   hipLaunchKernelGGL(k_batch_points, dim3(nblk(b->npts, 256)), dim3(256), 0, s, b->d_jobs, b->d_pt0, nj,
                      b->npts, b->d_pts);
   hipLaunchKernelGGL(k_batch_rows, dim3(nblk(b->nrows, 256)), dim3(256), 0, s, b->d_jobs, b->d_row0, nj,
                      b->nrows, b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_hist, b->d_counters + 4);
 }
 
-BatchRows batch_rows(const upc_batch* b)
+BatchRows batch_rows(const upc_batch* b, long long g0, long long g1)
 {
   return BatchRows{b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_perm, b->d_jobs, b->d_row0, (int)b->jobs.size(),
-                   b->d_job_failed};
+                   b->d_group_job, b->d_nsorted, g0, g1, b->d_job_failed};
 }
 
 void launch_qags(upc_batch* b, int choice, hipStream_t s)
 {
-  hipLaunchKernelGGL((k_flux_qags_rows<kQagsCap, BatchRows>), dim3(b->ncu * qags_blocks_per_cu(choice)),
-                     dim3(kQagsBlock), 0, s, batch_rows(b), b->d_counters + 6, b->d_counters + 5, b->d_flux,
-                     b->d_counters, b->d_overflow, kQagsCap);
+  unsigned long long* cursors = b->d_counters + 8;
+  const long long m = b->share_groups;
+  launch_qags_rows(true, batch_rows(b, 0, m), m, b->d_h, cursors, b->d_flux, b->d_counters, b->d_overflow, kQagsCap,
+                   b->ncu, kQagsBlockChoices[choice], s);
+  launch_qags_rows(false, batch_rows(b, m, b->groups), b->groups - m, nullptr, cursors + rows_cursors(m), b->d_flux,
+                   b->d_counters, b->d_overflow, kQagsCap, b->ncu, kQagsBlockChoices[choice], s);
 }
 
 void launch_qags_wave(upc_batch* b, hipStream_t s)
 {
-  hipLaunchKernelGGL((k_flux_qags_wave<BatchRows>), dim3(kQagsWaveBlocks), dim3(64), 0, s, batch_rows(b),
+  hipLaunchKernelGGL((k_flux_qags_wave<BatchRows>), dim3(kQagsWaveBlocks), dim3(64), 0, s, batch_rows(b, 0, 0),
                      b->d_overflow, b->d_counters, b->d_flux, (int*)nullptr);
 }
 
@@ -298,25 +233,19 @@ void launch_qags_wave(upc_batch* b, hipStream_t s)
 int enqueue(upc_batch* b, hipStream_t s)
 {
   const int nj = (int)b->jobs.size();
-  const long nhist = (long)nj * kBatchBuckets;
+  const long nhist = (long)nj * kRowBuckets;
   enqueue_rows(b, s);
-  hipLaunchKernelGGL(k_scan_part<>, dim3(b->nparts), dim3(kScanBlock), 0, s, b->d_hist, nhist, b->d_part);
-  hipLaunchKernelGGL(k_scan_top<>, dim3(1), dim3(kScanBlock), 0, s, b->d_part, b->nparts, b->d_counters + 6);
-  hipLaunchKernelGGL(k_scan_apply<>, dim3(b->nparts), dim3(kScanBlock), 0, s, b->d_hist, nhist, b->d_part,
-                     b->d_off);
+  const BatchRows rs = batch_rows(b, 0, b->groups);
+  hipLaunchKernelGGL((k_row_offsets<BatchRows, int>), dim3(nj), dim3(1024), 0, s, rs, b->d_hist, b->d_nsorted);
   hipLaunchKernelGGL(k_batch_point_rows, dim3(nblk(b->nrows * kNB1, 256)), dim3(256), 0, s, b->d_jobs, b->d_row0,
-                     nj, b->nrows, b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_flux,
-                     (unsigned long long*)b->d_off, b->d_perm);
+                     nj, b->nrows, b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_flux, b->d_hist, b->d_perm);
+  if (b->share_groups > 0)
+    hipLaunchKernelGGL(k_row_order<BatchRows>, dim3(nblk(nhist, 4)), dim3(256), 0, s, rs, b->d_hist, (long long)nhist);
   launch_qags(b, b->qags_choice, s);
   launch_qags_wave(b, s);
   if (b->form != UPC_FORM_FP64) return contract_mfma(b, kMfmaTileChoices[b->mfma_choice], s);
-  const int li = b->lumi_choice, w = kLumiWaveChoices[li];
-  BatchLumi jr{b->d_jobs, b->d_blk0[li], nj};
-  if (w == 2) hipLaunchKernelGGL((k_lumi_fp64<2, BatchLumi>), dim3(b->lumi_blocks[li]), dim3(128), 0, s, jr);
-  else if (w == 4) hipLaunchKernelGGL((k_lumi_fp64<4, BatchLumi>), dim3(b->lumi_blocks[li]), dim3(256), 0, s, jr);
-  else hipLaunchKernelGGL((k_lumi_fp64<8, BatchLumi>), dim3(b->lumi_blocks[li]), dim3(512), 0, s, jr);
-  UPC_HIP(hipGetLastError());
-  return 0;
+  const int li = b->lumi_choice;
+  return launch_lumi_batch(b->d_jobs, b->d_blk0[li], nj, kLumiWaveChoices[li], b->lumi_blocks[li], s);
 }
 
 }  // namespace
@@ -363,7 +292,20 @@ int upc_batch_create(const upc_config* cfgs, int njobs, void* stream, upc_batch*
   }
   b->npts = np;
   b->nrows = nr;
-  b->nparts = nblk((long)njobs * kBatchBuckets, kScanBlock);
+  // groups of rows: the jobs dense enough to share factors first (as their own
+  // context would decide), then the others; point-charge jobs have none
+  std::vector<int> grp0(njobs, 0), group_job;
+  for (int share = 1; share >= 0; --share) {
+    for (int j = 0; j < njobs; ++j) {
+      const long n = (j + 1 < njobs ? row0[j + 1] : nr) - row0[j];
+      if (cfgs[j].flux_point || (n >= kQagsShareRows) != (share == 1)) continue;
+      grp0[j] = (int)group_job.size();
+      group_job.insert(group_job.end(), (size_t)rows_groups(n), j);
+    }
+    if (share) b->share_groups = (long long)group_job.size();
+  }
+  b->groups = (long long)group_job.size();
+  b->ncursors = (int)(rows_cursors(b->share_groups) + kXcds);
   for (int i = 0; i < 3; ++i) b->lumi_blocks[i] = (int)blocks[i];
 #define BA(ptr, n)                                                  \
   do {                                                              \
@@ -379,12 +321,12 @@ int upc_batch_create(const upc_config* cfgs, int njobs, void* stream, upc_batch*
     BA(b->d_row_k, nr);
     BA(b->d_row_logd, nr);
     BA(b->d_row_cnt, nr);
-    BA(b->d_perm, nr);
-    BA(b->d_hist, (size_t)njobs * kBatchBuckets);
-    BA(b->d_off, (size_t)njobs * kBatchBuckets);
-    BA(b->d_part, b->nparts);
+    BA(b->d_perm, std::max(64 * b->groups, 1LL));
+    BA(b->d_group_job, std::max(b->groups, 1LL));
+    BA(b->d_nsorted, njobs);
+    BA(b->d_hist, (size_t)njobs * kRowBuckets);
     BA(b->d_flux, nr * kNB1);
-    BA(b->d_counters, 8);
+    BA(b->d_counters, 8 + b->ncursors);
     BA(b->d_job_failed, njobs);
     return 0;
   };
@@ -410,6 +352,7 @@ int upc_batch_create(const upc_config* cfgs, int njobs, void* stream, upc_batch*
     J.v.pol = g.use_polarized;
     J.v.mirror_out = mirror;
     J.ff = c->d_ff;
+    J.j1 = c->d_j1;
     J.nm = g.nm;
     J.ny = g.ny;
     J.mmin = g.mmin;
@@ -418,12 +361,16 @@ int upc_batch_create(const upc_config* cfgs, int njobs, void* stream, upc_batch*
     J.ymax = g.ymax;
     J.pt0 = pt0[j];
     J.row0 = row0[j];
+    J.nrows = (int)((j + 1 < njobs ? row0[j + 1] : nr) - row0[j]);
+    J.grp0 = grp0[j];
     b->jobs.push_back(J);
   }
   auto upload = [&]() -> int {
     UPC_HIP(hipMemcpy(b->d_jobs, b->jobs.data(), sizeof(BatchJob) * njobs, hipMemcpyHostToDevice));
     UPC_HIP(hipMemcpy(b->d_pt0, pt0.data(), sizeof(int) * njobs, hipMemcpyHostToDevice));
     UPC_HIP(hipMemcpy(b->d_row0, row0.data(), sizeof(int) * njobs, hipMemcpyHostToDevice));
+    if (!group_job.empty())
+      UPC_HIP(hipMemcpy(b->d_group_job, group_job.data(), sizeof(int) * group_job.size(), hipMemcpyHostToDevice));
     for (int i = 0; i < 3; ++i)
       UPC_HIP(hipMemcpy(b->d_blk0[i], blk0[i].data(), sizeof(int) * njobs, hipMemcpyHostToDevice));
     UPC_HIP(hipStreamCreateWithFlags(&b->cap_stream, hipStreamNonBlocking));
@@ -445,6 +392,11 @@ int upc_batch_create(const upc_config* cfgs, int njobs, void* stream, upc_batch*
     const size_t n = total > 0 ? (size_t)total : 1;
     UPC_HIP(hipMalloc(&b->d_overflow, sizeof(long long) * n));
     b->work_bytes += (long long)(sizeof(long long) * n);
+    if (b->share_groups > 0) {
+      const size_t h = sizeof(double) * rows_h_elems(b->share_groups);
+      UPC_HIP(hipMalloc(&b->d_h, h));
+      b->work_bytes += (long long)h;
+    }
     return 0;
   };
   if (int rc = size_tasks()) {
@@ -562,7 +514,7 @@ int upc_batch_autotune(upc_batch* b, void* stream, upc_tune* h_out)
   for (int i = 0; i < 3; ++i) {
     // QAGS alone: clear the counters except the integral and row totals, then time
     hipLaunchKernelGGL(k_batch_zero, dim3(1), dim3(64), 0, s, b->d_counters, 4);
-    hipLaunchKernelGGL(k_batch_zero, dim3(1), dim3(64), 0, s, b->d_counters + 5, 1);
+    hipLaunchKernelGGL(k_batch_zero, dim3(nblk(b->ncursors, 64)), dim3(64), 0, s, b->d_counters + 8, b->ncursors);
     UPC_HIP(hipEventRecord(e0, s));
     launch_qags(b, i, s);
     UPC_HIP(hipEventRecord(e1, s));
@@ -591,12 +543,14 @@ int upc_batch_autotune(upc_batch* b, void* stream, upc_tune* h_out)
     t.mfma_ms[i] = ms;
   }
   for (int i = 0; i < 3 && b->form == UPC_FORM_FP64; ++i) {
-    BatchLumi jr{b->d_jobs, b->d_blk0[i], nj};
     UPC_HIP(hipEventRecord(e0, s));
     const int w = kLumiWaveChoices[i];
-    if (w == 2) hipLaunchKernelGGL((k_lumi_fp64<2, BatchLumi>), dim3(b->lumi_blocks[i]), dim3(128), 0, s, jr);
-    else if (w == 4) hipLaunchKernelGGL((k_lumi_fp64<4, BatchLumi>), dim3(b->lumi_blocks[i]), dim3(256), 0, s, jr);
-    else hipLaunchKernelGGL((k_lumi_fp64<8, BatchLumi>), dim3(b->lumi_blocks[i]), dim3(512), 0, s, jr);
+    rc = launch_lumi_batch(b->d_jobs, b->d_blk0[i], nj, w, b->lumi_blocks[i], s);
+    if (rc) {
+      (void)hipEventDestroy(e0);
+      (void)hipEventDestroy(e1);
+      return rc;
+    }
     UPC_HIP(hipEventRecord(e1, s));
     UPC_HIP(hipEventSynchronize(e1));
     float ms = 0;

@@ -193,6 +193,34 @@ __device__ __forceinline__ double bessel_j1(double x)
   return x <= 8.0 ? bessel_j1_small(x) : bessel_j1_large(x);
 }
 
+// J0(x) and J1(x); the J1 is bessel_j1's, operation for operation.
+__device__ __forceinline__ void bessel_j01(double x, double* j0, double* j1)
+{
+  if (x <= 8.0) {
+    *j1 = bessel_j1_small(x);
+    *j0 = clenshaw(kJ0Small, x * x * (1.0 / 32.0) - 1.0);
+    return;
+  }
+  constexpr double kInvSqrtPi = 0.56418958354775628695;
+  const double y = rsqrt_nr(x);
+  const double r = y * y;  // 1/x
+  const double v = fma(128.0 * r, r, -1.0);
+  double P = kJ1P[kJ1P_N - 1], Q = kJ1Q[kJ1Q_N - 1], P0 = kJ0P[kJ0P_N - 1], Q0 = kJ0Q[kJ0Q_N - 1];
+#pragma unroll
+  for (int k = kJ1P_N - 2; k >= 0; --k) {
+    P = fma3(v, P, kJ1P[k]);
+    Q = fma3(v, Q, kJ1Q[k]);
+    P0 = fma3(v, P0, kJ0P[k]);
+    Q0 = fma3(v, Q0, kJ0Q[k]);
+  }
+  Q *= 8.0 * r;
+  Q0 *= 8.0 * r;
+  double s, c;
+  sincos_medium(x, &s, &c);
+  *j1 = (P * (s - c) + Q * (s + c)) * (y * kInvSqrtPi);
+  *j0 = (P0 * (s + c) - Q0 * (s - c)) * (y * kInvSqrtPi);
+}
+
 // K0(x), K1(x) for x > 0 (role of gsl_sf_bessel_K0/K1 in
 // src/UpcCrossSection.cpp:171-172).  Underflows quietly to 0 at large x.
 __device__ __forceinline__ void bessel_k01(double x, double* k0, double* k1)
@@ -453,6 +481,7 @@ __device__ __forceinline__ QK21Out qk21(const F& f, double a, double b)
 // pairs, e = 11..20 the Kronrod-only abscissae xgk(2j - 1) in pairs.
 __device__ __forceinline__ double qk21_abscissa(int e, double centr, double hlgth)
 {
+#pragma clang fp contract(off)  // absc rounded before the sum, as QUADPACK computes it
   const bool gauss = e <= 10;
   const int p = gauss ? (e - 1) >> 1 : (e - 11) >> 1;
   const int side = gauss ? (e - 1) & 1 : (e - 11) & 1;
@@ -519,9 +548,14 @@ __device__ __forceinline__ QK21Out qk21_tail(const GX& gx, double resg, double r
   rasc = rasc * dhlgth;
   double err = fabs((resk - resg) * hlgth);
   if (rasc != 0.0 && err != 0.0) {
-    const double t15 = 200.0 * err / rasc;
-    const double sc = t15 * sqrt(t15);
-    err = rasc * (sc < 1.0 ? sc : 1.0);
+    // (200 err / rasc)^1.5, at least 1 (the quotient rounds to 1 or more) where 200 err >= rasc
+    if (200.0 * err >= rasc) {
+      err = rasc;
+    } else {
+      const double t15 = 200.0 * err / rasc;
+      const double sc = t15 * sqrt(t15);
+      err = rasc * (sc < 1.0 ? sc : 1.0);
+    }
   }
   if (rabs > uflow / (50.0 * epmach)) {
     const double m = (epmach * 50.0) * rabs;
@@ -595,9 +629,10 @@ __device__ __forceinline__ QK21Out qk21_lds(const F& f, double a, double b, doub
   return qk21_sum([&](int, double x) { return f(x); }, a, b, fv, stride);
 }
 
-// dqelg (Wynn epsilon) on a 1-based table of length >= 55.
-__device__ __forceinline__ void qelg(int* n, double* epstab, double* result, double* abserr, double* res3la,
-                            int* nres)
+// dqelg (Wynn epsilon) on the 1-based table of a store (ep, set_ep) and its
+// last three results (r3, set_r3).
+template <class S>
+__device__ __forceinline__ void qelg(S& s, int* n, double* result, double* abserr, int* nres)
 {
   constexpr double epmach = DBL_EPSILON, oflow = DBL_MAX;
   constexpr int limexp = 50;
@@ -606,19 +641,19 @@ __device__ __forceinline__ void qelg(int* n, double* epstab, double* result, dou
       tol1, tol2, tol3;
   (*nres)++;
   *abserr = oflow;
-  *result = epstab[*n];
+  *result = s.ep(*n);
   if (*n < 3) goto L100;
-  epstab[*n + 2] = epstab[*n];
+  s.set_ep(*n + 2, *result);
   newelm = (*n - 1) / 2;
-  epstab[*n] = oflow;
+  s.set_ep(*n, oflow);
   num = *n;
   k1 = *n;
   for (i = 1; i <= newelm; ++i) {
     k2 = k1 - 1;
     k3 = k1 - 2;
-    res = epstab[k1 + 2];
-    e0 = epstab[k3];
-    e1 = epstab[k2];
+    res = s.ep(k1 + 2);
+    e0 = s.ep(k3);
+    e1 = s.ep(k2);
     e2 = res;
     e1abs = fabs(e1);
     delta2 = e2 - e1;
@@ -632,8 +667,8 @@ __device__ __forceinline__ void qelg(int* n, double* epstab, double* result, dou
       *abserr = err2 + err3;
       goto L100;
     }
-    e3 = epstab[k1];
-    epstab[k1] = e1;
+    e3 = s.ep(k1);
+    s.set_ep(k1, e1);
     delta1 = e1 - e3;
     err1 = fabs(delta1);
     tol1 = fmax(e1abs, fabs(e3)) * epmach;
@@ -646,7 +681,7 @@ __device__ __forceinline__ void qelg(int* n, double* epstab, double* result, dou
     goto L50;
   L30:
     res = e1 + 1.0 / ss;
-    epstab[k1] = res;
+    s.set_ep(k1, res);
     k1 = k1 - 2;
     error = err2 + fabs(res - e2) + err3;
     if (error > *abserr) continue;
@@ -659,24 +694,24 @@ L50:
   ie = newelm + 1;
   for (i = 1; i <= ie; ++i) {
     ib2 = ib + 2;
-    epstab[ib] = epstab[ib2];
+    s.set_ep(ib, s.ep(ib2));
     ib = ib2;
   }
   if (num != *n) {
     indx = num - *n + 1;
     for (i = 1; i <= *n; ++i) {
-      epstab[i] = epstab[indx];
+      s.set_ep(i, s.ep(indx));
       indx++;
     }
   }
   if (*nres < 4) {
-    res3la[*nres] = *result;
+    s.set_r3(*nres, *result);
     *abserr = oflow;
   } else {
-    *abserr = fabs(*result - res3la[3]) + fabs(*result - res3la[2]) + fabs(*result - res3la[1]);
-    res3la[1] = res3la[2];
-    res3la[2] = res3la[3];
-    res3la[3] = *result;
+    *abserr = fabs(*result - s.r3(3)) + fabs(*result - s.r3(2)) + fabs(*result - s.r3(1));
+    s.set_r3(1, s.r3(2));
+    s.set_r3(2, s.r3(3));
+    s.set_r3(3, *result);
   }
 L100:
   *abserr = fmax(*abserr, 5.0 * epmach * fabs(*result));

@@ -5,6 +5,7 @@
 #include "upc_internal.h"
 #include "upc_qags.h"
 
+#include <algorithm>
 #include <climits>
 
 namespace upc {
@@ -123,6 +124,9 @@ __device__ __forceinline__ double flux_point(double b, double k, double g1, doub
 // j <= 120 ln 40 / ln 100 = 96.09.
 constexpr int kMaxQagsNodesPerRow = 98;
 
+// Log step of a row's b grid.
+__device__ __forceinline__ double row_log_step(double bmax, double bmin) { return (log(bmax) - log(bmin)) / kNB1; }
+
 // Geometry of flux row r of a grid of npts points (src/UpcCrossSection.cpp:
 // 224-233): photon energy, log step of the b grid, and the number of its
 // nodes with b <= 2R (form-factor QAGS nodes; 0 for the point flux).
@@ -141,7 +145,7 @@ __device__ __forceinline__ void row_setup(const double* __restrict__ pts, int np
   const double k = side ? M / 2. * exp(-Y) : M / 2. * exp(Y);
   const double g = side ? fp.g2 : fp.g1;
   const double bmax = fmax(5. * g * kHc / k, 5. * fp.R);
-  const double logd = (log(bmax) - log(fp.bmin)) / kNB1;
+  const double logd = row_log_step(bmax, fp.bmin);
   int cnt = 0;
   if (!fp.isPoint) {
     // b_j increases with j: binary search for the number of nodes with b <= 2R
@@ -159,16 +163,13 @@ __device__ __forceinline__ void row_setup(const double* __restrict__ pts, int np
   *cnt_out = cnt < kMaxQagsNodesPerRow ? cnt : kMaxQagsNodesPerRow;  // more only where k is NaN
 }
 
-// Bucket of a row in the photon energy order of the QAGS kernel: `per_octave`
-// buckets per factor of two of k over 40 octaves about 1 GeV, the end buckets
-// taking what lies outside (NaN in the first).
-constexpr int kRowOctaves = 40;
-
-__device__ __forceinline__ int row_bucket(double k, int per_octave)
+// Bucket of a row in the photon energy order of the QAGS kernels:
+// kRowsPerOctave buckets per factor of two of k over 40 octaves about 1 GeV,
+// the end buckets taking what lies outside (NaN in the first).
+__device__ __forceinline__ int row_bucket(double k)
 {
-  const float v = (__log2f((float)k) + 0.5f * kRowOctaves) * per_octave;
-  const int n = kRowOctaves * per_octave;
-  return v > 0.f ? (v < (float)(n - 1) ? (int)v : n - 1) : 0;
+  const float v = (__log2f((float)k) + 0.5f * kRowOctaves) * kRowsPerOctave;
+  return v > 0.f ? (v < (float)(kRowBuckets - 1) ? (int)v : kRowBuckets - 1) : 0;
 }
 
 // fluxFormIntegrand (src/UpcCrossSection.cpp:181-191):
@@ -209,13 +210,16 @@ __device__ __forceinline__ void flux_prelude(const double4* __restrict__ ff, dou
   n->c = ff[n->i];
 }
 
-__device__ __forceinline__ double flux_finish(const FluxNode& n, double j1)
+// The integrand without J1.
+__device__ __forceinline__ double flux_h(const FluxNode& n)
 {
   const double d = n.tc - knot(kQ2min, kDQ2, n.i);
   const double f = n.c.x + d * (n.c.y + d * (n.c.z + d * n.c.w));
-  const double v = n.q * n.q * f * rcp_nr(n.t) * j1;  // t >= (k / g1)^2 > 0
-  return n.tc > kQ2Last ? __builtin_nan("") : v;
+  const double h = n.q * n.q * f * rcp_nr(n.t);  // t >= (k / g1)^2 > 0
+  return n.tc > kQ2Last ? __builtin_nan("") : h;
 }
+
+__device__ __forceinline__ double flux_finish(const FluxNode& n, double j1) { return flux_h(n) * j1; }
 
 template <int BR>
 __device__ __forceinline__ double bessel_j1_branch(double x)
@@ -309,20 +313,51 @@ struct PointTask {
 // What the integrals of one configuration share.
 struct RowJob {
   const double4* ff;
+  const double* j1;  // k_flux_j1's table
   double bmin, g1, factor;
   int A;
 };
 
-// Flux rows of one context for k_flux_qags_rows; as a task source, task
-// t = row * 120 + node (its flux slot).
+// A restricted grid takes part in its full grid's groups (all rows' factors,
+// some lanes' integrals: the full grid's bits, at most its time) where at least
+// one row in three is needed, else its rows in groups of their own: 0.45 of the
+// time per row against 1.
+constexpr int kNeedShare = 3;
+
+// Flux rows of one context for the row kernels; as a task source, task t =
+// row * 120 + node (its flux slot).
 struct GridRows {
-  static constexpr bool kManyJobs = false;
   const double* __restrict__ row_k;
   const double* __restrict__ row_logd;
   const int* __restrict__ row_cnt;
-  const int* __restrict__ perm;  // rows with form-factor nodes, ordered by k
+  int* __restrict__ perm;  // rows with form-factor nodes, ordered by k
+  const unsigned long long* __restrict__ nsorted;  // rows in perm
   RowJob job;
   long long nrows;
+  const unsigned char* __restrict__ need_row;  // null, or rows with 0 are left out
+  // Restricted grids: the counts of two candidate launches, of which this one
+  // runs when kNeedShare * *npart >= *nall (pick 1) or when not (pick 2).
+  int pick;
+  const unsigned long long *npart, *nall;
+  // groups of 64 positions of perm; group(g): its first position, rows and job
+  __device__ long long groups() const
+  {
+    if (pick != 0 && (kNeedShare * *npart >= *nall) != (pick == 1)) return 0;
+    return ((long long)*nsorted + 63) / 64;
+  }
+  __device__ bool need(int r) const { return !need_row || need_row[r]; }
+  __device__ int group(long long g, long long* first, int*) const
+  {
+    *first = g * 64;
+    const long long left = (long long)*nsorted - *first;
+    return left < 64 ? (int)left : 64;
+  }
+  // k_row_order: a job's rows [*r0, *r0 + return) and where they start in perm
+  __device__ long long span(int, long long* r0, long long* pos0) const
+  {
+    *r0 = *pos0 = 0;
+    return nrows;
+  }
   // team work ids: (row, node), kMaxQagsNodesPerRow slots per row
   __device__ long long ids() const { return nrows * kMaxQagsNodesPerRow; }
   __device__ long long overflow_id(long long id) const
@@ -647,15 +682,18 @@ void k_flux_qags(TS ts, const unsigned long long* __restrict__ ntasks_p, unsigne
 // (10.2 ms, slower on small grids); 4 waves per SIMD spill 66 (10.1 ms, same).
 //
 // Work ids are (group of 64 rows, j), taken from a global cursor; ids whose
-// group has no node j end at once.  nrows_p: rows in rs.perm.  stats as in
-// k_flux_qags; overflow receives flux slots (row * 120 + node).
+// group has no node j end at once.  stats as in k_flux_qags; overflow receives flux slots (row * 120
+// + node).  The kernel is in upc_flux_rows.hip; it runs where rows are too far
+// apart in k for the next one.
 // ---------------------------------------------------------------------------
 constexpr int kQagsRowsWaves = 3;        // waves per SIMD (register and LDS budget)
 constexpr int kQagsRowsBlocksPerCu = 3;  // resident workgroups of kQagsBlock per CU
 
-// One QK21 pass on [qa, qb] for every active lane: qk21_stored's sums in its
-// order, the integrand evaluated on the way.  fv: the lane's column of the
-// wavefront's table (stride 64).
+// One QK21 pass on [qa, qb] (the lane's own) for every active lane:
+// qk21_stored's sums in its order, the integrand evaluated on the way.  fv:
+// where the off-centre values wait for the mean deviation, STRIDE apart (the
+// nodes are visited in a rolled loop).
+template <int STRIDE>
 __device__ __forceinline__ QK21Out qk21_rows(double* fv, double qa, double qb, const double4* __restrict__ ff,
                                              double b, double w2g2)
 {
@@ -670,7 +708,7 @@ __device__ __forceinline__ QK21Out qk21_rows(double* fv, double qa, double qb, c
       rabs = fabs(resk);
       continue;
     }
-    fv[(e - 1) * 64] = f;
+    fv[(e - 1) * STRIDE] = f;
     if (e & 1) {
       f1 = f;
       continue;
@@ -682,71 +720,449 @@ __device__ __forceinline__ QK21Out qk21_rows(double* fv, double qa, double qb, c
     resk = resk + kWgk[j] * fsum;
     rabs = rabs + kWgk[j] * (fabs(f1) + fabs(f));
   }
-  return qk21_tail([&](int j, int side) { return fv[(qk21_node(j, side) - 1) * 64]; }, resg, resk, rabs, fc, hlgth);
+  return qk21_tail([&](int j, int side) { return fv[(qk21_node(j, side) - 1) * STRIDE]; }, resg, resk, rabs, fc, hlgth);
+}
+
+// ---------------------------------------------------------------------------
+// The same for rows that lie close together in k: the integrand's two factors,
+// h(q) of the row and J1(b q / hc), each shared by many integrals.
+//
+// - h at the nodes of the 25 intervals that nearly all passes are on is
+//   tabulated per row (k_flux_h) for the row's 30 to 97 integrals.
+// - J1: rows with k above gamma hc / R share one b grid (b_max = 5 R there) and
+//   read J1 from one table per configuration (k_flux_j1), half of the passes
+//   on the Pb-Pb and Au-Au grids; elsewhere the wavefront expands J1 once per
+//   node about the middle of its lanes' b (expand_j1) and every lane evaluates
+//   the polynomial.
+// - The lists of the bookkeeping are in LDS (QagsLdsStore), the pass's 21
+//   values in registers: 2 waves per SIMD.
+//
+// Lanes on other intervals than the first take their turn after it; intervals
+// outside the table and lanes too far apart for the expansion evaluate their
+// own nodes (qk21_rows).
+//
+// 1001 x 121 Pb-Pb: 10.4 -> 4.7 ms against k_flux_qags_rows, 124 -> 37 VALU
+// instructions per integrand value; 8 mixed jobs 55 -> 35 ms (whole batch).
+// Bound: instruction issue and the latency of dependent FP64 and LDS operations
+// at 2 waves per SIMD.  Parts (wave cycles): values and sums 40 %, bookkeeping
+// 28 %, expansions 16 %, loads of h 6 %, row set-up 6 %, own nodes 4 %.  Tried:
+// lists in private memory with 3 waves per SIMD 6.4 ms (values through LDS),
+// 9.8 ms (182 VGPRs spilled); coefficients broadcast from LDS to every lane
+// 4.9 ms (LDS 38 % busy).
+//
+// Work ids are (group of 64 rows, j).  A launch takes up to kRowsChunk groups
+// from g0 on (H bounds it: 269 KB per group).  The j of a group share its h, so
+// a group belongs to one XCD's cursor (workgroups are dealt to the XCDs in
+// turn): the few groups in flight on an XCD stay in its L2.
+// ---------------------------------------------------------------------------
+constexpr int kQagsTableWaves = 2;        // waves per SIMD (register and LDS budget)
+constexpr int kQagsTableBlocksPerCu = 2;  // resident workgroups of kQagsBlock per CU
+constexpr int kXcds = 8;
+constexpr int kRowsChunk = 4096;  // groups of 64 rows per launch (1.1 GB of h)
+constexpr int kRowsTurns = 4;     // intervals a step takes one by one before its other lanes evaluate their own
+
+// h of the intervals that most passes are on: level L of the bisection of
+// [0, 10] holds intervals m < kHCount[L], first slot kHFirst[L].  Below q ~ 1.4
+// the form factor falls off, so dqagse bisects towards q = 0: these 25
+// intervals take 99 % of the passes (Pb 5.02 TeV, O 7 TeV, Au 200 GeV grids).
+constexpr int kHLevels = 10, kHSlots = 25;
+__device__ constexpr int kHCount[kHLevels] = {1, 2, 2, 2, 2, 4, 6, 2, 2, 2};
+__device__ constexpr int kHFirst[kHLevels] = {0, 1, 3, 5, 7, 9, 13, 19, 21, 23};
+
+// Slot of interval m of level L, -1: none.
+__device__ __forceinline__ int h_slot(unsigned L, unsigned m)
+{
+  if (L >= (unsigned)kHLevels) return -1;
+  return m < (unsigned)kHCount[L] ? kHFirst[L] + (int)m : -1;
+}
+
+// h(q) = q^2 F(t) / t of the rows at the nodes of those intervals, which the
+// 30 to 97 integrals of a row all read: H[group][slot][node][lane], for the
+// groups of 64 rows from g0 on.  One block per group and slot.
+// Bound by its stores (10.75 KB per group and slot).
+template <class RS>
+__global__ __launch_bounds__(256) void k_flux_h(RS rs, long long g0,
+                                                double* __restrict__ H)
+{
+  const int slot = blockIdx.x % kHSlots, gl = blockIdx.x / kHSlots;
+  if (g0 + gl >= rs.groups()) return;
+  long long first;
+  int job = 0;
+  const int n = rs.group(g0 + gl, &first, &job);
+  if (n <= 0) return;
+  int L = 0;
+  while (L + 1 < kHLevels && kHFirst[L + 1] <= slot) ++L;
+  const double w = ldexp(kQagsB, -L), qa = (slot - kHFirst[L]) * w, qb = (slot - kHFirst[L] + 1) * w;
+  const int lane = threadIdx.x & 63;
+  const int r = rs.perm[first + (lane < n ? lane : n - 1)];
+  const RowJob P = rs.params(job);
+  const double k = rs.row_k[r];
+  const double w2g2 = k * k / P.g1 / P.g1;
+  double* out = H + ((long long)gl * kHSlots + slot) * (21 * 64) + lane;
+  for (int e = threadIdx.x >> 6; e < 21; e += 4) {
+    FluxNode node;
+    flux_prelude(P.ff, w2g2, qk21_abscissa(e, 0.5 * (qa + qb), 0.5 * (qb - qa)), &node);
+    out[e * 64] = flux_h(node);
+  }
+}
+
+// J1 at the nodes of those intervals on the b grid that all rows with b_max =
+// 5 R share (k above gamma hc / R): T[0] the grid's log step, then [j][slot][
+// node].  One block per j.
+constexpr int kJ1TableElems = 1 + kMaxQagsNodesPerRow * kHSlots * 21;
+
+// Scalar-cache reads of a table that no kernel of the launch writes.
+using ConstD = const __attribute__((address_space(4))) double;
+
+// J1 of a whole wavefront at one node.  Where the lanes are on one interval,
+// node e has one q and the lanes' arguments b q / hc lie within a fraction of
+// a percent of x0 = b0 q / hc, b0 the middle of their b.  One lane per node
+// expands J1 about its x0 (from J1, J0 and Bessel's equation, below), and
+// every lane evaluates the polynomial at its own db = (b - b0) / hc: T - 1
+// FMAs on coefficients (powers of q folded in) that all lanes read from the
+// same LDS address, where J1 itself takes 35 (x <= 8) or 75 FP64
+// instructions.  On rows whose b grids coincide (k above gamma hc / R: b_max
+// = 5 R) db is 0 and T = 1.
+//
+// With delta = q db, T terms leave |delta|^T / T!; kExpandMax[i] is the delta
+// up to which this is below 1.5e-19, i.e. below 1e-17 of J1 ~ x / 2 at the
+// smallest x of an interval's end (0.015).  The recurrence's rounding enters
+// as (delta / x0)^n and stays below the rounding of J1(x0): measured within
+// 4.9e-16 of the envelope (J1's own 4.2e-16) for delta / x0 up to 0.2.
+constexpr int kExpandKinds = 7;
+__device__ constexpr int kExpandTerms[kExpandKinds] = {1, 4, 6, 8, 10, 14, 20};
+__device__ constexpr double kExpandMax[kExpandKinds] = {0.0, 4.3e-5, 2.1e-3, 1.6e-2, 5.9e-2, 0.265, 0.939};
+constexpr int kExpandBoth = 10;    // up to this many terms both halves of a bisection are expanded at once
+constexpr int kExpandSlots = 436;  // coefficients: 42 nodes x 10 terms or 21 x 20
+
+// The recurrence's numbers, n = 0 .. 17: 1 / ((n+1)(n+2)), (n^2-1) / ((n+1)(n+2)), (2n+1) / (n+2).
+struct ExpandTable {
+  double v[18];
+};
+template <class F>
+constexpr ExpandTable expand_table(F f)
+{
+  ExpandTable t{};
+  for (int n = 0; n < 18; ++n) t.v[n] = f((double)n);
+  return t;
+}
+__constant__ static const ExpandTable kExpandAt = expand_table([](double n) { return 1.0 / ((n + 1) * (n + 2)); });
+__constant__ static const ExpandTable kExpandBt = expand_table([](double n) { return (n - 1) / (n + 2); });
+__constant__ static const ExpandTable kExpandCt = expand_table([](double n) { return (2 * n + 1) / (n + 2); });
+
+// A value that all lanes hold, in scalar registers.
+__device__ __forceinline__ double wave_uniform(double v)
+{
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
+// Index into kExpandTerms for delta (the same in all lanes); kExpandKinds: too
+// wide.  mymax: kExpandMax[lane] (beyond the table: infinite).
+__device__ __forceinline__ int expand_kind(double delta, double mymax)
+{
+  return __popcll(__ballot(delta > mymax));
+}
+
+// Coefficients a_n q^n, n < T, of J1 about x0 = b0 q / hc into cf.  With r = 1 /
+// x0, x^2 y'' + x y' + (x^2 - 1) y = 0 gives
+//   (n+1)(n+2) a_{n+2} = -[(n+1)(2n+1) r a_{n+1} + ((n^2-1) r^2 + 1) a_n
+//                          + 2 r a_{n-1} + r^2 a_{n-2}].
+__device__ __forceinline__ void expand_j1(double* cf, double b0, double q, int T)
+{
+  const double x0 = flux_j1_arg(b0, q);
+  if (T == 1) {
+    cf[0] = bessel_j1(x0);
+    return;
+  }
+  double j0, j1;
+  bessel_j01(x0, &j0, &j1);
+  cf[0] = j1;
+  const double r = rcp_nr(x0), r2 = r * r;
+  double am2 = 0.0, am1 = 0.0, a = j1, ap = fma(-j1, r, j0), qn = q;  // a_{n-2}, a_{n-1}, a_n, a_{n+1}, q^{n+1}
+  cf[1] = ap * q;
+#pragma unroll 2
+  for (int n = 0; n < T - 2; ++n) {
+    // everything but the a_{n+1} term first: one dependent FMA per coefficient
+    const double s = fma(fma(kExpandBt.v[n], r2, kExpandAt.v[n]), a, kExpandAt.v[n] * fma(2.0 * r, am1, r2 * am2));
+    const double an = -fma(kExpandCt.v[n] * r, ap, s);
+    qn *= q;
+    cf[n + 2] = an * qn;
+    am2 = am1;
+    am1 = a;
+    a = ap;
+    ap = an;
+  }
+}
+
+// f = h J1 at the 21 nodes of a pass: tabulated h in f, J1 expanded (cf: T
+// coefficients per node).  All lanes take part.
+using LdsCoef = const __attribute__((address_space(3))) double;
+
+// j += c[N] p0 + c[N + 1] p1, ...: c[n] lane n of each row of 16 lanes.
+//
+// Every lane needs every coefficient.  Read from LDS by all lanes, one costs
+// 512 B of the CU's LDS bandwidth (4 cycles; 24 terms of 3 nodes at a time
+// kept it 38 % busy and waited 5000 cycles per pass); here 16 coefficients
+// fill one register over a row of 16 lanes and the row broadcast of the FMA's
+// DPP form hands them out.  s_nop: a DPP source must not have been written by
+// the VALU in the last two wait states.
+template <int N>
+__device__ __forceinline__ void bcast_fma2(double& j, double c, const double* p)
+{
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %1, %3 row_newbcast:%5 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%4 row_mask:0xf bank_mask:0xf"
+      : "+v"(j)
+      : "v"(c), "v"(p[0]), "v"(p[1]), "i"(N), "i"(N + 1));
+}
+template <int N>
+__device__ __forceinline__ void bcast_fma4(double& j, double c, const double* p)
+{
+  asm("s_nop 1\n\t"
+      "v_fmac_f64_dpp %0, %1, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %4 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %3 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+      "v_fmac_f64_dpp %0, %1, %2 row_newbcast:%6 row_mask:0xf bank_mask:0xf"
+      : "+v"(j)
+      : "v"(c), "v"(p[0]), "v"(p[1]), "v"(p[2]), "v"(p[3]), "i"(N), "i"(N + 1), "i"(N + 2), "i"(N + 3));
+}
+
+// Terms K - 1 .. 0 of node E, the highest first (the smallest terms are summed
+// first, as in Horner's order).
+template <int T, int E, int K>
+__device__ __forceinline__ void bcast_terms(double& j, const double* cr, const double* pw)
+{
+  if constexpr (K > 0) {
+    constexpr int i = E * T + K;  // one past the term
+    constexpr int n = K >= 4 && (i - 4) / 16 == (i - 1) / 16 ? 4 : 2;
+    if constexpr (n == 4) bcast_fma4<(i - 4) % 16>(j, cr[(i - 4) / 16], pw + K - 4);
+    else bcast_fma2<(i - 2) % 16>(j, cr[(i - 2) / 16], pw + K - 2);
+    bcast_terms<T, E, K - n>(j, cr, pw);
+  }
+}
+
+template <int T, int E>
+__device__ __forceinline__ void bcast_nodes(double* f, const double* cr, const double* pw)
+{
+  if constexpr (E < 21) {
+    double j1 = 0.0;
+    bcast_terms<T, E, T>(j1, cr, pw);
+    f[E] *= j1;
+    asm volatile("" : "+v"(f[E]));  // rounded here: no contraction with the sums below
+    bcast_nodes<T, E + 1>(f, cr, pw);
+  }
+}
+
+template <int T>
+__device__ __forceinline__ void expanded_values(double* f, LdsCoef* cf, int lane, double db)
+{
+  static_assert(T % 2 == 0, "terms are taken in pairs");
+  if constexpr (T <= 10) {
+    double cr[(21 * T + 15) / 16], pw[T];
+    asm volatile("" : "+v"(db));  // its powers are made here, not kept in registers over the whole integral
+#pragma unroll
+    for (int i = 0; i < (21 * T + 15) / 16; ++i) cr[i] = cf[16 * i + (lane & 15)];
+    pw[0] = 1.0;
+#pragma unroll
+    for (int k = 1; k < T; ++k) pw[k] = pw[k - 1] * db;
+    bcast_nodes<T, 0>(f, cr, pw);
+  } else {
+    // too many powers for the registers: Horner's rule, coefficients from LDS
+#pragma unroll
+    for (int e = 0; e < 21; e += 3) {  // three chains side by side
+      LdsCoef* c = cf + e * T;
+      double j[3] = {c[T - 1], c[2 * T - 1], c[3 * T - 1]};
+#pragma unroll 4
+      for (int k = T - 2; k >= 0; --k) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) j[i] = fma(j[i], db, c[i * T + k]);
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        f[e + i] *= j[i];
+        asm volatile("" : "+v"(f[e + i]));
+      }
+      __builtin_amdgcn_sched_barrier(0);  // bounds the coefficients in flight
+    }
+  }
+}
+
+__device__ __forceinline__ void expanded_values_t(int kind, double* f, const double* cf_, int lane, double db)
+{
+  LdsCoef* cf = (LdsCoef*)cf_;
+  asm volatile("" : "+v"(cf));  // one address register, the coefficients at immediate offsets
+  switch (kind) {
+    case 0:  // db = 0: J1 itself
+#pragma unroll
+      for (int e = 0; e < 21; ++e) {
+        f[e] *= cf[e];
+        asm volatile("" : "+v"(f[e]));
+      }
+      break;
+    case 1: expanded_values<4>(f, cf, lane, db); break;
+    case 2: expanded_values<6>(f, cf, lane, db); break;
+    case 3: expanded_values<8>(f, cf, lane, db); break;
+    case 4: expanded_values<10>(f, cf, lane, db); break;
+    case 5: expanded_values<14>(f, cf, lane, db); break;
+    default: expanded_values<20>(f, cf, lane, db);
+  }
+}
+
+// f = h J1 with J1 from the shared grid's table.
+__device__ __forceinline__ void table_values(double* f, ConstD* j1)
+{
+#pragma unroll
+  for (int e = 0; e < 21; ++e) {
+    f[e] *= j1[e];
+    asm volatile("" : "+v"(f[e]));  // rounded here: no contraction with the sums below
+  }
+}
+
+// QK21 of the 21 values in registers, in its summation order.
+__device__ __forceinline__ QK21Out qk21_values(const double* f, double hlgth)
+{
+  double resg = 0.0, resk = kWgk[10] * f[0];
+  double rabs = fabs(resk);
+#pragma unroll
+  for (int p = 0; p < 10; ++p) {
+    const int j = p < 5 ? 2 * p + 1 : 2 * (p - 5);  // the Gauss pairs, then the Kronrod-only pairs
+    const double f1 = f[2 * p + 1], f2 = f[2 * p + 2];
+    const double fsum = f1 + f2;
+    if (p < 5) resg = resg + kWg[p] * fsum;
+    resk = resk + kWgk[j] * fsum;
+    rabs = rabs + kWgk[j] * (fabs(f1) + fabs(f2));
+  }
+  return qk21_tail([&](int j, int side) { return f[qk21_node(j, side)]; }, resg, resk, rabs, f[0], hlgth);
 }
 
 template <int CAP, class RS>
-__global__ __launch_bounds__(kQagsBlock) __attribute__((amdgpu_waves_per_eu(kQagsRowsWaves, kQagsRowsWaves)))
-void k_flux_qags_rows(RS rs, const unsigned long long* __restrict__ nrows_p, unsigned long long* __restrict__ cursor,
+__global__ __launch_bounds__(kQagsBlock) __attribute__((amdgpu_waves_per_eu(kQagsTableWaves, kQagsTableWaves)))
+void k_flux_qags_table(RS rs, long long g0,
+                      const double* __restrict__ H, unsigned long long* __restrict__ cursors,
                       double* __restrict__ flux, unsigned long long* __restrict__ stats,
                       long long* __restrict__ overflow, int fast_cap)
 {
-  __shared__ double lds[kQagsBlock / 64][20 * 64];
+  using Store = QagsLdsStore<CAP>;
+  struct WaveLds {
+    typename Store::Columns lists;
+    double cf[kExpandSlots];  // J1 expansions, [node][term]
+  };
+  __shared__ WaveLds lds[kQagsBlock / 64];
   const int lane = threadIdx.x & 63;
-  double* fv = lds[threadIdx.x >> 6] + lane;
-  typename QagsSmallStore<CAP>::Arrays lists;
-  Qags<QagsSmallStore<CAP>> q;
-  q.s.a = &lists;
+  double* cf = lds[threadIdx.x >> 6].cf;
+  typename Store::Arrays lists;
+  Qags<Store> q;
+  q.s.bind(&lds[threadIdx.x >> 6].lists, lane, &lists);
   q.s.lim = fast_cap < CAP ? fast_cap : CAP;
-  const long long nrows = (long long)*nrows_p;
-  const unsigned long long nids = (unsigned long long)((nrows + 63) / 64) * kMaxQagsNodesPerRow;
+  // groups of this launch, and those of cursor x: g0 + x, g0 + x + kXcds, ...
+  const long long left = rs.groups() - g0, ngroups = left < kRowsChunk ? left : kRowsChunk;
   unsigned my_evals = 0, my_bad = 0;  // 32-bit per lane; evaluations flushed before they could wrap
-  while (true) {
-    unsigned long long id = 0;
-    if (lane == 0) id = atomicAdd(cursor, 1ull);
-    id = __shfl(id, 0);
-    if (id >= nids) break;
-    const long long g = (long long)(id / kMaxQagsNodesPerRow);
-    const int j = (int)(id - (unsigned long long)g * kMaxQagsNodesPerRow);
-    const long long pos = g * 64 + lane;
-    int r = 0, job = 0;
-    bool act = false;
-    if (pos < nrows) {
-      r = rs.perm[pos];
-      act = j < rs.row_cnt[r];
-      if (RS::kManyJobs && act) job = rs.job_of(r);
+  const double mymax = lane < kExpandKinds ? kExpandMax[lane < kExpandKinds ? lane : 0] : __builtin_inf();
+  int x = blockIdx.x % kXcds, tried = 0;
+  unsigned next = 0;  // lane 0: the id after the current one, asked for while that one runs
+  if (lane == 0) next = (unsigned)atomicAdd(&cursors[x], 1ull);
+  while (ngroups > 0) {
+    const unsigned id = __builtin_amdgcn_readfirstlane(next);
+    const int gi = (int)(id / kMaxQagsNodesPerRow), j = (int)(id - gi * kMaxQagsNodesPerRow);
+    const int gl = gi * kXcds + x;
+    if (gl >= ngroups) {  // this cursor's groups are done: help with the next
+      if (++tried == kXcds) break;
+      x = (x + 1) % kXcds;
+      if (lane == 0) next = (unsigned)atomicAdd(&cursors[x], 1ull);
+      continue;
     }
-    unsigned long long todo = __ballot(act);
-    while (todo) {
-      // one configuration at a time (a group straddles two only where their rows meet)
-      int jb = 0;
-      bool live = act;
-      if (RS::kManyJobs) {
-        jb = __builtin_amdgcn_readlane(job, __ffsll((long long)todo) - 1);
-        live = act && job == jb;
-        todo &= ~__ballot(live);
-      } else {
-        todo = 0;
-      }
-      const RowJob P = rs.params(jb);
-      double b = 0.0, w2g2 = 0.0;
+    if (lane == 0) next = (unsigned)atomicAdd(&cursors[x], 1ull);
+    const double* hg = H + (long long)gl * (kHSlots * 21 * 64);
+    long long first;
+    int r = 0, job = 0;
+    bool live = false;
+    if (lane < rs.group(g0 + gl, &first, &job)) {
+      r = rs.perm[first + lane];
+      live = j < rs.row_cnt[r];
+    }
+    if (__ballot(live) != 0) {
+      const RowJob P = rs.params(job);
+      double b = 0.0;
       if (live) {
         b = row_node_b(P.bmin, rs.row_logd[r], j);
-        const double k = rs.row_k[r];
-        w2g2 = k * k / P.g1 / P.g1;
         q.start();
       }
-      while (__ballot(live) != 0) {
-        if (!live) continue;
+      // the middle of the lanes' b, and their distance from it in J1's argument per q
+      double blo = live ? b : DBL_MAX, bhi = live ? b : 0.0;
+      for (int o = 32; o > 0; o >>= 1) {
+        blo = fmin(blo, __shfl_xor(blo, o));
+        bhi = fmax(bhi, __shfl_xor(bhi, o));
+      }
+      const double b0 = wave_uniform(0.5 * (blo + bhi));
+      const double db = (b - b0) * (1.0 / kHc), dbm = wave_uniform(fmax(b0 - blo, bhi - b0) * (1.0 / kHc));
+      live = live && rs.need(r);
+      // every row on the shared b grid: J1 from its table
+      const bool shared = __ballot(live && rs.row_logd[r] != P.j1[0]) == 0;
+      ConstD* j1t = (ConstD*)(P.j1 + 1) + j * (kHSlots * 21);
+      int np = 1;  // passes of the step: the whole range first, then the halves of every lane's interval
+      unsigned long long rem;
+      while ((rem = __ballot(live)) != 0) {
         QK21Out o{}, o2{};
+        q.phase = np == 1 ? 0 : 2;
+        // the lanes of one interval at a time (nearly always all of them)
+        for (int turn = 0; rem != 0; ++turn) {
+          const unsigned iv = __builtin_amdgcn_readlane(q.cur, __ffsll((long long)rem) - 1);
+          const unsigned L = iv >> 26, im = iv & 0x3ffffffu;
+          // [lo, hi] = 10 2^-L [m, m + 1], built exactly (10 2^-L from its bits)
+          const double w = __hiloint2double(0x40240000 - ((int)L << 20), 0);
+          const double lo = wave_uniform((double)im * w), mid = wave_uniform(lo + 0.5 * w), hi = wave_uniform(lo + w);
+          const int slot = np == 1 ? h_slot(L, im) : h_slot(L + 1, 2 * im);
+          const int kind = shared ? 0 : expand_kind(hi * dbm, mymax);
+          const bool mine = (rem >> lane & 1) != 0;
+          if (slot < 0 || kind == kExpandKinds || turn == kRowsTurns) {
+            if (mine) {
 #pragma unroll 1
-        for (int pass = 0; pass < q.passes(); ++pass) {
-          double qa, qb;
-          q.interval(pass, &qa, &qb);
-          o = o2;
-          o2 = qk21_rows(fv, qa, qb, P.ff, b, w2g2);
+              for (int pass = 0; pass < np; ++pass) {
+                double la, lb;
+                q.interval(pass, &la, &lb);
+                // rare: b and (k/g)^2 are found again instead of kept in registers
+                const double k = rs.row_k[r];
+                o = o2;
+                double fv[20];
+                o2 = qk21_rows<1>(fv, la, lb, P.ff, row_node_b(P.bmin, rs.row_logd[r], j), k * k / P.g1 / P.g1);
+              }
+              if (np == 1) o = o2;
+            }
+            break;
+          }
+          const int T = kExpandTerms[kind];
+          const bool both = T <= kExpandBoth;
+          auto expand = [&](int first, int n) {
+            wave_lds_sync();
+            if (lane < n) {
+              const int second = lane >= 21, pass = first + second;
+              const double qa = pass ? mid : lo, qb = np == 2 && !pass ? mid : hi;
+              expand_j1(cf + lane * T, b0, qk21_abscissa(lane - 21 * second, 0.5 * (qa + qb), 0.5 * (qb - qa)), T);
+            }
+            wave_lds_sync();
+          };
+          const double* hp = hg + slot * (21 * 64);
+          const bool here = mine && q.cur == iv;
+#pragma unroll 1
+          for (int pass = 0; pass < np; ++pass) {
+            if (!shared && (pass == 0 || !both)) expand(pass, both ? 21 * np : 21);
+            double f[21];
+#pragma unroll
+            for (int e = 0; e < 21; ++e) f[e] = hp[(21 * pass + e) * 64 + lane];
+            if (shared) table_values(f, j1t + (slot + pass) * 21);
+            else expanded_values_t(kind, f, cf + (both ? 21 * pass * T : 0), lane, db);
+            const QK21Out on = qk21_values(f, np == 2 ? 0.25 * w : 0.5 * w);
+            if (here) {
+              o = o2;
+              o2 = on;
+            }
+          }
+          if (np == 1 && here) o = o2;
+          rem &= ~__ballot(here);
         }
-        if (q.phase == 0) o = o2;
+        np = 2;
+        if (!live) continue;
         const int st = q.consume(o, o2);
         if (st == kQagsRunning) continue;
         live = false;
@@ -761,7 +1177,7 @@ void k_flux_qags_rows(RS rs, const unsigned long long* __restrict__ nrows_p, uns
           }
           if (q.status() != 0) {
             my_bad++;
-            rs.failed(jb);
+            rs.failed(job);
           }
         } else {
           overflow[atomicAdd(&stats[2], 1ull)] = slot;
@@ -1230,67 +1646,126 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(JR::
   else lumi_fp64_body<false, WAVES>(v, p0, sm);
 }
 
-// Three-pass exclusive scan of the row counts: per-block sums, their scan in
-// one block, then the offsets.  *total receives the sum.
-constexpr int kScanBlock = 1024;
-
-template <int BS = kScanBlock>
-__global__ __launch_bounds__(BS) void k_scan_part(const int* __restrict__ cnt, long n,
-                                                          long long* __restrict__ part)
+// Exclusive prefix sums of the row counts per bucket (in place), one block per
+// job: off[job][bucket] counts from where the job's rows start in perm; their
+// number in nsorted[job].  10 buckets per thread, wave scans.
+template <class RS, class N>
+__global__ __launch_bounds__(1024) void k_row_offsets(RS rs, int* __restrict__ off, N* __restrict__ nsorted)
 {
-  __shared__ long long s[BS];
-  const long i = (long)blockIdx.x * BS + threadIdx.x;
-  s[threadIdx.x] = i < n ? cnt[i] : 0;
-  __syncthreads();
-  for (int d = BS / 2; d > 0; d >>= 1) {
-    if (threadIdx.x < d) s[threadIdx.x] += s[threadIdx.x + d];
-    __syncthreads();
+  constexpr int kPer = kRowBuckets / 1024;
+  __shared__ int wsum[16];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  off += (size_t)blockIdx.x * kRowBuckets;
+  long long r0, pos0;
+  rs.span(blockIdx.x, &r0, &pos0);
+  int v[kPer], s = 0;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    v[i] = off[t * kPer + i];
+    s += v[i];
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = s[0];
+  int inc = s;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(inc, o);
+    if (lane >= o) inc += u;
+  }
+  if (lane == 63) wsum[wv] = inc;
+  __syncthreads();
+  int base = (int)pos0 + inc - s;
+  for (int w = 0; w < wv; ++w) base += wsum[w];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    off[t * kPer + i] = base;
+    base += v[i];
+  }
+  if (t == 1023) nsorted[blockIdx.x] = (N)(base - (int)pos0);
 }
 
-template <int BS = kScanBlock>
-__global__ __launch_bounds__(BS) void k_scan_top(long long* __restrict__ part, int nparts,
-                                                         unsigned long long* __restrict__ total)
+// Orders the rows of each bucket by (k, row): the order they were dropped in
+// varies from run to run, and with it the groups that expand J1 together and
+// the last bits of what they compute.  off: the buckets' ends.  One wavefront
+// per bucket (50 rows on the 1001 x 121 grid); a bucket that does not fit its
+// LDS is filled again in row order.
+constexpr int kOrderMax = 1024;
+
+template <class RS>
+__global__ __launch_bounds__(256) void k_row_order(RS rs, const int* __restrict__ off, long long nbuckets)
 {
-  __shared__ long long s[BS];
-  long long carry = 0;
-  for (int base = 0; base < nparts; base += BS) {
-    const int i = base + threadIdx.x;
-    const long long v = i < nparts ? part[i] : 0;
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int d = 1; d < BS; d <<= 1) {
-      const long long t = threadIdx.x >= d ? s[threadIdx.x - d] : 0;
-      __syncthreads();
-      s[threadIdx.x] += t;
-      __syncthreads();
+  __shared__ long long kk[4][kOrderMax];
+  __shared__ int rr[4][kOrderMax];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const long long i = (long long)blockIdx.x * 4 + wv;
+  if (i >= nbuckets) return;
+  const int job = (int)(i / kRowBuckets), bucket = (int)(i - (long long)job * kRowBuckets);
+  long long r0, start;
+  const long long nrows = rs.span(job, &r0, &start);
+  if (bucket > 0) start = off[i - 1];
+  const int n = (int)(off[i] - start);
+  if (n <= 1) return;
+  if (n > kOrderMax) {
+    long long done = 0;
+    for (long long base = r0; base < r0 + nrows && done < n; base += 64) {
+      const long long r = base + lane;
+      const bool here = r < r0 + nrows && rs.row_cnt[r] > 0 && row_bucket(rs.row_k[r]) == bucket;
+      const unsigned long long m = __ballot(here);
+      const long long at = done + __popcll(m & ((1ull << lane) - 1));
+      if (here && at < n) rs.perm[start + at] = (int)r;
+      done += __popcll(m);
     }
-    if (i < nparts) part[i] = carry + s[threadIdx.x] - v;  // exclusive
-    const long long blk_total = s[BS - 1];
-    __syncthreads();
-    carry += blk_total;
+    return;
   }
-  if (threadIdx.x == 0) *total = (unsigned long long)carry;
+  for (int e = lane; e < n; e += 64) {
+    const int r = rs.perm[start + e];
+    rr[wv][e] = r;
+    kk[wv][e] = __double_as_longlong(rs.row_k[r]);
+  }
+  wave_lds_sync();
+  for (int e = lane; e < n; e += 64) {
+    const long long k = kk[wv][e];
+    const int r = rr[wv][e];
+    int rank = 0;
+    for (int m = 0; m < n; ++m) rank += kk[wv][m] < k || (kk[wv][m] == k && rr[wv][m] < r);
+    rs.perm[start + rank] = r;
+  }
 }
 
-template <int BS = kScanBlock>
-__global__ __launch_bounds__(BS) void k_scan_apply(const int* __restrict__ cnt, long n,
-                                                           const long long* __restrict__ part,
-                                                           long long* __restrict__ off)
+// Flux rows of a launch (of a job, in a batch) from which on neighbouring rows
+// lie close enough in k to share what k_flux_qags_table shares.  QAGS of Pb-Pb
+// points and grids, k_flux_qags_rows against k_flux_qags_table: 4,096 rows 0.69
+// against 0.89 ms, 6,000 0.86, 1.04; 8,192 1.03, 1.01; 11,000 1.24, 1.10;
+// 16,384 1.52, 1.30.  What decides it is the row count alone, so a job of a
+// batch takes the route of its own context.
+constexpr long long kQagsShareRows = 8192;
+
+// Launches over at most `groups` groups of rows, share: of k_flux_qags_table,
+// kRowsChunk of them at a time, else of k_flux_qags_rows.  cursors:
+// rows_cursors(groups) cleared counters; H: rows_h_elems(groups) (share only);
+// per_cu: workgroups per CU, at most 3.
+inline long long rows_groups(long long rows) { return (rows + 63) / 64; }
+inline size_t rows_cursors(long long groups) { return (size_t)((groups + kRowsChunk - 1) / kRowsChunk) * kXcds; }
+inline size_t rows_h_elems(long long groups)
 {
-  __shared__ long long s[BS];
-  const long i = (long)blockIdx.x * BS + threadIdx.x;
-  const long long v = i < n ? cnt[i] : 0;
-  s[threadIdx.x] = v;
-  __syncthreads();
-  for (int d = 1; d < BS; d <<= 1) {
-    const long long t = threadIdx.x >= d ? s[threadIdx.x - d] : 0;
-    __syncthreads();
-    s[threadIdx.x] += t;
-    __syncthreads();
+  return (size_t)(groups < kRowsChunk ? groups : kRowsChunk) * (kHSlots * 21 * 64);
+}
+
+// upc_flux_rows.hip
+template <class RS>
+void launch_qags_rows_direct(const RS& rs, unsigned long long* cursor, double* flux, unsigned long long* stats,
+                             long long* overflow, int cap, int blocks, hipStream_t s);
+
+template <class RS>
+inline void launch_qags_rows(bool share, const RS& rs, long long groups, double* H, unsigned long long* cursors,
+                             double* flux, unsigned long long* stats, long long* overflow, int cap, int ncu,
+                             int per_cu, hipStream_t s)
+{
+  if (groups <= 0) return;
+  if (!share) return launch_qags_rows_direct(rs, cursors, flux, stats, overflow, cap, ncu * per_cu, s);
+  for (long long g0 = 0; g0 < groups; g0 += kRowsChunk, cursors += kXcds) {
+    const long long n = groups - g0 < kRowsChunk ? groups - g0 : kRowsChunk;
+    hipLaunchKernelGGL(k_flux_h<RS>, dim3((unsigned)(n * kHSlots)), dim3(256), 0, s, rs, g0, H);
+    hipLaunchKernelGGL((k_flux_qags_table<kQagsCap, RS>), dim3(ncu * std::min(per_cu, kQagsTableBlocksPerCu)),
+                       dim3(kQagsBlock), 0, s, rs, g0, H, cursors, flux, stats, overflow, cap);
   }
-  if (i < n) off[i] = part[blockIdx.x] + s[threadIdx.x] - v;
 }
 
 inline FluxParams flux_params(const upc_ctx* c, int mirror_ny = 0)

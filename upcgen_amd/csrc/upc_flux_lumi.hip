@@ -13,7 +13,7 @@
 // k2 rows.  flux[r*120 + j].  Nodes with b <= 2R (form-factor flux) are left
 // to the QAGS kernel, which takes the rows in order of k (counting sort:
 // histogram in k_rows, offsets in k_row_offsets, ranks in
-// k_flux_point_rows); the rest take the point-charge flux.
+// k_flux_point_rows, the order within a bucket in k_row_order); the rest take the point-charge flux.
 #include "upc_internal.h"
 #include "upc_qags.h"
 #include "upc_flux.h"
@@ -47,10 +47,11 @@ __global__ void k_grid_points(int nm, double mmin, double mmax, int ny, double y
 // Row geometry, the number of form-factor (QAGS) nodes of each row, the
 // histogram of the rows that have some over the k buckets, and the total of
 // those nodes.
-// need (may be null): rows with need[r] == 0 get no QAGS nodes.
+// need (may be null): rows with need[r] == 0 get no QAGS nodes, or with `all`
+// keep their place in the order (their nodes are not in the total).
 __global__ __launch_bounds__(256) void k_rows(const double* __restrict__ pts, int npts, int nrows, FluxParams fp,
                                               double* __restrict__ row_k, double* __restrict__ row_logd,
-                                              int* __restrict__ row_cnt, const unsigned char* __restrict__ need,
+                                              int* __restrict__ row_cnt, const unsigned char* __restrict__ need, int all,
                                               int* __restrict__ hist, unsigned long long* __restrict__ total)
 {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
@@ -58,50 +59,23 @@ __global__ __launch_bounds__(256) void k_rows(const double* __restrict__ pts, in
   if (r < nrows) {
     double k;
     row_setup(pts, npts, r, fp, &k, &row_logd[r], &cnt);
-    if (need && !need[r]) cnt = 0;
+    const bool out = need && !need[r];
+    if (out && !all) cnt = 0;
     row_k[r] = k;
     row_cnt[r] = cnt;
-    if (cnt > 0) atomicAdd(&hist[row_bucket(k, kRowsPerOctave)], 1);
+    if (cnt > 0) atomicAdd(&hist[row_bucket(k)], 1);
+    if (out) cnt = 0;
   }
   if (fp.isPoint) return;
   for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o);
   if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(total, (unsigned long long)cnt);
 }
 
-// Exclusive prefix sums of the kRowBuckets row counts (in place), their total
-// in *nrows.  One block: 10 buckets per thread, wave scans.
-__global__ __launch_bounds__(1024) void k_row_offsets(int* __restrict__ hist, unsigned long long* __restrict__ nrows)
-{
-  constexpr int kPer = kRowBuckets / 1024;
-  __shared__ int wsum[16];
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  int v[kPer], s = 0;
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    v[i] = hist[t * kPer + i];
-    s += v[i];
-  }
-  int inc = s;
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u = __shfl_up(inc, o);
-    if (lane >= o) inc += u;
-  }
-  if (lane == 63) wsum[wv] = inc;
-  __syncthreads();
-  int base = inc - s;
-  for (int w = 0; w < wv; ++w) base += wsum[w];
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    hist[t * kPer + i] = base;
-    base += v[i];
-  }
-  if (t == 1023) *nrows = (unsigned long long)base;
-}
-
 // Point-charge flux of the nodes with b > 2R (or FLUX_POINT 1), and the rank
 // of each row that has form-factor nodes in the order of k (off: the bucket
 // offsets, advanced here; perm may be null: no order needed).
-// row_need (may be null): rows that no needed bin reads are skipped.
+// row_need (may be null): rows that no needed bin reads are skipped (they keep
+// their rank).
 __global__ void k_flux_point_rows(int nrows, FluxParams fp, const double* __restrict__ row_k,
                                   const double* __restrict__ row_logd, const int* __restrict__ row_cnt,
                                   double* __restrict__ flux, int* __restrict__ off, int* __restrict__ perm,
@@ -110,10 +84,37 @@ __global__ void k_flux_point_rows(int nrows, FluxParams fp, const double* __rest
   const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (gid >= (long)nrows * kNB1) return;
   const long r = gid / kNB1;
-  if (row_need && !row_need[r]) return;
   const int j = (int)(gid % kNB1);
-  if (perm && j == 0 && row_cnt[r] > 0) perm[atomicAdd(&off[row_bucket(row_k[r], kRowsPerOctave)], 1)] = (int)r;
+  if (perm && j == 0 && row_cnt[r] > 0) perm[atomicAdd(&off[row_bucket(row_k[r])], 1)] = (int)r;
+  if (row_need && !row_need[r]) return;
   point_row_node(r, j, fp, row_k, row_logd, row_cnt, flux);
+}
+
+// The needed rows of perm, 1024 positions of it in their order at a time.
+__global__ __launch_bounds__(1024) void k_need_rows(const int* __restrict__ perm,
+                                                    const unsigned long long* __restrict__ nsorted,
+                                                    const unsigned char* __restrict__ need, int* __restrict__ out,
+                                                    unsigned long long* __restrict__ n)
+{
+  __shared__ int wsum[16], base;
+  const long long pos = (long long)blockIdx.x * 1024 + threadIdx.x;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int r = pos < (long long)*nsorted ? perm[pos] : -1;
+  const bool in = r >= 0 && need[r];
+  const unsigned long long m = __ballot(in);
+  if (lane == 0) wsum[wv] = __popcll(m);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int total = 0;
+    for (int w = 0; w < 16; ++w) {
+      const int c = wsum[w];
+      wsum[w] = total;
+      total += c;
+    }
+    base = total ? (int)atomicAdd(n, (unsigned long long)total) : 0;
+  }
+  __syncthreads();
+  if (in) out[base + wsum[wv] + __popcll(m & ((1ull << lane) - 1))] = r;
 }
 
 // ---------------------------------------------------------------------------
@@ -121,13 +122,12 @@ __global__ void k_flux_point_rows(int nrows, FluxParams fp, const double* __rest
 // ---------------------------------------------------------------------------
 static inline int nblk(long n, int bs) { return (int)((n + bs - 1) / bs); }
 
-static int qags_persistent_blocks(int per_cu)
+static int cu_count()
 {
   int dev = 0, ncu = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-  if (ncu <= 0) ncu = 256;
-  return ncu * per_cu;  // as many workgroups as stay resident
+  return ncu > 0 ? ncu : 256;
 }
 
 // Lanes per integral for a launch of about n form-factor integrals (1: one
@@ -183,8 +183,13 @@ static int ensure_work(upc_ctx* c, size_t npts, size_t rows, size_t points_ff = 
   UPC_HIP(hipMalloc(&w.d_flux, sizeof(double) * rows * kNB1));
   UPC_HIP(hipMalloc(&w.d_idx, sizeof(int) * nidx));
   UPC_HIP(hipMalloc(&w.d_overflow, sizeof(long long) * nover));
-  UPC_HIP(hipMalloc(&w.d_counters, sizeof(unsigned long long) * 8 + sizeof(int) * kRowBuckets));
+  const size_t ncur = rows_cursors(rows_groups(rows)) + kXcds;  // and one launch of a restricted grid's
+  UPC_HIP(hipMalloc(&w.d_counters, sizeof(unsigned long long) * (8 + ncur) + sizeof(int) * kRowBuckets));
   w.d_hist = (int*)(w.d_counters + 8);
+  w.d_cursors = (unsigned long long*)(w.d_hist + kRowBuckets);
+  w.ncursors = ncur;
+  if (!c->cfg.flux_point && rows >= (size_t)kQagsShareRows)
+    UPC_HIP(hipMalloc(&w.d_h, sizeof(double) * rows_h_elems(rows_groups(rows))));
   UPC_HIP(hipMalloc(&w.d_points, sizeof(double) * 4 * npts));
   w.rows_cap = rows;
   w.over_cap = nover;
@@ -194,17 +199,17 @@ static int ensure_work(upc_ctx* c, size_t npts, size_t rows, size_t points_ff = 
 }
 
 // What the points kernels clear before a flux launch: the counters and, where
-// rows are sorted, the histogram behind them.
+// rows are sorted, the histogram and the row kernels' cursors behind them.
 static int flux_clear_ints(const upc_ctx* c)
 {
-  return (int)(sizeof(unsigned long long) * 8 / sizeof(int)) + (c->cfg.flux_point ? 0 : kRowBuckets);
+  return 16 + (c->cfg.flux_point ? 0 : kRowBuckets + 2 * (int)c->work.ncursors);
 }
 
 void free_work(upc_ctx* c)
 {
   LumiWork& w = c->work;
   void* ptrs[] = {w.d_row_k, w.d_row_logd, w.d_row_cnt, w.d_perm, w.d_flux,
-                  w.d_idx, w.d_overflow, w.d_counters, w.d_points};
+                  w.d_idx, w.d_overflow, w.d_counters, w.d_points, w.d_h};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   w = LumiWork{};
@@ -220,40 +225,83 @@ static long long flux_rows(int npts, int mirror_ny)
   return mirror_ny > 0 ? (long long)npts + npts / mirror_ny : 2LL * npts;
 }
 
-// Runs flux rows + QAGS for the points already in c->work.d_points.
-static int run_flux(upc_ctx* c, int npts, int mirror_ny, hipStream_t s, const unsigned char* row_need = nullptr)
+// Runs flux rows + QAGS for the points already in c->work.d_points; row_need:
+// only the rows with row_need[r] != 0, need_perm: room for their numbers.
+static int run_flux(upc_ctx* c, int npts, int mirror_ny, hipStream_t s, const unsigned char* row_need = nullptr,
+                    int* need_perm = nullptr)
 {
   LumiWork& w = c->work;
   const FluxParams fp = flux_params(c, mirror_ny);
   const int nrows = flux_rows(npts, mirror_ny);
   // a restricted grid has few rows of many: only the sort knows how many
   const int team = row_need ? 1 : qags_team((long long)nrows * kQagsNodesPerRow);
-  const bool sorted = !c->cfg.flux_point && team == 1;
+  const bool sorted = !c->cfg.flux_point && team == 1, share = sorted && nrows >= kQagsShareRows;
+  const GridRows rs{w.d_row_k, w.d_row_logd, w.d_row_cnt, w.d_perm, w.d_counters + 6,
+                    RowJob{c->d_ff, c->d_j1, fp.bmin, fp.g1, fp.factor, fp.A}, nrows,
+                    share ? row_need : nullptr, share && row_need ? 1 : 0, w.d_counters + 7, w.d_counters + 6};
   {
   PhaseScope ph(c, s, UPC_PHASE_FLUX);
   hipLaunchKernelGGL(k_rows, dim3(nblk(nrows, 256)), dim3(256), 0, s, w.d_points, npts, nrows, fp, w.d_row_k,
-                     w.d_row_logd, w.d_row_cnt, row_need, w.d_hist, w.d_counters + 4);
+                     w.d_row_logd, w.d_row_cnt, row_need, (int)share, w.d_hist, w.d_counters + 4);
   if (sorted)
-    hipLaunchKernelGGL(k_row_offsets, dim3(1), dim3(1024), 0, s, w.d_hist, w.d_counters + 6);
+    hipLaunchKernelGGL((k_row_offsets<GridRows, unsigned long long>), dim3(1), dim3(1024), 0, s, rs, w.d_hist,
+                       w.d_counters + 6);
   hipLaunchKernelGGL(k_flux_point_rows, dim3(nblk((long)nrows * kNB1, 256)), dim3(256), 0, s, nrows, fp,
                      w.d_row_k, w.d_row_logd, w.d_row_cnt, w.d_flux, w.d_hist, sorted ? w.d_perm : nullptr, row_need);
+  if (share)
+    hipLaunchKernelGGL(k_row_order<GridRows>, dim3(nblk(kRowBuckets, 4)), dim3(256), 0, s, rs, w.d_hist,
+                       (long long)kRowBuckets);
+  if (share && row_need)
+    hipLaunchKernelGGL(k_need_rows, dim3(nblk(nrows, 1024)), dim3(1024), 0, s, w.d_perm, w.d_counters + 6, row_need,
+                       need_perm, w.d_counters + 7);
   UPC_HIP(hipGetLastError());
   }
   if (!c->cfg.flux_point) {
     PhaseScope ph(c, s, UPC_PHASE_QAGS);
-    const GridRows rs{w.d_row_k, w.d_row_logd, w.d_row_cnt, w.d_perm,
-                      RowJob{c->d_ff, fp.bmin, fp.g1, fp.factor, fp.A}, nrows};
     if (team > 1)
       launch_qags_team(team, rs, (long long)nrows * kMaxQagsNodesPerRow, w.d_flux, nullptr, w.d_counters,
                        w.d_overflow, c->qags_cap, s);
     else
-      hipLaunchKernelGGL((k_flux_qags_rows<kQagsCap, GridRows>), dim3(qags_persistent_blocks(kQagsRowsBlocksPerCu)),
-                         dim3(kQagsBlock), 0, s, rs, w.d_counters + 6, w.d_counters + 5, w.d_flux, w.d_counters,
-                         w.d_overflow, c->qags_cap);
+      launch_qags_rows(share, rs, rows_groups(nrows), w.d_h, w.d_cursors, w.d_flux, w.d_counters, w.d_overflow,
+                       c->qags_cap, cu_count(), kQagsRowsBlocksPerCu, s);
+    if (share && row_need) {
+      GridRows few = rs;
+      few.perm = need_perm;
+      few.nsorted = few.npart;
+      few.need_row = nullptr;
+      few.pick = 2;
+      launch_qags_rows(false, few, rows_groups(nrows), nullptr, w.d_cursors + rows_cursors(rows_groups(nrows)), w.d_flux,
+                       w.d_counters, w.d_overflow, c->qags_cap, cu_count(), kQagsRowsBlocksPerCu, s);
+    }
     hipLaunchKernelGGL((k_flux_qags_wave<GridRows>), dim3(kQagsWaveBlocks), dim3(64), 0, s, rs, w.d_overflow,
                        w.d_counters, w.d_flux, (int*)nullptr);
     UPC_HIP(hipGetLastError());
   }
+  return 0;
+}
+
+// J1 on the b grid shared by the context's large-k rows (form-factor flux).
+size_t flux_j1_elems() { return kJ1TableElems; }
+
+__global__ __launch_bounds__(256) void k_flux_j1(double R, double bmin, double* __restrict__ T)
+{
+  const double logd = row_log_step(5. * R, bmin);
+  const int j = blockIdx.x;
+  if (j == 0 && threadIdx.x == 0) T[0] = logd;
+  const double b = row_node_b(bmin, logd, j);
+  for (int i = threadIdx.x; i < kHSlots * 21; i += 256) {
+    const int slot = i / 21, e = i - 21 * slot;
+    int L = 0;
+    while (L + 1 < kHLevels && kHFirst[L + 1] <= slot) ++L;
+    const double w = ldexp(kQagsB, -L), qa = (slot - kHFirst[L]) * w, qb = (slot - kHFirst[L] + 1) * w;
+    T[1 + j * (kHSlots * 21) + i] = bessel_j1(flux_j1_arg(b, qk21_abscissa(e, 0.5 * (qa + qb), 0.5 * (qb - qa))));
+  }
+}
+
+int launch_flux_j1(upc_ctx* c, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_flux_j1, dim3(kMaxQagsNodesPerRow), dim3(256), 0, s, c->cfg.R, flux_params(c).bmin, c->d_j1);
+  UPC_HIP(hipGetLastError());
   return 0;
 }
 
@@ -314,30 +362,15 @@ int lumi_points_fp64(upc_ctx* c, const double* d_pts, int npts, double* d_L, dou
   FluxParams fp;
   int rc = prepare_flux(c, d_pts, npts, &fp, s);
   if (rc) return rc;
-  constexpr int kWaves = 4;
-  const int mirror_out = fp.mirror_ny > 0;
-  SingleLumi jr{LumiView{c->work.d_points, c->work.d_row_logd, c->work.d_flux, fp, c->d_gaa, c->d_bk,
-                         c->d_scalars, npts, c->cfg.breakup_mode, c->cfg.use_polarized, d_L, d_Ls, d_Lp,
-                         mirror_out}};
-  const int nwork = lumi_work_items(npts, fp.mirror_ny, mirror_out);
+  const LumiView v{c->work.d_points, c->work.d_row_logd, c->work.d_flux, fp, c->d_gaa, c->d_bk,
+                   c->d_scalars, npts, c->cfg.breakup_mode, c->cfg.use_polarized, d_L, d_Ls, d_Lp,
+                   fp.mirror_ny > 0};
   {
     PhaseScope ph(c, s, UPC_PHASE_LUMI);
-    hipLaunchKernelGGL((k_lumi_fp64<kWaves, SingleLumi>), dim3(nblk(nwork, kWaves)), dim3(64 * kWaves), 0, s,
-                       jr);
+    rc = launch_lumi_fp64(v, s);
   }
-  UPC_HIP(hipGetLastError());
+  if (rc) return rc;
   return read_stats(c, s);
-}
-
-int launch_lumi_fp64(const LumiView& v, hipStream_t s)
-{
-  constexpr int kWaves = 4;
-  const int nwork = lumi_work_items(v.npts, v.fp.mirror_ny, v.mirror_out);
-  if (nwork <= 0) return 0;
-  hipLaunchKernelGGL((k_lumi_fp64<kWaves, SingleLumi>), dim3(nblk(nwork, kWaves)), dim3(64 * kWaves), 0, s,
-                     SingleLumi{v});
-  UPC_HIP(hipGetLastError());
-  return 0;
 }
 
 // Row and work-item masks of a grid restricted to the bins with
@@ -382,25 +415,26 @@ int lumi_grid_subset_fp64(upc_ctx* c, const unsigned char* d_need_bin, double* d
   const int mirror_out = mirror_ny > 0;
   const int nwork = lumi_work_items(npts, mirror_ny, mirror_out);
   unsigned char *row_need = nullptr, *item_need = nullptr;
+  int* need_perm = nullptr;
   UPC_HIP(hipMallocAsync((void**)&row_need, (size_t)nrows, s));
   UPC_HIP(hipMallocAsync((void**)&item_need, (size_t)nwork, s));
+  UPC_HIP(hipMallocAsync((void**)&need_perm, sizeof(int) * (size_t)nrows, s));
   hipLaunchKernelGGL(k_subset_masks, dim3(nblk(std::max(nrows, nwork), 256)), dim3(256), 0, s, d_need_bin, npts,
                      nrows, mirror_ny, nwork, mirror_out, row_need, item_need);
-  rc = run_flux(c, npts, mirror_ny, s, row_need);
+  rc = run_flux(c, npts, mirror_ny, s, row_need, need_perm);
   if (rc) return rc;
   const FluxParams fp = flux_params(c, mirror_ny);
-  constexpr int kWaves = 4;
   LumiView v{c->work.d_points, c->work.d_row_logd, c->work.d_flux, fp, c->d_gaa, c->d_bk, c->d_scalars, npts,
              g.breakup_mode, 0, d_Lt, nullptr, nullptr, mirror_out};
   v.need = item_need;
-  SingleLumi jr{v};
   {
     PhaseScope ph(c, s, UPC_PHASE_LUMI);
-    hipLaunchKernelGGL((k_lumi_fp64<kWaves, SingleLumi>), dim3(nblk(nwork, kWaves)), dim3(64 * kWaves), 0, s,
-                       jr);
+    rc = launch_lumi_fp64(v, s);
   }
   (void)hipFreeAsync(row_need, s);
   (void)hipFreeAsync(item_need, s);
+  (void)hipFreeAsync(need_perm, s);
+  if (rc) return rc;
   UPC_HIP(hipGetLastError());
   return read_stats(c, s);
 }
@@ -565,7 +599,7 @@ int enqueue_flux_form(upc_ctx* c, const double* d_b, const double* d_k, int n, d
   if (team > 1)
     launch_qags_team(team, ts, n, d_out, d_ier, w.counters, w.overflow, c->qags_cap, s);
   else
-    hipLaunchKernelGGL((k_flux_qags<kQagsCap, PointTask>), dim3(qags_persistent_blocks(kQagsBlocksPerCu)),
+    hipLaunchKernelGGL((k_flux_qags<kQagsCap, PointTask>), dim3(cu_count() * kQagsBlocksPerCu),
                      dim3(kQagsBlock), 0, s, ts, w.counters + 4, w.counters + 5, d_out, d_ier, w.counters, w.overflow, c->qags_cap);
   hipLaunchKernelGGL((k_flux_qags_wave<PointTask>), dim3(kQagsWaveBlocks), dim3(64), 0, s, ts, w.overflow,
                      w.counters, d_out, d_ier);

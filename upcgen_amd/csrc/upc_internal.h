@@ -41,7 +41,8 @@ constexpr int kNBkUsed = 20000 + kBkGuard;
 // Rows are bucketed by photon energy at 256 buckets per octave (0.3 %): on the
 // 1001 x 121 grid a group of 64 rows spans three buckets.
 constexpr int kRowsPerOctave = 256;
-constexpr int kRowBuckets = 40 * kRowsPerOctave;
+constexpr int kRowOctaves = 40;
+constexpr int kRowBuckets = kRowOctaves * kRowsPerOctave;
 
 struct LumiWork {
   size_t rows_cap = 0;
@@ -52,9 +53,12 @@ struct LumiWork {
   double* d_flux = nullptr;       // [rows][120]
   size_t idx_cap = 0, over_cap = 0;
   int* d_idx = nullptr;           // per-point calls: point indices
-  // [0] evals [1] qags bad [2] overflow n [4] integrals [5] cursor [6] rows in d_perm
+  // [0] evals [1] qags bad [2] overflow n [4] integrals [5] cursor (per-point calls) [6] rows in d_perm
   unsigned long long* d_counters = nullptr;
   int* d_hist = nullptr;          // [kRowBuckets] behind d_counters: rows per k bucket, then their offsets
+  unsigned long long* d_cursors = nullptr;  // behind d_hist: work cursors of the row QAGS launches
+  size_t ncursors = 0;
+  double* d_h = nullptr;          // integrand factors of up to kRowsChunk groups of 64 rows
   long long* d_overflow = nullptr;  // tasks that exceeded the fast workspace
   double* d_points = nullptr;     // (M, Y, dm, dy) per point
   size_t points_cap = 0;
@@ -97,6 +101,7 @@ struct upc_ctx {
   double* d_ff_y = nullptr;         // 10^6 knot values
   double* d_ff_c = nullptr;         // 10^6 second-derivative coefficients
   double4* d_ff = nullptr;          // 10^6 - 1 intervals
+  double* d_j1 = nullptr;           // J1 on the shared b grid (k_flux_j1; form-factor flux only)
   double* d_bk_y = nullptr;         // kNBkUsed knot values
   double* d_bk_c = nullptr;
   double4* d_bk = nullptr;          // kNBkUsed - 1 intervals
@@ -155,6 +160,8 @@ int launch_overlap(upc_ctx* c, const double* d_b, int n, int which, double* d_ou
 int lumi_points_fp64(upc_ctx* c, const double* d_pts, int npts, double* d_L, double* d_Ls,
                      double* d_Lp, hipStream_t s);
 int make_grid_points(upc_ctx* c, hipStream_t s);
+size_t flux_j1_elems();
+int launch_flux_j1(upc_ctx* c, hipStream_t s);
 // The FP64 grid of the bins with d_need_bin[i] != 0 only (flux rows and
 // contraction items they need; other bins of d_Lt are undefined).
 int lumi_grid_subset_fp64(upc_ctx* c, const unsigned char* d_need_bin, double* d_Lt, hipStream_t s);

@@ -76,8 +76,76 @@ struct QagsSmallStore {
     const int sh = 4 * (k - 1);
     io = (io & ~(15ull << sh)) | ((unsigned long long)(v - 1) << sh);
   }
-  __device__ double* eps() { return a->eps; }
-  __device__ double* r3() { return a->r3; }
+  __device__ double ep(int k) const { return a->eps[k]; }
+  __device__ void set_ep(int k, double v) { a->eps[k] = v; }
+  __device__ double r3(int k) const { return a->r3[k]; }
+  __device__ void set_r3(int k, double v) { a->r3[k] = v; }
+};
+
+// The same lists in LDS (a column of the wavefront's table per lane, stride
+// 64), the interval lists past their first entries in private memory.  The
+// flux integrals end with 7.5 intervals on average and 15 at most, their
+// epsilon table with at most 11 entries (Pb, Xe, O, Au grids; an integral that
+// needs more than the 13 here goes to the 1000-interval kernel).  A step of
+// the bookkeeping waits for some twenty list reads one after another: private
+// memory answers in about 700 cycles, LDS in 100.
+template <int CAP>
+struct QagsLdsStore : QagsSmallStore<CAP> {
+  static constexpr int kLists = 8, kLdsEps = 13;
+  static constexpr int kEps = kLdsEps + 1;  // 1-based
+  struct Columns {                          // per wavefront
+    double rl[kLists][64], el[kLists][64], eps[kLdsEps][64];
+    unsigned iv[kLists][64];
+  };
+  struct Arrays {
+    unsigned iv[CAP - kLists];
+    double rl[CAP - kLists], el[CAP - kLists];
+  };
+  using Iv = unsigned;
+  using LdsD = __attribute__((address_space(3))) double;
+  using LdsU = __attribute__((address_space(3))) unsigned;
+  static constexpr int kEl = kLists * 64, kEp = 2 * kLists * 64;  // columns after rl's
+  LdsD* l;   // the lane's rl column
+  LdsU* liv;
+  Arrays* a;
+  double r1, r2, r3v;
+
+  // The two addresses are opaque to the compiler, so that an entry is one of
+  // them plus an immediate offset and not an address of its own in a register.
+  __device__ void bind(Columns* c, int lane, Arrays* priv)
+  {
+    l = (LdsD*)&c->rl[0][lane];
+    liv = (LdsU*)&c->iv[0][lane];
+    asm volatile("" : "+v"(l), "+v"(liv));
+    a = priv;
+  }
+  __device__ Iv iv(int k) const { return k <= kLists ? liv[(k - 1) * 64] : a->iv[k - 1 - kLists]; }
+  __device__ void set_iv(int k, Iv v)
+  {
+    if (k <= kLists) liv[(k - 1) * 64] = v;
+    else a->iv[k - 1 - kLists] = v;
+  }
+  __device__ double rl(int k) const { return k <= kLists ? l[(k - 1) * 64] : a->rl[k - 1 - kLists]; }
+  __device__ void set_rl(int k, double v)
+  {
+    if (k <= kLists) l[(k - 1) * 64] = v;
+    else a->rl[k - 1 - kLists] = v;
+  }
+  __device__ double el(int k) const { return k <= kLists ? l[kEl + (k - 1) * 64] : a->el[k - 1 - kLists]; }
+  __device__ void set_el(int k, double v)
+  {
+    if (k <= kLists) l[kEl + (k - 1) * 64] = v;
+    else a->el[k - 1 - kLists] = v;
+  }
+  __device__ double ep(int k) const { return l[kEp + (k - 1) * 64]; }
+  __device__ void set_ep(int k, double v) { l[kEp + (k - 1) * 64] = v; }
+  __device__ double r3(int k) const { return k == 1 ? r1 : (k == 2 ? r2 : r3v); }
+  __device__ void set_r3(int k, double v)
+  {
+    r1 = k == 1 ? v : r1;
+    r2 = k == 2 ? v : r2;
+    r3v = k == 3 ? v : r3v;
+  }
 };
 
 // The reference's workspace: limit 1000, FP64 end points, one per lane in
@@ -116,8 +184,10 @@ struct QagsBigStore {
   __device__ void set_el(int k, double v) { a->elist[k - 1] = v; }
   __device__ int io_at(int k) const { return a->iord[k - 1]; }
   __device__ void set_io(int k, int v) { a->iord[k - 1] = v; }
-  __device__ double* eps() { return a->eps; }
-  __device__ double* r3() { return a->r3; }
+  __device__ double ep(int k) const { return a->eps[k]; }
+  __device__ void set_ep(int k, double v) { a->eps[k] = v; }
+  __device__ double r3(int k) const { return a->r3[k]; }
+  __device__ void set_r3(int k, double v) { a->r3[k] = v; }
 };
 
 // dqpsrt over a store (1-based indices).
@@ -181,8 +251,36 @@ struct Qags {
   static constexpr int limit = kQagsLimit;
   S s;
   Iv cur;  // the interval being bisected (the root before the first QK21)
-  double result, abserr, area, errsum, errbnd, errmax, erlarg, ertest, small, correc, defabs, erlast;
+  double result, abserr, area, errsum, errbnd, errmax, erlarg, ertest, small, correc, defabs;
   int ier, last, ierro, iroff1, iroff2, iroff3, ksgn, ktmin, maxerr, nrmax, nres, numrl2, extrap, noext, phase;
+  // The counters between steps, in three registers instead of thirteen: iroff1,
+  // iroff2 <= 10, iroff3 <= 20, the rest by the limit of 1000 intervals (ier is
+  // 0 while the integral runs).
+  unsigned p0, p1, p2;
+  __device__ __forceinline__ void pack()
+  {
+    p0 = (unsigned)ierro | (unsigned)iroff1 << 2 | (unsigned)iroff2 << 6 | (unsigned)iroff3 << 10 |
+         (unsigned)(ksgn > 0) << 15 | (unsigned)extrap << 16 | (unsigned)noext << 17 | (unsigned)numrl2 << 18;
+    p1 = (unsigned)last | (unsigned)maxerr << 10 | (unsigned)nrmax << 20;
+    p2 = (unsigned)nres | (unsigned)ktmin << 16;
+  }
+  __device__ __forceinline__ void unpack()
+  {
+    ier = 0;
+    ierro = p0 & 3;
+    iroff1 = p0 >> 2 & 15;
+    iroff2 = p0 >> 6 & 15;
+    iroff3 = p0 >> 10 & 31;
+    ksgn = p0 >> 15 & 1 ? 1 : -1;
+    extrap = p0 >> 16 & 1;
+    noext = p0 >> 17 & 1;
+    numrl2 = p0 >> 18;
+    last = p1 & 1023;
+    maxerr = p1 >> 10 & 1023;
+    nrmax = p1 >> 20;
+    nres = p2 & 65535;
+    ktmin = p2 >> 16;
+  }
 
   __device__ void start()
   {
@@ -204,8 +302,8 @@ struct Qags {
   {
     if (last > s.limit()) return kQagsOverflow;
     cur = s.iv(maxerr);
-    erlast = errmax;
     phase = 2;
+    pack();
     return kQagsRunning;
   }
 
@@ -268,7 +366,7 @@ struct Qags {
       if (abserr <= 100.0 * epmach * defabs && abserr > errbnd) ier = 2;
       if (limit == 1) ier = 1;
       if (ier != 0 || (abserr <= errbnd && abserr != resasc0) || abserr == 0.0) return kQagsDone;
-      s.eps()[1] = result;
+      s.set_ep(1, result);
       errmax = abserr;
       maxerr = 1;
       area = result;
@@ -289,6 +387,8 @@ struct Qags {
       return begin_bisection();
     }
     // phase 2: body of the dqagse main loop for this value of `last`
+    unpack();
+    const double erlast = errmax;  // the error of the interval just bisected
     const double a1 = S::lo(cur), b1 = S::mid(cur), a2 = b1, b2 = S::hi(cur);
     const double area1 = o.result, error1 = o.abserr, defab1 = o.resasc;
     const double area2 = o2.result, error2 = o2.abserr, defab2 = o2.resasc;
@@ -331,7 +431,7 @@ struct Qags {
       small = fabs(kQagsB - kQagsA) * 0.375;
       erlarg = errsum;
       ertest = errbnd;
-      s.eps()[2] = area;
+      s.set_ep(2, area);
       ++last;
       return begin_bisection();
     }
@@ -365,9 +465,9 @@ struct Qags {
     }
     if (numrl2 + 3 > S::kEps - 1) return kQagsOverflow;  // small tables only
     numrl2++;
-    s.eps()[numrl2] = area;
+    s.set_ep(numrl2, area);
     double reseps, abseps;
-    qelg(&numrl2, s.eps(), &reseps, &abseps, s.r3(), &nres);
+    qelg(s, &numrl2, &reseps, &abseps, &nres);
     ktmin++;
     if (ktmin > 5 && abserr < 1e-3 * errsum) ier = 5;
     if (abseps < abserr) {

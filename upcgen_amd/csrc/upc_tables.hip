@@ -544,6 +544,7 @@ int alloc_tables(upc_ctx* c)
   c->bk_scratch_elems = (size_t)2 * (kSplineChunk + 2 * kSplineGuard) * nblk(kNBkUsed, kSplineChunk);
   UPC_HIP(hipMalloc(&c->d_bk_scratch, sizeof(double) * c->bk_scratch_elems));
   UPC_HIP(hipMalloc(&c->d_gaa_scratch, sizeof(double) * kNB));
+  if (!c->cfg.flux_point) UPC_HIP(hipMalloc(&c->d_j1, sizeof(double) * flux_j1_elems()));
   for (int i = 0; i < 2; ++i) {
     UPC_HIP(hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking));
     UPC_HIP(hipEventCreateWithFlags(&c->ev_join[i], hipEventDisableTiming));
@@ -564,7 +565,7 @@ void free_tables(upc_ctx* c)
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   void* ptrs[] = {c->d_scalars, c->d_ta, c->d_gaa, c->d_ff_y, c->d_ff_c, c->d_ff,
                   c->d_bk_y, c->d_bk_c, c->d_bk, c->d_ee, c->d_se, c->d_spline_scratch,
-                  c->d_bk_scratch, c->d_gaa_scratch};
+                  c->d_bk_scratch, c->d_gaa_scratch, c->d_j1};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
 }
@@ -603,6 +604,8 @@ int build_tables(upc_ctx* c, hipStream_t s)
   hipLaunchKernelGGL(k_gaa_g, dim3(kNB), dim3(256), 0, sg, c->d_scalars, c->d_ta, c->d_gaa_scratch);
   hipLaunchKernelGGL(k_gaa_spline, dim3(1), dim3(256), 0, sg, c->d_gaa_scratch, c->d_gaa);
   UPC_HIP(hipGetLastError());
+  if (!p.flux_point)
+    if (int rc = launch_flux_j1(c, sg)) return rc;
   UPC_HIP(hipEventRecord(c->ev_join[0], sg));
   hipLaunchKernelGGL(k_breakup_init, dim3(1), dim3(256), 0, sb, c->g1, c->d_ee, c->d_se, c->d_scalars);
   int rc = 0;
