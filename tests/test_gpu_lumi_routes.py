@@ -1,0 +1,43 @@
+"""The contraction gives a point one wavefront, or the eight of a workgroup where
+a launch has at most 8192 work items.  Both cut a point's pair list into the
+same runs and add them in the same order, so a point's luminosity has the same
+bits on both.  No term of the sum is negative, so a point whose flux lies mostly
+below the hadronic knee keeps its relative accuracy: 1e-10 against the oracle
+(6,000 nodes and 240 flux values, each within 1e-12)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+N = 8193  # one wavefront per point
+
+
+@pytest.mark.parametrize("mode,pol", [(1, 0), (2, 0), (4, 1)])
+def test_routes_give_the_same_bits(gpu, mode, pol):
+    import torch
+    rng = np.random.default_rng(11)
+    M = np.exp(rng.uniform(np.log(1.0), np.log(100.0), N))
+    Y = rng.uniform(-5.0, 5.0, N)
+    t = lambda x: torch.as_tensor(x, device="cuda")
+    c = gpu.Context(flux_point=1, breakup_mode=mode, use_polarized=pol, nm=3, ny=3)
+
+    def run(n):
+        out = c.lumi_points(t(M[:n].copy()), t(Y[:n].copy()))
+        return [o.cpu().numpy() for o in (out if isinstance(out, tuple) else (out,))]
+
+    whole = run(N)
+    for n in (1, 3, 100, 8192):
+        for a, b in zip(run(n), whole):
+            assert np.array_equal(a.view(np.uint64), b[:n].view(np.uint64)), n
+
+
+@pytest.mark.parametrize("M,Y", [(81.06126864613289, -0.06555698284985478), (72.86267059069179, 0.2097470597513258)])
+def test_flux_below_the_knee(gpu, oracle_ctx, M, Y):
+    """Au-Au at 200 GeV: 1e-9 and less of the flux product has any overlap term."""
+    import torch
+    cfg = dict(Z=79, A=197, a=0.54, sqrts=200.0, flux_point=0, breakup_mode=4)
+    c = gpu.Context(R=gpu.wood_saxon_radius(197), nm=3, ny=3, **cfg)
+    L = c.lumi_points(torch.tensor([M], device="cuda", dtype=torch.float64),
+                      torch.tensor([Y], device="cuda", dtype=torch.float64)).cpu().numpy()[0]
+    o = oracle_ctx(R=gpu.wood_saxon_radius(197), **cfg)
+    assert abs(L / o.lumi(M, Y) - 1) <= 1e-10

@@ -64,51 +64,6 @@ __device__ __forceinline__ double node_b2(double b1, double b2, double c)
   return fma(2.0 * b1 * b2, c, fma(b1, b1, b2 * b2));
 }
 
-// The phi sum of one node pair: sum_k w_k P(min(b, 20)) G(b) (G = 1 for
-// b >= 20); polarised: cos^2 and sin^2 weighted sums.
-//
-// Below the hadronic knee (b < ~11 fm for Pb-Pb) the G_AA spline holds only
-// the decaying ringing of the natural spline, |G| < 1e-30.  Below bskip
-// (x < bskip2) |G| < gskip = p20 2^-70 holds for every b, and P G is taken
-// as 0 without sqrt, G or P: the caller subtracts p20 sum_k w_k from the
-// same sum, and |P G| <= |G| is below 2^-70 of that term, 10^5 times below
-// the rounding that the order of the pair sums already brings.  Above
-// bskip, modes 2-4 still skip the breakup spline wherever the G just
-// evaluated is below gskip (mode 1 has P = 1 and reads no breakup spline).
-template <bool POL>
-__device__ __forceinline__ void node_k(double b1, double b2, const double* cosk, const double* w5,
-                                       int mode, double p20, double gskip, double bskip2, const double4* gaa,
-                                       const double4* __restrict__ bk, double* ks, double* kp)
-{
-  const double db = 20. / (kNB - 1);
-  double s = 0.0, p = 0.0;
-#pragma unroll
-  for (int k = 0; k < 5; ++k) {
-    const double c = cosk[k];
-    const double x = node_b2(b1, b2, POL ? -c : c);
-    double breakup = mode != 1 ? p20 : 1., gaa_v = 1.;
-    if (x < bskip2) {
-      breakup = 0.0;
-    } else if (x < 400.) {  // sqrt(x) >= 20 whenever x >= 400
-      const double b = sqrt(x);
-      if (b < 20.) {
-        gaa_v = spline_eval_near(gaa, 0.0, db, 1.0 / db, kNB, b);
-        if (mode != 1)
-          breakup = fabs(gaa_v) < gskip ? 0.0 : spline_eval_near(bk, kBkMin, kDBk, 1.0 / kDBk, kNBkUsed, b);
-      }
-    }
-    if (POL) {  // w5[5 + k] = sin^2(phi_k)
-      s += breakup * gaa_v * w5[k] * c * c;
-      p += breakup * gaa_v * w5[k] * w5[5 + k];
-    } else {
-      s += breakup * gaa_v * w5[k];
-    }
-  }
-  *ks = s;
-  *kp = p;
-}
-
-
 // fluxPoint (src/UpcCrossSection.cpp:166-178): g1 for both beams.
 __device__ __forceinline__ double flux_point(double b, double k, double g1, double factor)
 {
@@ -1354,19 +1309,6 @@ __global__ __launch_bounds__(64) void k_flux_qags_wave(TS ts, const long long* _
   }
 }
 
-// ---------------------------------------------------------------------------
-// FP64 luminosity: one wavefront per (M, Y) point.
-//
-// For a pair of nodes (b1_i, b2_j) the phi sum K_ij = sum_k w_k P(b) G(b),
-// b^2 = b1^2 + b2^2 +- 2 b1 b2 cos(phi_k).  Where every node has b >= 20 fm
-// the reference evaluates P at the 20 fm clamp and G = 1, so K_ij is the
-// constant S0 (same arithmetic).  For fixed i the pairs with some b < 20 form
-// one contiguous j range (the smallest b^2 is always the extreme-cos node), so
-//   L = 2 pi^2 M [ S0 (sum_i W1_i)(sum_j W2_j) + sum_{band} W1_i W2_j (K_ij - S0) ]
-// with W = N(b, k) b (b_h - b_l).  The band pairs are spread evenly over the
-// 64 lanes.
-// ---------------------------------------------------------------------------
-
 // What the contraction reads of one job (one context's grid).
 struct LumiView {
   const double* pts;       // (M, Y, dm, dy) of the job's points
@@ -1411,239 +1353,6 @@ __device__ __forceinline__ void work_point(int q, int mirror_ny, int mirror_out,
 __device__ __forceinline__ void lumi_work_point(const LumiView& v, int q, int* p, int* pm)
 {
   work_point(q, v.fp.mirror_ny, v.mirror_out, p, pm);
-}
-
-// Job resolvers: the job and first point of a block.
-struct SingleLumi {
-  static constexpr int kWavesPerEu = 5;  // register budget of k_lumi_fp64 (waves per SIMD)
-  LumiView v;
-  __device__ void get(int blk, int waves, LumiView* out, int* p0) const
-  {
-    *out = v;
-    *p0 = blk * waves;
-  }
-};
-
-template <int WAVES>
-struct LumiSmem {
-  double4 gaa[kNB];
-  double sb1[WAVES][kNB1], sb2[WAVES][kNB2];
-  double sw1[WAVES][kNB1], sw2[WAVES][kNB2];
-  int spre[WAVES][kNB1 + 1], sjlo[WAVES][kNB1];
-  double sp2[WAVES][kNB2 + 1];  // prefix sums of sw2
-  double cosk[5], w5[10];
-};
-
-template <bool POL, int WAVES>
-__device__ __forceinline__ void lumi_fp64_body(const LumiView& v, int p0, LumiSmem<WAVES>& sm)
-{
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int q = p0 + wv;
-  const bool live = q < lumi_work_items(v.npts, v.fp.mirror_ny, v.mirror_out) && (!v.need || v.need[q]);
-  // a masked launch (block-uniform v.need): blocks with no needed item end here
-  if (v.need && !__syncthreads_or(live)) return;
-  for (int i = threadIdx.x; i < kNB - 1; i += blockDim.x) sm.gaa[i] = v.gaa[i];
-  if (threadIdx.x < 5) {
-    const double c = cos(kPi * kGLx5[threadIdx.x]);
-    const double sn = sin(kPi * kGLx5[threadIdx.x]);
-    sm.cosk[threadIdx.x] = c;
-    sm.w5[threadIdx.x] = kGLw5[threadIdx.x];
-    sm.w5[5 + threadIdx.x] = sn * sn;
-  }
-  int p = 0, pm = -1;
-  if (live) lumi_work_point(v, q, &p, &pm);
-  const FluxParams& fp = v.fp;
-  const double p20 = v.sc->p20;
-  double M = 0, dm = 1, dy = 1;
-  LogGrid lg2{};
-  if (live) {
-    M = v.pts[4 * p];
-    dm = v.pts[4 * p + 2];
-    dy = v.pts[4 * p + 3];
-    const int r2 = k2_row(p, v.npts, fp.mirror_ny);
-    const double logd1 = v.row_logd[p], logd2 = v.row_logd[r2];
-    lg2.init(fp.bmin, logd2);
-    const double* f1 = v.flux + (long)p * kNB1;
-    const double* f2 = v.flux + (long)r2 * kNB1;
-    for (int j = lane; j < kNB1; j += 64) {
-      double bl, bh;
-      const double b1 = row_node(fp.bmin, logd1, j, &bl, &bh);
-      sm.sb1[wv][j] = b1;
-      sm.sw1[wv][j] = f1[j] * b1 * (bh - bl);
-      const double b2 = row_node(fp.bmin, logd2, j, &bl, &bh);
-      sm.sb2[wv][j] = b2;
-      sm.sw2[wv][j] = f2[j] * b2 * (bh - bl);
-    }
-  }
-  __syncthreads();
-  // the extreme-cos node has the smallest b for every pair, cmax the largest
-  const double cext = POL ? -sm.cosk[0] : sm.cosk[4];
-  const double cmax = POL ? -sm.cosk[4] : sm.cosk[0];
-  if (!live) return;
-  // prefix sums of sw2: sp2[j] = sum_{j' < j} sw2[j']
-  {
-    double a0 = sm.sw2[wv][lane], a1 = lane + 64 < kNB2 ? sm.sw2[wv][lane + 64] : 0.0;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const double u0 = __shfl_up(a0, o), u1 = __shfl_up(a1, o);
-      if (lane >= o) {
-        a0 += u0;
-        a1 += u1;
-      }
-    }
-    const double half = __shfl(a0, 63);
-    sm.sp2[wv][lane + 1] = a0;
-    if (lane + 64 < kNB2) sm.sp2[wv][lane + 65] = half + a1;
-    if (lane == 0) sm.sp2[wv][0] = 0.0;
-  }
-  const double bskip = v.sc->bskip, bskip2 = bskip * bskip;
-  // Pairs whose largest node is below bskip have P G = 0 at every node, so
-  // they add -s0 sw1[i] sw2[j]: per row, -s0 sw1[i] sp2[ja] for the run
-  // j < ja (b^2 at cmax > 0 grows with b2).  Those pairs are in the band
-  // (b^2 < bskip^2 <= 400 at every node), which therefore starts at j = 0;
-  // the walk takes the band from ja on.
-  double wan = 0.0;  // sum over rows of sw1[i] sp2[ja]
-  wave_sync_lds();
-  // Band of row i: the j with b^2 < 400 at the extreme cosine.  b^2 is convex
-  // in b2 (smallest at b2 = -b1 cext), so the band is the run of j around
-  // that vertex.  The vertex and both ends (roots b2 = vtx -+ sqrt(400 -
-  // b1^2 (1 - cext^2))) are guessed on the log grid of b2 and stepped to
-  // exactness with the same comparisons a bisection would make.
-  int cnt[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int i = lane + 64 * h;
-    cnt[h] = 0;
-    if (i < kNB1) {
-      const double b1 = sm.sb1[wv][i];
-      const double* b2s = sm.sb2[wv];
-      auto inb = [&](int j) { return node_b2(b1, b2s[j], cext) < 400.0; };
-      const double vtx = -b1 * cext;
-      int lo = lg2.first_ge(vtx, kNB2);  // first j with b2_j >= vtx
-      while (lo > 0 && b2s[lo - 1] >= vtx) --lo;
-      while (lo < kNB2 && b2s[lo] < vtx) ++lo;
-      int jc = -1;
-      if (lo < kNB2 && inb(lo)) jc = lo;
-      if (lo > 0 && inb(lo - 1)) jc = lo - 1;
-      int jlo = 0;
-      if (jc >= 0) {
-        const double d = 400.0 - b1 * b1 * (1.0 - cext * cext), sd = sqrt(d > 0.0 ? d : 0.0);
-        int a = lg2.first_ge(vtx - sd, kNB2);  // first j in band: outside before it, inside from it to jc
-        a = a > jc ? jc : a;
-        while (a > 0 && inb(a - 1)) --a;
-        while (a < jc && !inb(a)) ++a;
-        jlo = a;
-        a = lg2.first_ge(vtx + sd, kNB2) - 1;  // last j in band
-        a = a < jc ? jc : (a > kNB2 - 1 ? kNB2 - 1 : a);
-        while (a < kNB2 - 1 && inb(a + 1)) ++a;
-        while (a > jc && !inb(a)) --a;
-        // first j with b^2 >= bskip^2 at cmax (b^2 grows with b2 there)
-        auto low = [&](int j) { return node_b2(b1, b2s[j], cmax) < bskip2; };
-        const double da = bskip2 - b1 * b1 * (1.0 - cmax * cmax);
-        int ja = da > 0.0 ? lg2.first_ge(-b1 * cmax + sqrt(da), kNB2) : 0;
-        while (ja > 0 && !low(ja - 1)) --ja;
-        while (ja < kNB2 && low(ja)) ++ja;
-        if (ja > 0) {
-          wan += sm.sw1[wv][i] * sm.sp2[wv][ja];
-          jlo = ja;
-        }
-        cnt[h] = a >= jlo ? a - jlo + 1 : 0;
-      }
-      sm.sjlo[wv][i] = jlo;
-    }
-  }
-  // inclusive wave scan of the two halves of the row counts
-  int c0 = cnt[0], c1 = cnt[1];
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u0 = __shfl_up(c0, o), u1 = __shfl_up(c1, o);
-    if (lane >= o) {
-      c0 += u0;
-      c1 += u1;
-    }
-  }
-  const int half = __shfl(c0, 63);
-  sm.spre[wv][lane + 1] = c0;
-  if (lane + 64 < kNB1) sm.spre[wv][lane + 65] = half + c1;
-  if (lane == 0) sm.spre[wv][0] = 0;
-  wave_sync_lds();
-  // S0: the phi sum when every node is at or beyond 20 fm
-  double s0s = 0, s0p = 0;
-  {
-    const double br = v.mode != 1 ? p20 : 1.;
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      if (POL) {
-        s0s += br * 1. * sm.w5[k] * sm.cosk[k] * sm.cosk[k];
-        s0p += br * 1. * sm.w5[k] * sm.w5[5 + k];
-      } else {
-        s0s += br * 1. * sm.w5[k];
-      }
-    }
-  }
-  const int T = sm.spre[wv][kNB1];
-  const double gskip = p20 * 0x1p-70;
-  double accs = 0, accp = 0;
-  int i = 0;  // row of pair t: pre[i] <= t < pre[i + 1]; t only grows
-  for (int t = lane; t < T; t += 64) {
-    while (sm.spre[wv][i + 1] <= t) ++i;
-    const int j = sm.sjlo[wv][i] + (t - sm.spre[wv][i]);
-    double ks, kp;
-    node_k<POL>(sm.sb1[wv][i], sm.sb2[wv][j], sm.cosk, sm.w5, v.mode, p20, gskip, bskip2, sm.gaa, v.bk, &ks,
-                &kp);
-    const double ww = sm.sw1[wv][i] * sm.sw2[wv][j];
-    accs += ww * (ks - s0s);
-    if (POL) accp += ww * (kp - s0p);
-  }
-  double sw1t = 0, sw2t = 0;
-  for (int j = lane; j < kNB1; j += 64) {
-    sw1t += sm.sw1[wv][j];
-    sw2t += sm.sw2[wv][j];
-  }
-  for (int o = 32; o > 0; o >>= 1) {
-    accs += __shfl_down(accs, o);
-    accp += __shfl_down(accp, o);
-    sw1t += __shfl_down(sw1t, o);
-    sw2t += __shfl_down(sw2t, o);
-    wan += __shfl_down(wan, o);
-  }
-  if (lane == 0) {
-    const double pre = 2 * kPi * kPi * M;
-    const double tot_s = s0s * (sw1t * sw2t - wan) + accs;
-    if (POL) {
-      const double tot_p = s0p * (sw1t * sw2t - wan) + accp;
-      const double ls = pre * tot_s * dm * dy, lp = pre * tot_p * dm * dy;
-      v.Ls[p] = ls;
-      v.Lp[p] = lp;
-      if (pm >= 0) {
-        v.Ls[pm] = ls;
-        v.Lp[pm] = lp;
-      }
-    } else {
-      const double l = pre * tot_s * dm * dy;
-      v.L[p] = l;
-      if (pm >= 0) v.L[pm] = l;
-    }
-  }
-}
-
-// WAVES points per block; the resolver maps the block to its job (all
-// threads of a block take the same branch, so the barriers are uniform).
-// JR::kWavesPerEu budgets the registers: the breakup-spline gathers from L2
-// bound the kernel, and for one grid a fifth wave per SIMD hides more of
-// their latency (96 VGPRs, a few spilled; the LDS of 4-wave blocks allows 5
-// blocks per CU: 1.58 -> 1.48 ms on the 1001 x 121 grid), while the batch's
-// mostly polarised jobs spill more at that budget and keep 4.
-template <int WAVES, class JR>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(JR::kWavesPerEu))) void k_lumi_fp64(
-    JR jr)
-{
-  __shared__ LumiSmem<WAVES> sm;
-  LumiView v;
-  int p0;
-  jr.get(blockIdx.x, WAVES, &v, &p0);
-  if (v.pol) lumi_fp64_body<true, WAVES>(v, p0, sm);
-  else lumi_fp64_body<false, WAVES>(v, p0, sm);
 }
 
 // Exclusive prefix sums of the row counts per bucket (in place), one block per
