@@ -63,16 +63,23 @@ __device__ __forceinline__ unsigned short bf16_bits(float f)
 __device__ __forceinline__ float bf16_value(unsigned short h) { return __uint_as_float((uint32_t)h << 16); }
 __device__ __forceinline__ float bf16_round(float f) { return bf16_value(bf16_bits(f)); }
 
-enum { kEpiStore = 0, kEpiBiasSilu = 1 };
+enum { kEpiSiluBwd = 0, kEpiBiasSilu = 1 };
 
-// C[M x N] = opA(A)[M x K] opB(B)[K x N], bf16 operands, FP32 accumulation.
-// TA: element (m, k) of A at A[k * lda + m], else A[m * lda + k].
+// silu'(z)
+__device__ __forceinline__ float silu_grad(float z)
+{
+  const float s = 1.f / (1.f + expf(-z));
+  return s * (1.f + z * (1.f - s));
+}
+
+// C[M x N] = A[M x K] opB(B)[K x N], bf16 operands, FP32 accumulation.
 // TB: element (k, n) of B at B[n * ldb + k], else B[k * ldb + n].
 // M, N multiples of 16, K a multiple of 32.  One wave per 16 x 16 tile with
 // the 16x16x32 MFMA layout: lane l supplies row / column (l & 15) and k
 // values 8 (l >> 4) .. +7 of each 32-deep step, and holds C[4 (l >> 4) + i][l & 15].
 // kEpiBiasSilu: C = acc + bias[n] (pre-activation) and H = silu(C).
-template <bool TA, bool TB, int EPI, bool SPLIT>
+// kEpiSiluBwd: C = acc silu'(H), H the layer's pre-activations.
+template <bool TB, int EPI, bool SPLIT>
 __global__ __launch_bounds__(256) void k_sur_mm(int M, int N, int K, const float* __restrict__ A, int lda,
                                                 const float* __restrict__ B, int ldb, float* __restrict__ C,
                                                 int ldc, const float* __restrict__ bias, float* __restrict__ H)
@@ -89,7 +96,7 @@ __global__ __launch_bounds__(256) void k_sur_mm(int M, int N, int K, const float
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const int k = k0 + g4 * 8 + e;
-      const float av = TA ? A[(long)k * lda + m0 + r] : A[(long)(m0 + r) * lda + k];
+      const float av = A[(long)(m0 + r) * lda + k];
       const float bv = TB ? B[(long)(n0 + r) * ldb + k] : B[(long)k * ldb + n0 + r];
       a[e] = bf16_bits(av);
       b[e] = bf16_bits(bv);
@@ -116,8 +123,70 @@ __global__ __launch_bounds__(256) void k_sur_mm(int M, int N, int K, const float
       C[m * ldc + n] = v;
       H[m * ldc + n] = v / (1.f + expf(-v));
     } else {
-      C[m * ldc + n] = v;
+      C[m * ldc + n] = v * silu_grad(H[m * ldc + n]);
     }
+  }
+}
+
+// Gradients of one layer's weights and biases over a slice of the batch,
+//   dW[m][n] = sum_b dZ[b][m] In[b][n],  db[m] = sum_b dZ[b][m],
+// left in the slice's own copy of the parameter vector (k_sur_grad_sum adds the
+// copies in order).  The sum over the batch is the long one: one wavefront per
+// 16 x 16 tile of dW is 64 chains of B / 32 steps, 140 us at B = 8192; slices of
+// the batch times 32-column blocks fill the chip, 8 us.  A workgroup's four
+// wavefronts take 32 of the 128 rows of dW each (2 x 2 tiles; the operands as
+// in k_sur_mm, their rows 64 contiguous bytes).  Products as k_sur_mm.
+constexpr int kSurSlices = 64;
+
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void k_sur_dw(int B, int rows, const float* __restrict__ dZ,
+                                                const float* __restrict__ In, int N, float* __restrict__ part,
+                                                int offw, int offb)
+{
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g4 = lane >> 4;
+  const int m0 = wv * 32, n0 = blockIdx.y * 32;
+  const int b0 = blockIdx.x * rows, b1 = min(B, b0 + rows);
+  float* out = part + (size_t)blockIdx.x * kSurParams;
+  f32x4 acc[2][2] = {};
+  float bsum[2] = {0.f, 0.f};
+  for (int k0 = b0; k0 < b1; k0 += 32) {
+    bf16x8 hi[4], lo[4];  // dZ tiles, In tiles
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float* src = q < 2 ? dZ + m0 + 16 * q + r : In + n0 + 16 * (q - 2) + r;
+      const int ld = q < 2 ? kSurH : N;
+      u16x8 h, l;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = src[(size_t)(k0 + g4 * 8 + e) * ld];
+        if (q < 2) bsum[q] += v;
+        h[e] = bf16_bits(v);
+        l[e] = bf16_bits(v - bf16_value(h[e]));
+      }
+      hi[q] = __builtin_bit_cast(bf16x8, h);
+      lo[q] = __builtin_bit_cast(bf16x8, l);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[i], hi[2 + j], acc[i][j], 0, 0, 0);
+        if (SPLIT) {
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi[i], lo[2 + j], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo[i], hi[2 + j], acc[i][j], 0, 0, 0);
+        }
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        out[offw + (m0 + 16 * i + 4 * g4 + e) * N + n0 + 16 * j + r] = acc[i][j][e];
+    bsum[i] += __shfl_xor(bsum[i], 16);
+    bsum[i] += __shfl_xor(bsum[i], 32);
+    if (blockIdx.y == 0 && g4 == 0) out[offb + m0 + 16 * i + r] = bsum[i];
   }
 }
 
@@ -347,56 +416,48 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_sur_infer(int B, const flo
   }
 }
 
-// dZ3 = g[b] w4(W4[o]) silu'(Z3)
+// dZ3 = g[b] w4(W4[o]) silu'(Z3) of a slice of the batch, and the slice's
+// gradients of the output layer, dW4 = sum_b g[b] H3[b] and db4 = sum_b g[b].
 template <bool SPLIT>
-__global__ void k_sur_out_bwd(int B, const float* __restrict__ g, const float* __restrict__ p,
-                              const float* __restrict__ Z, float* __restrict__ dZ)
+__global__ __launch_bounds__(1024) void k_sur_out_bwd(int B, int rows, const float* __restrict__ g,
+                                                      const float* __restrict__ p, const float* __restrict__ Z,
+                                                      const float* __restrict__ H, float* __restrict__ dZ,
+                                                      float* __restrict__ part)
 {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (long)B * kSurH) return;
-  const int o = (int)(i % kSurH);
-  const float z = Z[i], s = 1.f / (1.f + expf(-z));
-  dZ[i] = g[i / kSurH] * out_weight<SPLIT>(p[kOffW4 + o]) * (s * (1.f + z * (1.f - s)));
-}
-
-// dZ = dH silu'(Z), in place on dH
-__global__ void k_sur_silu_bwd(long n, const float* __restrict__ Z, float* __restrict__ dH)
-{
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float z = Z[i], s = 1.f / (1.f + expf(-z));
-  dH[i] *= s * (1.f + z * (1.f - s));
-}
-
-// out[n] = sum_b w[b] X[b][n] (w = 1 when null): one block per column, fixed order.
-__global__ __launch_bounds__(256) void k_sur_colsum(int B, int N, const float* __restrict__ X,
-                                                    const float* __restrict__ w, float* __restrict__ out)
-{
-  __shared__ float red[256];
-  const int n = blockIdx.x;
-  float s = 0.f;
-  for (int b = threadIdx.x; b < B; b += 256) s += (w ? w[b] : 1.f) * X[(long)b * N + n];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int d = 128; d > 0; d >>= 1) {
-    if (threadIdx.x < d) red[threadIdx.x] += red[threadIdx.x + d];
-    __syncthreads();
+  __shared__ float red[8][kSurH], redg[8];
+  const int o = threadIdx.x & (kSurH - 1), w = threadIdx.x / kSurH;
+  const int b0 = blockIdx.x * rows, b1 = min(B, b0 + rows);
+  const float w4 = out_weight<SPLIT>(p[kOffW4 + o]);
+  float s = 0.f, sg = 0.f;
+  for (int b = b0 + w; b < b1; b += 8) {
+    const long i = (long)b * kSurH + o;
+    const float gb = g[b];
+    dZ[i] = gb * w4 * silu_grad(Z[i]);
+    s += gb * H[i];
+    sg += gb;
   }
-  if (threadIdx.x == 0) out[n] = red[0];
+  red[w][o] = s;
+  if (o == 0) redg[w] = sg;
+  __syncthreads();
+  if (w > 0) return;
+  for (int k = 1; k < 8; ++k) s += red[k][o];
+  float* out = part + (size_t)blockIdx.x * kSurParams;
+  out[kOffW4 + o] = s;
+  if (o == 0) {
+    for (int k = 1; k < 8; ++k) sg += redg[k];
+    out[kOffB4] = sg;
+  }
 }
 
-__global__ void k_sur_sum(int B, const float* __restrict__ g, float* __restrict__ out)
+// The slices' gradients, added in order.
+__global__ void k_sur_grad_sum(int slices, const float* __restrict__ part, float* __restrict__ g)
 {
-  __shared__ float red[256];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= kSurParams) return;
   float s = 0.f;
-  for (int b = threadIdx.x; b < B; b += 256) s += g[b];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int d = 128; d > 0; d >>= 1) {
-    if (threadIdx.x < d) red[threadIdx.x] += red[threadIdx.x + d];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = red[0];
+#pragma unroll 8
+  for (int k = 0; k < slices; ++k) s += part[(size_t)k * kSurParams + i];
+  g[i] = s;
 }
 
 // Training-step bookkeeping on the device so a captured step replays as is.
@@ -640,6 +701,7 @@ struct upc_sur {
   float* d_m = nullptr;   // Adam moments
   float* d_v = nullptr;
   float* d_g = nullptr;   // [P] gradient of the current step
+  float* d_part = nullptr;  // [kSurSlices][P] of slices of its batch
   float* d_act = nullptr; // Z1 H1 Z2 H2 Z3 H3 [6][max_batch][128]
   float* d_xb = nullptr;  // [max_batch][32]
   unsigned short* d_img = nullptr;  // k_sur_infer's weight image of one network (prepared per call)
@@ -660,16 +722,16 @@ namespace {
 
 float* act(upc_sur* s, int which) { return s->d_act + (long)which * kSurMaxBatch * kSurH; }
 
-// C = opA(A) opB(B) (+ bias, SiLU) in the surrogate's product precision.
-template <bool TA, bool TB, int EPI>
+// C = A opB(B) with its epilogue, in the surrogate's product precision.
+template <bool TB, int EPI>
 void mm(const upc_sur* s, int tiles, hipStream_t st, int M, int N, int K, const float* A, int lda, const float* B,
         int ldb, float* C, int ldc, const float* bias, float* H)
 {
   if (s->split)
-    hipLaunchKernelGGL((k_sur_mm<TA, TB, EPI, true>), dim3(nblk(tiles, 4)), dim3(256), 0, st, M, N, K, A, lda, B,
+    hipLaunchKernelGGL((k_sur_mm<TB, EPI, true>), dim3(nblk(tiles, 4)), dim3(256), 0, st, M, N, K, A, lda, B,
                        ldb, C, ldc, bias, H);
   else
-    hipLaunchKernelGGL((k_sur_mm<TA, TB, EPI, false>), dim3(nblk(tiles, 4)), dim3(256), 0, st, M, N, K, A, lda, B,
+    hipLaunchKernelGGL((k_sur_mm<TB, EPI, false>), dim3(nblk(tiles, 4)), dim3(256), 0, st, M, N, K, A, lda, B,
                        ldb, C, ldc, bias, H);
 }
 
@@ -700,11 +762,11 @@ int forward(upc_sur* s, int net, const float* X, int B, const float* T, float* p
   const float* p = s->d_p + (long)net * kSurParams;
   float *Z1 = act(s, 0), *H1 = act(s, 1), *Z2 = act(s, 2), *H2 = act(s, 3), *Z3 = act(s, 4), *H3 = act(s, 5);
   const int tiles = (B / 16) * (kSurH / 16);
-  mm<false, true, kEpiBiasSilu>(s, tiles, st, B, kSurH, kSurIn,
+  mm<true, kEpiBiasSilu>(s, tiles, st, B, kSurH, kSurIn,
                      X, kSurIn, p + kOffW1, kSurIn, Z1, kSurH, p + kOffB1, H1);
-  mm<false, true, kEpiBiasSilu>(s, tiles, st, B, kSurH, kSurH,
+  mm<true, kEpiBiasSilu>(s, tiles, st, B, kSurH, kSurH,
                      H1, kSurH, p + kOffW2, kSurH, Z2, kSurH, p + kOffB2, H2);
-  mm<false, true, kEpiBiasSilu>(s, tiles, st, B, kSurH, kSurH,
+  mm<true, kEpiBiasSilu>(s, tiles, st, B, kSurH, kSurH,
                      H2, kSurH, p + kOffW3, kSurH, Z3, kSurH, p + kOffB3, H3);
   if (s->split)
     hipLaunchKernelGGL(k_sur_out<true>, dim3(nblk(B, 4)), dim3(256), 0, st, B, H3, p, T, pred, s->d_gout, loss,
@@ -720,39 +782,32 @@ int forward(upc_sur* s, int net, const float* X, int B, const float* T, float* p
 int backward(upc_sur* s, int net, const float* X, int B, hipStream_t st)
 {
   const float* p = s->d_p + (long)net * kSurParams;
-  float* g = s->d_g;
   float *Z1 = act(s, 0), *H1 = act(s, 1), *Z2 = act(s, 2), *H2 = act(s, 3), *Z3 = act(s, 4), *H3 = act(s, 5);
-  // reuse Z buffers' partners for dZ: dZ3 -> buffer 6? keep separate scratch after the activations
-  float* dA = s->d_act + 6L * kSurMaxBatch * kSurH;  // dZ / dH scratch, 2 buffers
+  float* dA = s->d_act + 6L * kSurMaxBatch * kSurH;  // dZ scratch, 2 buffers
   float* dB = dA + (long)kSurMaxBatch * kSurH;
-  const long n = (long)B * kSurH;
-  hipLaunchKernelGGL(k_sur_colsum, dim3(kSurH), dim3(256), 0, st, B, kSurH, H3, s->d_gout, g + kOffW4);
-  hipLaunchKernelGGL(k_sur_sum, dim3(1), dim3(256), 0, st, B, s->d_gout, g + kOffB4);
-  if (s->split)  // dZ3
-    hipLaunchKernelGGL(k_sur_out_bwd<true>, dim3(nblk(n, 256)), dim3(256), 0, st, B, s->d_gout, p, Z3, dA);
-  else
-    hipLaunchKernelGGL(k_sur_out_bwd<false>, dim3(nblk(n, 256)), dim3(256), 0, st, B, s->d_gout, p, Z3, dA);
-  // layer 3: dW3 = dZ3^T H2, db3, dH2 = dZ3 W3
-  const int tw = (kSurH / 16) * (kSurH / 16);
-  mm<true, false, kEpiStore>(s, tw, st, kSurH, kSurH, B, dA,
-                     kSurH, H2, kSurH, g + kOffW3, kSurH, (const float*)nullptr, (float*)nullptr);
-  hipLaunchKernelGGL(k_sur_colsum, dim3(kSurH), dim3(256), 0, st, B, kSurH, dA, (const float*)nullptr, g + kOffB3);
+  const int rows = ((B / 32 + kSurSlices - 1) / kSurSlices) * 32, slices = (B + rows - 1) / rows;
+  auto dw = [&](const float* dZ, const float* in, int n, int offw, int offb) {
+    const dim3 grid(slices, n / 32);
+    if (s->split)
+      hipLaunchKernelGGL(k_sur_dw<true>, grid, dim3(256), 0, st, B, rows, dZ, in, n, s->d_part, offw, offb);
+    else
+      hipLaunchKernelGGL(k_sur_dw<false>, grid, dim3(256), 0, st, B, rows, dZ, in, n, s->d_part, offw, offb);
+  };
   const int tb = (B / 16) * (kSurH / 16);
-  mm<false, false, kEpiStore>(s, tb, st, B, kSurH, kSurH, dA,
-                     kSurH, p + kOffW3, kSurH, dB, kSurH, (const float*)nullptr, (float*)nullptr);
-  hipLaunchKernelGGL(k_sur_silu_bwd, dim3(nblk(n, 256)), dim3(256), 0, st, n, Z2, dB);  // dZ2
-  // layer 2
-  mm<true, false, kEpiStore>(s, tw, st, kSurH, kSurH, B, dB,
-                     kSurH, H1, kSurH, g + kOffW2, kSurH, (const float*)nullptr, (float*)nullptr);
-  hipLaunchKernelGGL(k_sur_colsum, dim3(kSurH), dim3(256), 0, st, B, kSurH, dB, (const float*)nullptr, g + kOffB2);
-  mm<false, false, kEpiStore>(s, tb, st, B, kSurH, kSurH, dB,
-                     kSurH, p + kOffW2, kSurH, dA, kSurH, (const float*)nullptr, (float*)nullptr);
-  hipLaunchKernelGGL(k_sur_silu_bwd, dim3(nblk(n, 256)), dim3(256), 0, st, n, Z1, dA);  // dZ1
-  // layer 1: dW1 = dZ1^T X [128 x 32], db1
-  const int t1 = (kSurH / 16) * (kSurIn / 16);
-  mm<true, false, kEpiStore>(s, t1, st, kSurH, kSurIn, B, dA,
-                     kSurH, X, kSurIn, g + kOffW1, kSurIn, (const float*)nullptr, (float*)nullptr);
-  hipLaunchKernelGGL(k_sur_colsum, dim3(kSurH), dim3(256), 0, st, B, kSurH, dA, (const float*)nullptr, g + kOffB1);
+  // output layer and dZ3
+  if (s->split)
+    hipLaunchKernelGGL(k_sur_out_bwd<true>, dim3(slices), dim3(1024), 0, st, B, rows, s->d_gout, p, Z3, H3, dA,
+                       s->d_part);
+  else
+    hipLaunchKernelGGL(k_sur_out_bwd<false>, dim3(slices), dim3(1024), 0, st, B, rows, s->d_gout, p, Z3, H3, dA,
+                       s->d_part);
+  // layer 3: dW3 = dZ3^T H2, db3, dZ2 = dZ3 W3 silu'(Z2); layer 2; layer 1: dW1 = dZ1^T X, db1
+  dw(dA, H2, kSurH, kOffW3, kOffB3);
+  mm<false, kEpiSiluBwd>(s, tb, st, B, kSurH, kSurH, dA, kSurH, p + kOffW3, kSurH, dB, kSurH, nullptr, Z2);
+  dw(dB, H1, kSurH, kOffW2, kOffB2);
+  mm<false, kEpiSiluBwd>(s, tb, st, B, kSurH, kSurH, dB, kSurH, p + kOffW2, kSurH, dA, kSurH, nullptr, Z1);
+  dw(dA, X, kSurIn, kOffW1, kOffB1);
+  hipLaunchKernelGGL(k_sur_grad_sum, dim3(nblk(kSurParams, 256)), dim3(256), 0, st, slices, s->d_part, s->d_g);
   UPC_HIP(hipGetLastError());
   return 0;
 }
@@ -760,7 +815,7 @@ int backward(upc_sur* s, int net, const float* X, int B, hipStream_t st)
 void free_sur(upc_sur* s)
 {
   void* ptrs[] = {s->d_p, s->d_m, s->d_v, s->d_g, s->d_act, s->d_xb, s->d_tb, s->d_pred, s->d_gout, s->d_loss,
-                  s->d_step, s->d_img};
+                  s->d_step, s->d_img, s->d_part};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (s->cap_stream) (void)hipStreamDestroy(s->cap_stream);
@@ -934,6 +989,7 @@ int upc_sur_create(unsigned long long seed, upc_sur** out)
     UPC_HIP(hipMalloc(&s->d_m, sizeof(float) * kSurParams * kSurNets));
     UPC_HIP(hipMalloc(&s->d_v, sizeof(float) * kSurParams * kSurNets));
     UPC_HIP(hipMalloc(&s->d_g, sizeof(float) * kSurParams));
+    UPC_HIP(hipMalloc(&s->d_part, sizeof(float) * (size_t)kSurSlices * kSurParams));
     UPC_HIP(hipMalloc(&s->d_act, sizeof(float) * 8L * kSurMaxBatch * kSurH));
     UPC_HIP(hipMalloc(&s->d_xb, sizeof(float) * (long)kSurMaxBatch * kSurIn));
     UPC_HIP(hipMalloc(&s->d_img, sizeof(unsigned short) * kInferWords));
