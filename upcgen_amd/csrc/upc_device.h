@@ -80,7 +80,7 @@ __device__ __forceinline__ void clenshaw2(const double (&c)[N], const double (&d
 {
   double b1 = 0.0, b2 = 0.0, e1 = 0.0, e2 = 0.0;
   const double u2 = 2.0 * u;
-#pragma unroll 4
+#pragma unroll
   for (int k = N - 1; k >= 1; --k) {
     const double t = fma(u2, b1, c[k] - b2);
     b2 = b1;
@@ -97,7 +97,7 @@ template <int N>
 __device__ __forceinline__ double horner(const double (&c)[N], double y)
 {
   double s = c[N - 1];
-#pragma unroll 1
+#pragma unroll
   for (int k = N - 2; k >= 0; --k) s = c[k] + y * s;
   return s;
 }
