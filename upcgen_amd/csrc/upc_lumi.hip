@@ -27,7 +27,7 @@ namespace upc {
 // two exponentials per node, scaled square roots and interval clamps of 64 bits
 // at 96 VGPRs (now 68).
 // The pairs of a point are cut into kLumiParts runs that are summed apart and
-// then in order, so one wavefront and kLumiParts of them give the same bits.
+// then in order, so one wavefront, four and eight give the same bits.
 // ---------------------------------------------------------------------------
 constexpr int kLumiParts = 8;
 
@@ -156,7 +156,7 @@ struct LumiSmem {
 template <bool POL, int WAVES, int WPP>
 __device__ __forceinline__ void lumi_fp64_body(const LumiView& v, int p0, LumiSmem<WAVES, WPP>& sm)
 {
-  static_assert(WPP == 1 || (WPP == WAVES && WPP == kLumiParts), "a point takes one wavefront or the workgroup");
+  static_assert(WPP == 1 || (WPP == WAVES && kLumiParts % WPP == 0), "a point takes one wavefront or the workgroup");
   constexpr int kThreads = 64 * WPP;
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int sub = WPP > 1 ? wv : 0, tid = WPP > 1 ? threadIdx.x : lane;  // within the point's threads
@@ -407,27 +407,34 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(JR::
   else lumi_fp64_body<false, WAVES, WPP>(v, p0, sm);
 }
 
-// Work items of a launch up to which each takes a workgroup of kLumiParts
-// wavefronts: a point's pair list is one serial walk of up to 225 steps, and
-// few points wait for the longest; with many, the set-up that seven of the
-// eight wavefronts wait for costs more.  Pb-Pb points (modes 1 / 2 / 4
-// polarised), one wavefront against eight: 33 points 83 / 98 / 88 against 20 /
-// 24 / 23 us; 2,048: 109 / 187 / 154, 57 / 87 / 76; 8,192: 206 / 320 / 252,
-// 184 / 253 / 230; the 9,331 items of a 301 x 61 grid 181 / 268 / 213, 203 /
-// 289 / 272; 16,384 points 317 / 500 / 412, 340 / 487 / 438.
-constexpr int kLumiTeamPoints = 8192;
+// Work items of a launch up to which each takes a workgroup of 8, and of 4
+// wavefronts: a point's pair list is one serial walk of up to 225 steps, and few
+// points wait for the longest; with many, the set-up that the other wavefronts
+// wait for costs more.  Pb-Pb points (modes 1 / 2 / 4 polarised), us:
+//                     1 wavefront        4                 8
+//        33 points    83 /   98 /   88   32 /  37 /  32    20 /  24 /  23
+//     2,048          109 /  185 /  153   62 /  92 /  81    56 /  82 /  76
+//     4,096          135 /  206 /  168   98 / 138 / 116   100 / 138 / 129
+//     9,331 (grid)   181 /  265 /  212  171 / 243 / 204   195 / 289 / 272
+//    32,768          549 /  844 /  700  542 / 768 / 639   645 / 908 / 847
+//    61,061 (grid)   861 / 1381 / 1139  975 /1444 /1264  1156 /1735 /1612
+constexpr int kLumiTeam8 = 3072, kLumiTeam4 = 32768;
+
+template <int WAVES, int WPP>
+static void launch_lumi(const LumiView& v, int nwork, hipStream_t s)
+{
+  constexpr int kPoints = WAVES / WPP;
+  hipLaunchKernelGGL((k_lumi_fp64<WAVES, WPP, SingleLumi>), dim3((nwork + kPoints - 1) / kPoints), dim3(64 * WAVES), 0,
+                     s, SingleLumi{v});
+}
 
 int launch_lumi_fp64(const LumiView& v, hipStream_t s)
 {
-  constexpr int kWaves = 4;
   const int nwork = lumi_work_items(v.npts, v.fp.mirror_ny, v.mirror_out);
   if (nwork <= 0) return 0;
-  if (nwork <= kLumiTeamPoints)
-    hipLaunchKernelGGL((k_lumi_fp64<kLumiParts, kLumiParts, SingleLumi>), dim3(nwork), dim3(64 * kLumiParts), 0, s,
-                       SingleLumi{v});
-  else
-    hipLaunchKernelGGL((k_lumi_fp64<kWaves, 1, SingleLumi>), dim3((nwork + kWaves - 1) / kWaves), dim3(64 * kWaves), 0,
-                       s, SingleLumi{v});
+  if (nwork <= kLumiTeam8) launch_lumi<8, 8>(v, nwork, s);
+  else if (nwork <= kLumiTeam4) launch_lumi<4, 4>(v, nwork, s);
+  else launch_lumi<4, 1>(v, nwork, s);
   UPC_HIP(hipGetLastError());
   return 0;
 }
