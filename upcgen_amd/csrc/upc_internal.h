@@ -101,7 +101,7 @@ struct upc_ctx {
   double* d_ff_y = nullptr;         // 10^6 knot values
   double* d_ff_c = nullptr;         // 10^6 second-derivative coefficients
   double4* d_ff = nullptr;          // 10^6 - 1 intervals
-  double* d_j1 = nullptr;           // J1 on the shared b grid (k_flux_j1; form-factor flux only)
+  double* d_j1 = nullptr;           // behind d_ff_y: J1 on the shared b grid (k_flux_j1; form-factor flux only)
   double* d_bk_y = nullptr;         // kNBkUsed knot values
   double* d_bk_c = nullptr;
   double4* d_bk = nullptr;          // kNBkUsed - 1 intervals

@@ -531,7 +531,7 @@ int alloc_tables(upc_ctx* c)
   UPC_HIP(hipMalloc(&c->d_scalars, sizeof(DevScalars)));
   UPC_HIP(hipMalloc(&c->d_ta, sizeof(double4) * kNB));
   UPC_HIP(hipMalloc(&c->d_gaa, sizeof(double4) * kNB));
-  UPC_HIP(hipMalloc(&c->d_ff_y, sizeof(double) * kNQ2));
+  UPC_HIP(hipMalloc(&c->d_ff_y, sizeof(double) * (kNQ2 + (c->cfg.flux_point ? 0 : flux_j1_elems()))));
   UPC_HIP(hipMalloc(&c->d_ff_c, sizeof(double) * kNQ2));
   UPC_HIP(hipMalloc(&c->d_ff, sizeof(double4) * kNQ2));
   UPC_HIP(hipMalloc(&c->d_bk_y, sizeof(double) * kNBkUsed));
@@ -544,7 +544,7 @@ int alloc_tables(upc_ctx* c)
   c->bk_scratch_elems = (size_t)2 * (kSplineChunk + 2 * kSplineGuard) * nblk(kNBkUsed, kSplineChunk);
   UPC_HIP(hipMalloc(&c->d_bk_scratch, sizeof(double) * c->bk_scratch_elems));
   UPC_HIP(hipMalloc(&c->d_gaa_scratch, sizeof(double) * kNB));
-  if (!c->cfg.flux_point) UPC_HIP(hipMalloc(&c->d_j1, sizeof(double) * flux_j1_elems()));
+  if (!c->cfg.flux_point) c->d_j1 = c->d_ff_y + kNQ2;
   for (int i = 0; i < 2; ++i) {
     UPC_HIP(hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking));
     UPC_HIP(hipEventCreateWithFlags(&c->ev_join[i], hipEventDisableTiming));
@@ -565,7 +565,7 @@ void free_tables(upc_ctx* c)
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   void* ptrs[] = {c->d_scalars, c->d_ta, c->d_gaa, c->d_ff_y, c->d_ff_c, c->d_ff,
                   c->d_bk_y, c->d_bk_c, c->d_bk, c->d_ee, c->d_se, c->d_spline_scratch,
-                  c->d_bk_scratch, c->d_gaa_scratch, c->d_j1};
+                  c->d_bk_scratch, c->d_gaa_scratch};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
 }
