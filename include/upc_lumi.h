@@ -259,7 +259,7 @@ int upc_generate_pairs(upc_ctx *ctx, const double *d_sum_ym, const double *d_sum
  * reference processes compute in UpcCrossSection::init + prepareTwoPhotonLumi
  * (src/UpcCrossSection.cpp:116-137, 463-592), each job with its own system,
  * breakup mode, flux type, polarisation and grid.  The flux integrals of all
- * jobs share one persistent QAGS launch and the contraction is one launch;
+ * jobs share their QAGS launches and the contraction is one launch;
  * upc_batch_run(use_graph = 1) captures the sequence into a hipGraph on its
  * first call and replays it afterwards. */
 typedef struct upc_batch upc_batch;
