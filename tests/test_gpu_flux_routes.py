@@ -82,6 +82,23 @@ def test_shared_factors_evaluation_counts(gpu, data):
     assert total == whole
 
 
+@pytest.mark.parametrize("cap", [9, 8, 3, 1])
+def test_shared_factors_hand_integrals_on(gpu, data, cap):
+    """Integrals that outgrow the lists (or a smaller cap) go to the
+    1000-interval kernel: the same decisions and, to rounding, values."""
+    import torch
+    rng = np.random.default_rng(8)
+    t = lambda x: torch.as_tensor(x, device="cuda")
+    M, Y = t(np.exp(rng.uniform(np.log(2.0), np.log(60.0), 4100))), t(rng.uniform(-3.5, 3.5, 4100))
+    with gpu.Context(**CFG) as c:
+        L = c.lumi_points(M, Y).cpu().numpy()
+        evals = c.info.qags_evals
+        c.set_qags_cap(cap)
+        got = c.lumi_points(M, Y).cpu().numpy()
+        assert c.info.qags_evals == evals
+        assert np.max(np.abs(got - L) / np.abs(L)) <= 1e-11
+
+
 def test_points_against_oracle(data, oracle_ctx):
     _, M, Y, L, _ = data
     o = oracle_ctx(**CFG)
