@@ -1051,6 +1051,8 @@ void k_flux_qags_table(RS rs, long long g0,
       }
       const double b0 = wave_uniform(0.5 * (blo + bhi));
       const double db = (b - b0) * (1.0 / kHc), dbm = wave_uniform(fmax(b0 - blo, bhi - b0) * (1.0 / kHc));
+      // a row without a photon energy (M = 0) has no b: its values are NaN, not its neighbours' J1
+      const bool nob = __ballot(live && b != b) != 0;
       live = live && rs.need(r);
       // every row on the shared b grid: J1 from its table
       const bool shared = __ballot(live && rs.row_logd[r] != P.j1[0]) == 0;
@@ -1068,7 +1070,7 @@ void k_flux_qags_table(RS rs, long long g0,
           const double w = __hiloint2double(0x40240000 - ((int)L << 20), 0);
           const double lo = wave_uniform((double)im * w), mid = wave_uniform(lo + 0.5 * w), hi = wave_uniform(lo + w);
           const int slot = np == 1 ? h_slot(L, im) : h_slot(L + 1, 2 * im);
-          const int kind = shared ? 0 : expand_kind(hi * dbm, mymax);
+          const int kind = shared ? 0 : (nob ? kExpandKinds : expand_kind(hi * dbm, mymax));
           const bool mine = (rem >> lane & 1) != 0;
           if (slot < 0 || kind == kExpandKinds || turn == kRowsTurns) {
             if (mine) {
