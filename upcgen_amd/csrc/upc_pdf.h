@@ -11,7 +11,7 @@ template <class T>
 __device__ __forceinline__ T pdf_search(const double* __restrict__ sum, T lo, T hi, double r)
 {
   while (hi - lo > 1) {
-    const T mid = (lo + hi) >> 1;
+    const T mid = lo + ((hi - lo) >> 1);  // n may be up to the type's largest value
     if (r >= sum[mid]) lo = mid;
     else hi = mid;
   }
