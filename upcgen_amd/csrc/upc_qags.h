@@ -91,15 +91,16 @@ struct QagsSmallStore {
 // memory answers in about 700 cycles, LDS in 100.
 template <int CAP>
 struct QagsLdsStore : QagsSmallStore<CAP> {
-  static constexpr int kLists = 8, kLdsEps = 13;
+  static constexpr int kLists = CAP < 8 ? CAP : 8, kLdsEps = 13;
   static constexpr int kEps = kLdsEps + 1;  // 1-based
   struct Columns {                          // per wavefront
     double rl[kLists][64], el[kLists][64], eps[kLdsEps][64];
     unsigned iv[kLists][64];
   };
+  static constexpr int kMore = CAP > kLists ? CAP - kLists : 1;
   struct Arrays {
-    unsigned iv[CAP - kLists];
-    double rl[CAP - kLists], el[CAP - kLists];
+    unsigned iv[kMore];
+    double rl[kMore], el[kMore];
   };
   using Iv = unsigned;
   using LdsD = __attribute__((address_space(3))) double;
