@@ -1,0 +1,218 @@
+// The library's host side on a stand-in for the HIP runtime: a device of a given
+// memory whose kernels are recorded and not run.  For what only a full device
+// shows: which kernels a call launches when an allocation fails.
+//   host_paths <case>, exit code 0 and "ok" when the case holds.
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "upc_lumi.h"
+
+namespace {
+
+size_t capacity = ~size_t(0), live = 0;  // bytes of the device
+bool pool_fails = false;                 // hipMallocAsync finds no memory
+hipError_t last_error = hipSuccess;
+std::map<void*, size_t> blocks;
+std::vector<std::string> launches;
+std::map<const void*, std::string>& kernels()  // the library registers its own before main's statics
+{
+  static std::map<const void*, std::string> k;
+  return k;
+}
+
+hipError_t fail(hipError_t e) { return last_error = e; }
+
+hipError_t take(void** p, size_t n)
+{
+  *p = nullptr;
+  if (n > capacity - live) return fail(hipErrorOutOfMemory);
+  *p = calloc(1, n ? n : 1);
+  blocks[*p] = n;
+  live += n;
+  return hipSuccess;
+}
+
+hipError_t give(void* p)
+{
+  const auto it = blocks.find(p);
+  if (it == blocks.end()) return p ? fail(hipErrorInvalidValue) : hipSuccess;
+  live -= it->second;
+  blocks.erase(it);
+  free(p);
+  return hipSuccess;
+}
+
+struct CallConfig {
+  dim3 grid, block;
+  size_t shmem;
+  hipStream_t stream;
+} config;
+
+}  // namespace
+
+extern "C" {
+
+void** __hipRegisterFatBinary(const void*)
+{
+  static void* module = nullptr;
+  return &module;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*, int*)
+{
+  kernels()[host] = name;
+}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t shmem, hipStream_t stream)
+{
+  config = {grid, block, shmem, stream};
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hipStream_t* stream)
+{
+  *grid = config.grid, *block = config.block, *shmem = config.shmem, *stream = config.stream;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, hipStream_t)
+{
+  launches.push_back(kernels()[f]);
+  return hipSuccess;
+}
+
+hipError_t hipMalloc(void** p, size_t n) { return take(p, n); }
+hipError_t hipFree(void* p) { return give(p); }
+hipError_t hipMallocAsync(void** p, size_t n, hipStream_t)
+{
+  return pool_fails ? (*p = nullptr, fail(hipErrorOutOfMemory)) : take(p, n);
+}
+hipError_t hipFreeAsync(void* p, hipStream_t) { return give(p); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned)
+{
+  *p = calloc(1, n);
+  return hipSuccess;
+}
+hipError_t hipHostFree(void* p)
+{
+  free(p);
+  return hipSuccess;
+}
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind)
+{
+  memcpy(d, s, n);
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
+hipError_t hipMemset(void* d, int v, size_t n)
+{
+  memset(d, v, n);
+  return hipSuccess;
+}
+hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t) { return hipMemset(d, v, n); }
+
+hipError_t hipGetLastError()
+{
+  const hipError_t e = last_error;
+  last_error = hipSuccess;
+  return e;
+}
+const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = nullptr, hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s)
+{
+  return *s = hipStreamCaptureStatusNone, hipSuccess;
+}
+hipError_t hipEventCreate(hipEvent_t* e) { return *e = nullptr, hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return *e = nullptr, hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 0.f, hipSuccess; }
+
+}  // extern "C"
+
+namespace {
+
+#define CHECK(cond)                                                                          \
+  do {                                                                                       \
+    if (!(cond)) {                                                                           \
+      printf("line %d: %s\nlast error: %s\nlaunches:", __LINE__, #cond, upc_last_error());   \
+      for (const std::string& l : launches) printf(" %s", l.c_str());                        \
+      printf("\n");                                                                          \
+      exit(1);                                                                               \
+    }                                                                                        \
+  } while (0)
+
+int launched(const char* name)
+{
+  int n = 0;
+  for (const std::string& l : launches) n += l.find(name) != std::string::npos;
+  return n;
+}
+
+upc_config config_of(int flux_point, int nm, int ny, int nz)
+{
+  upc_config c{};
+  c.Z = 82, c.A = 208, c.R = 6.68, c.a = 0.447, c.sqrts = 5020.0;
+  c.flux_point = flux_point, c.breakup_mode = 2;
+  c.nm = nm, c.mmin = 3.5, c.mmax = 50.0;
+  c.ny = ny, c.ymin = -6.0, c.ymax = 6.0;
+  c.nz = nz, c.zmin = -1.0, c.zmax = 1.0;
+  c.proc_id = 13;
+  return c;
+}
+
+upc_ctx* context(const upc_config& c)
+{
+  upc_ctx* ctx = nullptr;
+  CHECK(upc_ctx_create(&c, nullptr, &ctx) == 0);
+  launches.clear();
+  return ctx;
+}
+
+double cell[1];  // stands for every array that only kernels touch
+
+// Draws: guides to the tables where a call makes many; without memory for them
+// the plain search, which needs none.
+void draws(bool pairs, bool full)
+{
+  upc_ctx* ctx = context(config_of(1, 101, 41, 50));
+  pool_fails = full;
+  const upc_event_opts opts{};
+  const long long n = 1 << 20;
+  int out[1];
+  const int rc = pairs ? upc_generate_pairs(ctx, cell, cell, nullptr, nullptr, nullptr, &opts, 1, 0, n, cell, out, out, nullptr)
+                       : upc_sample_events(ctx, cell, cell, nullptr, nullptr, nullptr, 1, 0, n, cell, cell, cell, nullptr);
+  CHECK(rc == 0);
+  CHECK(launched("k_pdf_guides") == (full ? 0 : 1));
+  CHECK(launched(pairs ? "k_generate_pairs" : "k_sample_events") == 1);
+  CHECK(hipGetLastError() == hipSuccess);
+  upc_ctx_destroy(ctx);
+  CHECK(live == 0);
+}
+
+}  // namespace
+
+int main(int argc, char** argv)
+{
+  const std::string what = argc > 1 ? argv[1] : "";
+  if (what == "draws") draws(false, false);
+  else if (what == "draws_full") draws(false, true);
+  else if (what == "pairs") draws(true, false);
+  else if (what == "pairs_full") draws(true, true);
+  else return printf("no case %s\n", what.c_str()), 2;
+  printf("ok\n");
+  return 0;
+}

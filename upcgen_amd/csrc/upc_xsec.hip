@@ -379,7 +379,7 @@ static int guide_bits(int n, int most)
 // x 121 grid with 100 z bins, searched against guided: 524,288 draws 34 against
 // 43 us, 1,048,576 61, 42; 4,194,304 222, 86.  Not while the stream is captured
 // (the guides' memory belongs to the call), nor where a z bin does not fit 16
-// bits.
+// bits or there is no memory for them.
 constexpr int kGuideDraws = 3;
 
 int PdfGuides::build(const double* sum_ym, const double* sum_z, const double* sum_zp, int nym, int nz, int nm,
@@ -389,9 +389,16 @@ int PdfGuides::build(const double* sum_ym, const double* sum_z, const double* su
   const long long ycell = (1 << ybits) + 1, zcell = (long long)((1 << zbits) + 1) * nm * (sum_zp ? 2 : 1);
   if (nz > 0xffff || n / kGuideDraws < ycell + zcell) return 0;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  UPC_HIP(hipStreamIsCapturing(s, &cap));
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
   if (cap != hipStreamCaptureStatusNone) return 0;
-  UPC_HIP(hipMallocAsync(&buf, sizeof(int) * ycell + sizeof(unsigned short) * zcell, s));
+  if (hipMallocAsync(&buf, sizeof(int) * ycell + sizeof(unsigned short) * zcell, s) != hipSuccess) {
+    (void)hipGetLastError();  // the search without guides is no error of the call
+    buf = nullptr;
+    return 0;
+  }
   stream = s;
   int* y = (int*)buf;
   unsigned short* zc = (unsigned short*)(y + ycell);
