@@ -4,6 +4,7 @@
 //   host_paths <case>, exit code 0 and "ok" when the case holds.
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -183,6 +184,7 @@ upc_ctx* context(const upc_config& c)
 }
 
 double cell[1];  // stands for every array that only kernels touch
+double cells[5000];  // and that the host copies
 
 // Draws: guides to the tables where a call makes many; without memory for them
 // the plain search, which needs none.
@@ -203,6 +205,59 @@ void draws(bool pairs, bool full)
   CHECK(live == 0);
 }
 
+size_t largest_block()
+{
+  size_t n = 0;
+  for (const auto& b : blocks) n = std::max(n, b.second);
+  return n;
+}
+
+// Whole form-factor grids on a device with `left` bytes beside the context's
+// tables: the integrand factors take what is there, and where they do not fit,
+// the kernel that needs none.
+constexpr int kBig[2] = {1024, 200};  // 205,824 flux rows, 3,216 groups of 64: 864 MB of factors
+constexpr size_t kRows = 371000000;    // flux rows, points and the list of integrals handed on
+
+void grid(size_t left, int table_launches, int direct_launches)
+{
+  upc_ctx* ctx = context(config_of(0, kBig[0], kBig[1], 50));
+  if (left) capacity = live + left;
+  CHECK(upc_lumi_grid(ctx, UPC_FORM_FP64, cell, nullptr, nullptr, nullptr) == 0);
+  CHECK(launched("k_flux_h") == table_launches && launched("k_flux_qags_table") == table_launches);
+  CHECK(launched("k_flux_qags_rows") == direct_launches);
+  CHECK(launched("k_flux_qags_wave") == 1 && launched("k_lumi_fp64") == 1);
+  CHECK(hipGetLastError() == hipSuccess);
+  // again, and a smaller call, in the buffers that are there
+  const size_t held = live;
+  CHECK(upc_lumi_grid(ctx, UPC_FORM_FP64, cell, nullptr, nullptr, nullptr) == 0);
+  CHECK(upc_lumi_points(ctx, cells, cells, 5000, cells, nullptr, nullptr, nullptr) == 0);
+  CHECK(live == held);
+  upc_ctx_destroy(ctx);
+  CHECK(live == 0);
+}
+
+void batch(size_t left, int table_launches, int direct_launches)
+{
+  const upc_config jobs[2] = {config_of(0, kBig[0], kBig[1], 50), config_of(0, 21, 11, 50)};  // the second: no factors
+  upc_batch* b = nullptr;
+  CHECK(upc_batch_create(jobs, 2, nullptr, &b) == 0);
+  const size_t held = live - largest_block();  // everything but the factors
+  CHECK(upc_batch_destroy(b) == 0);
+  CHECK(live == 0);
+  if (left) capacity = held + left;
+  CHECK(upc_batch_create(jobs, 2, nullptr, &b) == 0);
+  double* L[2] = {cell, cell};
+  CHECK(upc_batch_set_outputs(b, L, nullptr, nullptr) == 0);
+  launches.clear();
+  CHECK(upc_batch_run(b, 0, nullptr) == 0);
+  CHECK(launched("k_flux_h") == table_launches && launched("k_flux_qags_table") == table_launches);
+  CHECK(launched("k_flux_qags_rows") == direct_launches);
+  CHECK(launched("k_flux_qags_wave") == 1 && launched("k_lumi_fp64") == 1);
+  CHECK(hipGetLastError() == hipSuccess);
+  CHECK(upc_batch_destroy(b) == 0);
+  CHECK(live == 0);
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -212,6 +267,12 @@ int main(int argc, char** argv)
   else if (what == "draws_full") draws(false, true);
   else if (what == "pairs") draws(true, false);
   else if (what == "pairs_full") draws(true, true);
+  else if (what == "grid") grid(0, 1, 0);
+  else if (what == "grid_short") grid(kRows + 450000000, 2, 0);  // half of the factors
+  else if (what == "grid_full") grid(kRows + 30000000, 0, 1);
+  else if (what == "batch") batch(0, 1, 1);
+  else if (what == "batch_short") batch(240000000, 4, 1);  // a quarter
+  else if (what == "batch_full") batch(30000000, 0, 1);
   else return printf("no case %s\n", what.c_str()), 2;
   printf("ok\n");
   return 0;

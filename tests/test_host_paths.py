@@ -21,7 +21,8 @@ def host_paths(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["draws", "draws_full", "pairs", "pairs_full"])
+@pytest.mark.parametrize("case", ["draws", "draws_full", "pairs", "pairs_full",
+                                  "grid", "grid_short", "grid_full", "batch", "batch_short", "batch_full"])
 def test_host_path(host_paths, case):
     r = subprocess.run([host_paths, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -137,7 +137,8 @@ struct upc_batch {
   long long ntasks = 0;          // QAGS integrals of every job (counted at creation)
   long long work_bytes = 0;      // device memory of the buffers below
   long long* d_overflow = nullptr;
-  double* d_h = nullptr;         // integrand factors of one launch's groups of rows
+  double* d_h = nullptr;         // integrand factors of h_groups groups of rows
+  int h_groups = 0;
   int ncursors = 0;
   // [0] evals [1] bad [2] overflow n [4] tasks, [8..] work cursors of the row QAGS launches
   unsigned long long* d_counters = nullptr;
@@ -216,10 +217,10 @@ BatchRows batch_rows(const upc_batch* b, long long g0, long long g1)
 void launch_qags(upc_batch* b, int choice, hipStream_t s)
 {
   unsigned long long* cursors = b->d_counters + 8;
-  const long long m = b->share_groups;
-  launch_qags_rows(true, batch_rows(b, 0, m), m, b->d_h, cursors, b->d_flux, b->d_counters, b->d_overflow, kQagsCap,
-                   b->ncu, kQagsBlockChoices[choice], s);
-  launch_qags_rows(false, batch_rows(b, m, b->groups), b->groups - m, nullptr, cursors + rows_cursors(m), b->d_flux,
+  const long long m = b->h_groups > 0 ? b->share_groups : 0;
+  launch_qags_rows(b->h_groups, batch_rows(b, 0, m), m, b->d_h, cursors, b->d_flux, b->d_counters, b->d_overflow,
+                   kQagsCap, b->ncu, kQagsBlockChoices[choice], s);
+  launch_qags_rows(0, batch_rows(b, m, b->groups), b->groups - m, nullptr, cursors + b->ncursors - kXcds, b->d_flux,
                    b->d_counters, b->d_overflow, kQagsCap, b->ncu, kQagsBlockChoices[choice], s);
 }
 
@@ -239,7 +240,7 @@ int enqueue(upc_batch* b, hipStream_t s)
   hipLaunchKernelGGL((k_row_offsets<BatchRows, int>), dim3(nj), dim3(1024), 0, s, rs, b->d_hist, b->d_nsorted);
   hipLaunchKernelGGL(k_batch_point_rows, dim3(nblk(b->nrows * kNB1, 256)), dim3(256), 0, s, b->d_jobs, b->d_row0,
                      nj, b->nrows, b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_flux, b->d_hist, b->d_perm);
-  if (b->share_groups > 0)
+  if (b->h_groups > 0)
     hipLaunchKernelGGL(k_row_order<BatchRows>, dim3(nblk(nhist, 4)), dim3(256), 0, s, rs, b->d_hist, (long long)nhist);
   launch_qags(b, b->qags_choice, s);
   launch_qags_wave(b, s);
@@ -305,7 +306,7 @@ int upc_batch_create(const upc_config* cfgs, int njobs, void* stream, upc_batch*
     if (share) b->share_groups = (long long)group_job.size();
   }
   b->groups = (long long)group_job.size();
-  b->ncursors = (int)(rows_cursors(b->share_groups) + kXcds);
+  b->ncursors = (int)rows_cursors(b->share_groups);
   for (int i = 0; i < 3; ++i) b->lumi_blocks[i] = (int)blocks[i];
 #define BA(ptr, n)                                                  \
   do {                                                              \
@@ -393,9 +394,8 @@ int upc_batch_create(const upc_config* cfgs, int njobs, void* stream, upc_batch*
     UPC_HIP(hipMalloc(&b->d_overflow, sizeof(long long) * n));
     b->work_bytes += (long long)(sizeof(long long) * n);
     if (b->share_groups > 0) {
-      const size_t h = sizeof(double) * rows_h_elems(b->share_groups);
-      UPC_HIP(hipMalloc(&b->d_h, h));
-      b->work_bytes += (long long)h;
+      b->h_groups = alloc_factors(&b->d_h, b->share_groups);
+      b->work_bytes += (long long)(sizeof(double) * kHGroupElems) * b->h_groups;
     }
     return 0;
   };

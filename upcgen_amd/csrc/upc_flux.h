@@ -705,8 +705,8 @@ __device__ __forceinline__ QK21Out qk21_rows(double* fv, double qa, double qb, c
 // 9.8 ms (182 VGPRs spilled); coefficients broadcast from LDS to every lane
 // 4.9 ms (LDS 38 % busy).
 //
-// Work ids are (group of 64 rows, j).  A launch takes up to kRowsChunk groups
-// from g0 on (H bounds it: 269 KB per group).  The j of a group share its h, so
+// Work ids are (group of 64 rows, j).  A launch takes `chunk` groups from g0 on,
+// as many as H holds (269 KB each).  The j of a group share its h, so
 // a group belongs to one XCD's cursor (workgroups are dealt to the XCDs in
 // turn): the few groups in flight on an XCD stay in its L2.
 // ---------------------------------------------------------------------------
@@ -721,6 +721,7 @@ constexpr int kRowsTurns = 4;     // intervals a step takes one by one before it
 // the form factor falls off, so dqagse bisects towards q = 0: these 25
 // intervals take 99 % of the passes (Pb 5.02 TeV, O 7 TeV, Au 200 GeV grids).
 constexpr int kHLevels = 10, kHSlots = 25;
+constexpr int kHGroupElems = kHSlots * 21 * 64;  // of one group of rows
 __device__ constexpr int kHCount[kHLevels] = {1, 2, 2, 2, 2, 4, 6, 2, 2, 2};
 __device__ constexpr int kHFirst[kHLevels] = {0, 1, 3, 5, 7, 9, 13, 19, 21, 23};
 
@@ -993,7 +994,7 @@ __device__ __forceinline__ QK21Out qk21_values(const double* f, double hlgth)
 
 template <int CAP, class RS>
 __global__ __launch_bounds__(kQagsBlock) __attribute__((amdgpu_waves_per_eu(kQagsTableWaves, kQagsTableWaves)))
-void k_flux_qags_table(RS rs, long long g0,
+void k_flux_qags_table(RS rs, long long g0, int chunk,
                       const double* __restrict__ H, unsigned long long* __restrict__ cursors,
                       double* __restrict__ flux, unsigned long long* __restrict__ stats,
                       long long* __restrict__ overflow, int fast_cap)
@@ -1011,7 +1012,7 @@ void k_flux_qags_table(RS rs, long long g0,
   q.s.bind(&lds[threadIdx.x >> 6].lists, lane, &lists);
   q.s.lim = fast_cap < CAP ? fast_cap : CAP;
   // groups of this launch, and those of cursor x: g0 + x, g0 + x + kXcds, ...
-  const long long left = rs.groups() - g0, ngroups = left < kRowsChunk ? left : kRowsChunk;
+  const long long left = rs.groups() - g0, ngroups = left < chunk ? left : chunk;
   unsigned my_evals = 0, my_bad = 0;  // 32-bit per lane; evaluations flushed before they could wrap
   const double mymax = lane < kExpandKinds ? kExpandMax[lane < kExpandKinds ? lane : 0] : __builtin_inf();
   int x = blockIdx.x % kXcds, tried = 0;
@@ -1028,7 +1029,7 @@ void k_flux_qags_table(RS rs, long long g0,
       continue;
     }
     if (lane == 0) next = (unsigned)atomicAdd(&cursors[x], 1ull);
-    const double* hg = H + (long long)gl * (kHSlots * 21 * 64);
+    const double* hg = H + (long long)gl * kHGroupElems;
     long long first;
     int r = 0, job = 0;
     bool live = false;
@@ -1448,15 +1449,32 @@ __global__ __launch_bounds__(256) void k_row_order(RS rs, const int* __restrict_
 // batch takes the route of its own context.
 constexpr long long kQagsShareRows = 8192;
 
-// Launches over at most `groups` groups of rows, share: of k_flux_qags_table,
-// kRowsChunk of them at a time, else of k_flux_qags_rows.  cursors:
-// rows_cursors(groups) cleared counters; H: rows_h_elems(groups) (share only);
-// per_cu: workgroups per CU, at most 3.
+// The factor table H of a launch sequence over at most `groups` groups of rows:
+// the groups it holds, kRowsChunk at most, fewer where memory is short, 0 (and
+// no table) where kRowsChunkMin do not fit.  The end of a launch leaves the chip
+// half idle for 0.3 ms: whole grids of 1001 x 121, 2001 x 241 bins and a 16-job
+// batch take 6.1, 21.8 and 64.4 ms with 4,096 groups, 6.1, 22.5 and 65.6 with
+// 2,048, 6.4, 23.6 and 68.4 with 1,024.
 inline long long rows_groups(long long rows) { return (rows + 63) / 64; }
-inline size_t rows_cursors(long long groups) { return (size_t)((groups + kRowsChunk - 1) / kRowsChunk) * kXcds; }
-inline size_t rows_h_elems(long long groups)
+constexpr int kRowsChunkMin = (int)(kQagsShareRows / 64);  // 34 MB
+
+inline int alloc_factors(double** H, long long groups)
 {
-  return (size_t)(groups < kRowsChunk ? groups : kRowsChunk) * (kHSlots * 21 * 64);
+  *H = nullptr;
+  for (int n = (int)std::min<long long>(groups, kRowsChunk); n > 0;) {
+    if (hipMalloc(H, sizeof(double) * (size_t)n * kHGroupElems) == hipSuccess) return n;
+    (void)hipGetLastError();  // k_flux_qags_rows needs no table
+    *H = nullptr;
+    n = n > kRowsChunkMin ? std::max(n / 2, kRowsChunkMin) : 0;
+  }
+  return 0;
+}
+
+// Work cursors of that sequence, whatever the table holds, and of one launch of
+// k_flux_qags_rows after it.
+inline size_t rows_cursors(long long groups)
+{
+  return (size_t)((groups + kRowsChunkMin - 1) / kRowsChunkMin + 1) * kXcds;
 }
 
 // upc_flux_rows.hip
@@ -1464,18 +1482,23 @@ template <class RS>
 void launch_qags_rows_direct(const RS& rs, unsigned long long* cursor, double* flux, unsigned long long* stats,
                              long long* overflow, int cap, int blocks, hipStream_t s);
 
+// Launches over at most `groups` groups of rows: of k_flux_qags_table, `chunk` of
+// them at a time (what H holds), or with chunk 0 of k_flux_qags_rows.  cursors:
+// cleared, kXcds per launch; per_cu: workgroups per CU, at most 3.
 template <class RS>
-inline void launch_qags_rows(bool share, const RS& rs, long long groups, double* H, unsigned long long* cursors,
+inline void launch_qags_rows(int chunk, const RS& rs, long long groups, double* H, unsigned long long* cursors,
                              double* flux, unsigned long long* stats, long long* overflow, int cap, int ncu,
                              int per_cu, hipStream_t s)
 {
   if (groups <= 0) return;
-  if (!share) return launch_qags_rows_direct(rs, cursors, flux, stats, overflow, cap, ncu * per_cu, s);
-  for (long long g0 = 0; g0 < groups; g0 += kRowsChunk, cursors += kXcds) {
-    const long long n = groups - g0 < kRowsChunk ? groups - g0 : kRowsChunk;
+  if (!chunk) return launch_qags_rows_direct(rs, cursors, flux, stats, overflow, cap, ncu * per_cu, s);
+  const long long launches = (groups + chunk - 1) / chunk;
+  chunk = (int)((groups + launches - 1) / launches);  // all of one size
+  for (long long g0 = 0; g0 < groups; g0 += chunk, cursors += kXcds) {
+    const long long n = groups - g0 < chunk ? groups - g0 : chunk;
     hipLaunchKernelGGL(k_flux_h<RS>, dim3((unsigned)(n * kHSlots)), dim3(256), 0, s, rs, g0, H);
     hipLaunchKernelGGL((k_flux_qags_table<kQagsCap, RS>), dim3(ncu * std::min(per_cu, kQagsTableBlocksPerCu)),
-                       dim3(kQagsBlock), 0, s, rs, g0, H, cursors, flux, stats, overflow, cap);
+                       dim3(kQagsBlock), 0, s, rs, g0, chunk, H, cursors, flux, stats, overflow, cap);
   }
 }
 

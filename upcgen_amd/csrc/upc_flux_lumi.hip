@@ -187,14 +187,14 @@ static int ensure_work(upc_ctx* c, size_t npts, size_t rows, size_t points_ff = 
   UPC_HIP(hipMalloc(&w.d_flux, sizeof(double) * rows * kNB1));
   UPC_HIP(hipMalloc(&w.d_idx, sizeof(int) * nidx));
   UPC_HIP(hipMalloc(&w.d_overflow, sizeof(long long) * nover));
-  const size_t ncur = rows_cursors(rows_groups(rows)) + kXcds;  // and one launch of a restricted grid's
+  const size_t ncur = rows_cursors(rows_groups(rows));
   UPC_HIP(hipMalloc(&w.d_counters, sizeof(unsigned long long) * (8 + ncur) + sizeof(int) * kRowBuckets));
   w.d_hist = (int*)(w.d_counters + 8);
   w.d_cursors = (unsigned long long*)(w.d_hist + kRowBuckets);
   w.ncursors = ncur;
-  if (!c->cfg.flux_point && rows >= (size_t)kQagsShareRows)
-    UPC_HIP(hipMalloc(&w.d_h, sizeof(double) * rows_h_elems(rows_groups(rows))));
   UPC_HIP(hipMalloc(&w.d_points, sizeof(double) * 4 * npts));
+  if (!c->cfg.flux_point && rows >= (size_t)kQagsShareRows)
+    w.h_groups = alloc_factors(&w.d_h, rows_groups(rows));
   w.rows_cap = rows;
   w.over_cap = nover;
   w.idx_cap = nidx;
@@ -239,7 +239,7 @@ static int run_flux(upc_ctx* c, int npts, int mirror_ny, hipStream_t s, const un
   const int nrows = flux_rows(npts, mirror_ny);
   // a restricted grid has few rows of many: only the sort knows how many
   const int team = row_need ? 1 : qags_team((long long)nrows * kQagsNodesPerRow);
-  const bool sorted = !c->cfg.flux_point && team == 1, share = sorted && nrows >= kQagsShareRows;
+  const bool sorted = !c->cfg.flux_point && team == 1, share = sorted && nrows >= kQagsShareRows && w.h_groups > 0;
   const GridRows rs{w.d_row_k, w.d_row_logd, w.d_row_cnt, w.d_perm, w.d_counters + 6,
                     RowJob{c->d_ff, c->d_j1, fp.bmin, fp.g1, fp.factor, fp.A}, nrows,
                     share ? row_need : nullptr, share && row_need ? 1 : 0, w.d_counters + 7, w.d_counters + 6};
@@ -266,7 +266,7 @@ static int run_flux(upc_ctx* c, int npts, int mirror_ny, hipStream_t s, const un
       launch_qags_team(team, rs, (long long)nrows * kMaxQagsNodesPerRow, w.d_flux, nullptr, w.d_counters,
                        w.d_overflow, c->qags_cap, s);
     else
-      launch_qags_rows(share, rs, rows_groups(nrows), w.d_h, w.d_cursors, w.d_flux, w.d_counters, w.d_overflow,
+      launch_qags_rows(share ? w.h_groups : 0, rs, rows_groups(nrows), w.d_h, w.d_cursors, w.d_flux, w.d_counters, w.d_overflow,
                        c->qags_cap, cu_count(), kQagsRowsBlocksPerCu, s);
     if (share && row_need) {
       GridRows few = rs;
@@ -274,7 +274,7 @@ static int run_flux(upc_ctx* c, int npts, int mirror_ny, hipStream_t s, const un
       few.nsorted = few.npart;
       few.need_row = nullptr;
       few.pick = 2;
-      launch_qags_rows(false, few, rows_groups(nrows), nullptr, w.d_cursors + rows_cursors(rows_groups(nrows)), w.d_flux,
+      launch_qags_rows(0, few, rows_groups(nrows), nullptr, w.d_cursors + w.ncursors - kXcds, w.d_flux,
                        w.d_counters, w.d_overflow, c->qags_cap, cu_count(), kQagsRowsBlocksPerCu, s);
     }
     hipLaunchKernelGGL((k_flux_qags_wave<GridRows>), dim3(kQagsWaveBlocks), dim3(64), 0, s, rs, w.d_overflow,

@@ -58,7 +58,8 @@ struct LumiWork {
   int* d_hist = nullptr;          // [kRowBuckets] behind d_counters: rows per k bucket, then their offsets
   unsigned long long* d_cursors = nullptr;  // behind d_hist: work cursors of the row QAGS launches
   size_t ncursors = 0;
-  double* d_h = nullptr;          // integrand factors of up to kRowsChunk groups of 64 rows
+  double* d_h = nullptr;          // integrand factors of h_groups groups of 64 rows
+  int h_groups = 0;
   long long* d_overflow = nullptr;  // tasks that exceeded the fast workspace
   double* d_points = nullptr;     // (M, Y, dm, dy) per point
   size_t points_cap = 0;
