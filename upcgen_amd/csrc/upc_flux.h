@@ -781,10 +781,15 @@ using ConstD = const __attribute__((address_space(4))) double;
 // = 5 R) db is 0 and T = 1.
 //
 // With delta = q db, T terms leave |delta|^T / T!; kExpandMax[i] is the delta
-// up to which this is below 1.5e-19, i.e. below 1e-17 of J1 ~ x / 2 at the
+// up to which this is below 1.5e-19, i.e. 2e-17 of J1 ~ x / 2 at the
 // smallest x of an interval's end (0.015).  The recurrence's rounding enters
-// as (delta / x0)^n and stays below the rounding of J1(x0): measured within
-// 4.9e-16 of the envelope (J1's own 4.2e-16) for delta / x0 up to 0.2.
+// as (delta / x0)^n and stays below the rounding of J1(x0) for delta / x0 = db /
+// (b0 / hc) up to kExpandRatio: with the kernel's J1 (itself 4.2e-16) within
+// 4.9e-16 of the envelope there; with exact J0 and J1(x0) 2.0e-16, and 4.8e-16 at
+// 0.5, 2.6e-15 at 0.8, 2.8e-13 at 0.99.  A group of rows further apart evaluates
+// its own nodes: none on grids or points spread evenly (0.04 on 1001 x 121, 0.18
+// at most from 8,192 rows on), but a dense cluster of points beside distant ones.
+constexpr double kExpandRatio = 0.2;
 constexpr int kExpandKinds = 7;
 __device__ constexpr int kExpandTerms[kExpandKinds] = {1, 4, 6, 8, 10, 14, 20};
 __device__ constexpr double kExpandMax[kExpandKinds] = {0.0, 4.3e-5, 2.1e-3, 1.6e-2, 5.9e-2, 0.265, 0.939};
@@ -1051,9 +1056,11 @@ void k_flux_qags_table(RS rs, long long g0, int chunk,
         bhi = fmax(bhi, __shfl_xor(bhi, o));
       }
       const double b0 = wave_uniform(0.5 * (blo + bhi));
-      const double db = (b - b0) * (1.0 / kHc), dbm = wave_uniform(fmax(b0 - blo, bhi - b0) * (1.0 / kHc));
-      // a row without a photon energy (M = 0) has no b: its values are NaN, not its neighbours' J1
-      const bool nob = __ballot(live && b != b) != 0;
+      // Rows too far apart for an expansion: none (infinitely far), and likewise where
+      // a row has no b (no photon energy, M = 0): its values are NaN, not its neighbours' J1.
+      const bool apart = __ballot(live && !(fabs(b - b0) <= kExpandRatio * b0)) != 0;
+      const double db = (b - b0) * (1.0 / kHc);
+      const double dbm = wave_uniform(apart ? __builtin_inf() : fmax(b0 - blo, bhi - b0) * (1.0 / kHc));
       live = live && rs.need(r);
       // every row on the shared b grid: J1 from its table
       const bool shared = __ballot(live && rs.row_logd[r] != P.j1[0]) == 0;
@@ -1071,7 +1078,7 @@ void k_flux_qags_table(RS rs, long long g0, int chunk,
           const double w = __hiloint2double(0x40240000 - ((int)L << 20), 0);
           const double lo = wave_uniform((double)im * w), mid = wave_uniform(lo + 0.5 * w), hi = wave_uniform(lo + w);
           const int slot = np == 1 ? h_slot(L, im) : h_slot(L + 1, 2 * im);
-          const int kind = shared ? 0 : (nob ? kExpandKinds : expand_kind(hi * dbm, mymax));
+          const int kind = shared ? 0 : expand_kind(hi * dbm, mymax);
           const bool mine = (rem >> lane & 1) != 0;
           if (slot < 0 || kind == kExpandKinds || turn == kRowsTurns) {
             if (mine) {
