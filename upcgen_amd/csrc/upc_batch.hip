@@ -515,6 +515,7 @@ int upc_batch_autotune(upc_batch* b, void* stream, upc_tune* h_out)
     // QAGS alone: clear the counters except the integral and row totals, then time
     hipLaunchKernelGGL(k_batch_zero, dim3(1), dim3(64), 0, s, b->d_counters, 4);
     hipLaunchKernelGGL(k_batch_zero, dim3(nblk(b->ncursors, 64)), dim3(64), 0, s, b->d_counters + 8, b->ncursors);
+    hipLaunchKernelGGL(k_batch_zero, dim3(nblk(nj, 64)), dim3(64), 0, s, b->d_job_failed, nj);
     UPC_HIP(hipEventRecord(e0, s));
     launch_qags(b, i, s);
     UPC_HIP(hipEventRecord(e1, s));
