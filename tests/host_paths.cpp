@@ -258,6 +258,25 @@ void batch(size_t left, int table_launches, int direct_launches)
   CHECK(live == 0);
 }
 
+// Tuning times the launch shapes that differ: three for the kernel without
+// factors, two for the one with them (two workgroups fill a CU).
+void tune(int njobs, int table_launches, int direct_launches)
+{
+  const upc_config jobs[2] = {config_of(0, kBig[0], kBig[1], 50), config_of(0, 21, 11, 50)};
+  upc_batch* b = nullptr;
+  CHECK(upc_batch_create(jobs, njobs, nullptr, &b) == 0);
+  double* L[2] = {cell, cell};
+  CHECK(upc_batch_set_outputs(b, L, nullptr, nullptr) == 0);
+  launches.clear();
+  upc_tune t;
+  CHECK(upc_batch_autotune(b, nullptr, &t) == 0);
+  CHECK(launched("k_flux_qags_table") == 1 + table_launches);  // and once before the timed passes
+  CHECK(launched("k_flux_qags_rows") == direct_launches);
+  CHECK(t.qags_candidates[2] == 3 && t.qags_blocks_per_cu >= 1);
+  CHECK(njobs > 1 || (t.qags_ms[2] == t.qags_ms[1] && t.qags_blocks_per_cu < 3));
+  CHECK(upc_batch_destroy(b) == 0);
+}
+
 }  // namespace
 
 int main(int argc, char** argv)
@@ -273,6 +292,8 @@ int main(int argc, char** argv)
   else if (what == "batch") batch(0, 1, 1);
   else if (what == "batch_short") batch(240000000, 4, 1);  // a quarter
   else if (what == "batch_full") batch(30000000, 0, 1);
+  else if (what == "tune_shared") tune(1, 2, 0);
+  else if (what == "tune_mixed") tune(2, 3, 4);
   else return printf("no case %s\n", what.c_str()), 2;
   printf("ok\n");
   return 0;

@@ -22,7 +22,8 @@ def host_paths(tmp_path_factory):
 
 
 @pytest.mark.parametrize("case", ["draws", "draws_full", "pairs", "pairs_full",
-                                  "grid", "grid_short", "grid_full", "batch", "batch_short", "batch_full"])
+                                  "grid", "grid_short", "grid_full", "batch", "batch_short", "batch_full",
+                                  "tune_shared", "tune_mixed"])
 def test_host_path(host_paths, case):
     r = subprocess.run([host_paths, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr

@@ -224,6 +224,15 @@ void launch_qags(upc_batch* b, int choice, hipStream_t s)
                    b->d_counters, b->d_overflow, kQagsCap, b->ncu, kQagsBlockChoices[choice], s);
 }
 
+// Whether two choices launch anything differently (k_flux_qags_table fills a CU
+// with kQagsTableBlocksPerCu workgroups).
+bool qags_differ(const upc_batch* b, int c0, int c1)
+{
+  const int n0 = kQagsBlockChoices[c0], n1 = kQagsBlockChoices[c1];
+  const bool direct = b->groups > (b->h_groups > 0 ? b->share_groups : 0);
+  return direct || std::min(n0, kQagsTableBlocksPerCu) != std::min(n1, kQagsTableBlocksPerCu);
+}
+
 void launch_qags_wave(upc_batch* b, hipStream_t s)
 {
   hipLaunchKernelGGL((k_flux_qags_wave<BatchRows>), dim3(kQagsWaveBlocks), dim3(64), 0, s, batch_rows(b, 0, 0),
@@ -512,6 +521,11 @@ int upc_batch_autotune(upc_batch* b, void* stream, upc_tune* h_out)
   UPC_HIP(hipEventCreate(&e1));
   const int nj = (int)b->jobs.size();
   for (int i = 0; i < 3; ++i) {
+    t.qags_candidates[i] = kQagsBlockChoices[i];
+    if (i > 0 && !qags_differ(b, i - 1, i)) {
+      t.qags_ms[i] = t.qags_ms[i - 1];  // the same launches: not chosen before the one timed
+      continue;
+    }
     // QAGS alone: clear the counters except the integral and row totals, then time
     hipLaunchKernelGGL(k_batch_zero, dim3(1), dim3(64), 0, s, b->d_counters, 4);
     hipLaunchKernelGGL(k_batch_zero, dim3(nblk(b->ncursors, 64)), dim3(64), 0, s, b->d_counters + 8, b->ncursors);
@@ -522,7 +536,6 @@ int upc_batch_autotune(upc_batch* b, void* stream, upc_tune* h_out)
     UPC_HIP(hipEventSynchronize(e1));
     float ms = 0;
     UPC_HIP(hipEventElapsedTime(&ms, e0, e1));
-    t.qags_candidates[i] = kQagsBlockChoices[i];
     t.qags_ms[i] = ms;
   }
   // restore the overflow results (the timed passes re-ran every task)
