@@ -129,7 +129,7 @@ struct upc_batch {
   double* d_row_k = nullptr;
   double* d_row_logd = nullptr;
   int* d_row_cnt = nullptr;
-  int* d_perm = nullptr;         // rows with QAGS nodes, by job and photon energy
+  int* d_perm = nullptr;         // rows with QAGS nodes, by job and photon energy; as many again for the ordering
   int* d_hist = nullptr;         // [njobs][kRowBuckets] rows per k bucket, then their offsets in d_perm
   int* d_group_job = nullptr;    // job of each group of 64 positions in d_perm
   int* d_nsorted = nullptr;      // [njobs] rows in d_perm
@@ -250,7 +250,8 @@ int enqueue(upc_batch* b, hipStream_t s)
   hipLaunchKernelGGL(k_batch_point_rows, dim3(nblk(b->nrows * kNB1, 256)), dim3(256), 0, s, b->d_jobs, b->d_row0,
                      nj, b->nrows, b->d_row_k, b->d_row_logd, b->d_row_cnt, b->d_flux, b->d_hist, b->d_perm);
   if (b->h_groups > 0)
-    hipLaunchKernelGGL(k_row_order<BatchRows>, dim3(nblk(nhist, 4)), dim3(256), 0, s, rs, b->d_hist, (long long)nhist);
+    hipLaunchKernelGGL(k_row_order<BatchRows>, dim3(nblk(nhist, 4)), dim3(256), 0, s, rs, b->d_hist, (long long)nhist,
+                       b->d_perm + 64 * b->groups);
   launch_qags(b, b->qags_choice, s);
   launch_qags_wave(b, s);
   if (b->form != UPC_FORM_FP64) return contract_mfma(b, kMfmaTileChoices[b->mfma_choice], s);
@@ -331,7 +332,7 @@ int upc_batch_create(const upc_config* cfgs, int njobs, void* stream, upc_batch*
     BA(b->d_row_k, nr);
     BA(b->d_row_logd, nr);
     BA(b->d_row_cnt, nr);
-    BA(b->d_perm, std::max(64 * b->groups, 1LL));
+    BA(b->d_perm, std::max(2 * 64 * b->groups, 1LL));
     BA(b->d_group_job, std::max(b->groups, 1LL));
     BA(b->d_nsorted, njobs);
     BA(b->d_hist, (size_t)njobs * kRowBuckets);

@@ -1402,49 +1402,108 @@ __global__ __launch_bounds__(1024) void k_row_offsets(RS rs, int* __restrict__ o
 
 // Orders the rows of each bucket by (k, row): the order they were dropped in
 // varies from run to run, and with it the groups that expand J1 together and
-// the last bits of what they compute.  off: the buckets' ends.  One wavefront
-// per bucket (50 rows on the 1001 x 121 grid); a bucket that does not fit its
-// LDS is filled again in row order.
-constexpr int kOrderMax = 1024;
+// the last bits of what they compute.  off: the buckets' ends; spare: as long as
+// perm.  A workgroup takes four buckets, one per wavefront (50 rows on the 1001 x
+// 121 grid); a bucket of more rows (points close together) takes the workgroup,
+// up to kOrderMax of them ordered by their ranks, more by row alone: those are
+// marked in a bitmap of kOrderWindow rows at a time and read off it.  8,192 rows
+// within 0.4 % of two energies 0.13 ms, 262,144 and 2,000,000 rows of two energies
+// 0.43 and 9.0 (0.57, 2.3 and 25 when one wavefront looked through all rows for
+// those of its bucket), of calls of 1.1, 17 and 133 ms.
+constexpr int kOrderWave = 128, kOrderMax = 1024;
+constexpr int kOrderWindow = 1 << 18;
 
 template <class RS>
-__global__ __launch_bounds__(256) void k_row_order(RS rs, const int* __restrict__ off, long long nbuckets)
+__global__ __launch_bounds__(256) void k_row_order(RS rs, const int* __restrict__ off, long long nbuckets,
+                                                   int* __restrict__ spare)
 {
-  __shared__ long long kk[4][kOrderMax];
-  __shared__ int rr[4][kOrderMax];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const long long i = (long long)blockIdx.x * 4 + wv;
-  if (i >= nbuckets) return;
-  const int job = (int)(i / kRowBuckets), bucket = (int)(i - (long long)job * kRowBuckets);
-  long long r0, start;
-  const long long nrows = rs.span(job, &r0, &start);
-  if (bucket > 0) start = off[i - 1];
-  const int n = (int)(off[i] - start);
-  if (n <= 1) return;
-  if (n > kOrderMax) {
-    long long done = 0;
-    for (long long base = r0; base < r0 + nrows && done < n; base += 64) {
-      const long long r = base + lane;
-      const bool here = r < r0 + nrows && rs.row_cnt[r] > 0 && row_bucket(rs.row_k[r]) == bucket;
-      const unsigned long long m = __ballot(here);
-      const long long at = done + __popcll(m & ((1ull << lane) - 1));
-      if (here && at < n) rs.perm[start + at] = (int)r;
-      done += __popcll(m);
+  constexpr int kWords = kOrderWindow / 32;  // of the bitmap
+  __shared__ union {
+    struct {
+      long long k[kOrderMax];
+      int r[kOrderMax];
+    } one;
+    struct {
+      long long k[4][kOrderWave];
+      int r[4][kOrderWave];
+    } four;
+    unsigned bits[kWords + kWords / 32];  // a word of padding after each 32
+  } S;
+  __shared__ int wsum[4];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  // rows of bucket i and where they start in perm
+  long long r0 = 0, nrows = 0, start = 0;
+  auto bucket = [&](long long i) {
+    if (i >= nbuckets) return 0;
+    const int job = (int)(i / kRowBuckets);
+    nrows = rs.span(job, &r0, &start);
+    if (i > (long long)job * kRowBuckets) start = off[i - 1];
+    return (int)(off[i] - start);
+  };
+  // the rank of each row among the n in k, r, by every step'th thread
+  auto ranks = [&](const long long* k, const int* r, int n, int first, int step) {
+    for (int e = first; e < n; e += step) {
+      int rank = 0;
+#pragma unroll 8
+      for (int m = 0; m < n; ++m) rank += (k[m] < k[e]) | ((k[m] == k[e]) & (r[m] < r[e]));
+      rs.perm[start + rank] = r[e];
     }
-    return;
+  };
+  const long long i0 = (long long)blockIdx.x * 4;
+  int n = bucket(i0 + wv);
+  if (n > 1 && n <= kOrderWave) {
+    for (int e = lane; e < n; e += 64) {
+      const int r = rs.perm[start + e];
+      S.four.r[wv][e] = r;
+      S.four.k[wv][e] = __double_as_longlong(rs.row_k[r]);
+    }
+    wave_lds_sync();
+    ranks(S.four.k[wv], S.four.r[wv], n, lane, 64);
   }
-  for (int e = lane; e < n; e += 64) {
-    const int r = rs.perm[start + e];
-    rr[wv][e] = r;
-    kk[wv][e] = __double_as_longlong(rs.row_k[r]);
-  }
-  wave_lds_sync();
-  for (int e = lane; e < n; e += 64) {
-    const long long k = kk[wv][e];
-    const int r = rr[wv][e];
-    int rank = 0;
-    for (int m = 0; m < n; ++m) rank += kk[wv][m] < k || (kk[wv][m] == k && rr[wv][m] < r);
-    rs.perm[start + rank] = r;
+  for (int q = 0; q < 4; ++q) {
+    n = bucket(i0 + q);
+    if (n <= kOrderWave) continue;
+    __syncthreads();
+    if (n <= kOrderMax) {
+      for (int e = t; e < n; e += 256) {
+        const int r = rs.perm[start + e];
+        S.one.r[e] = r;
+        S.one.k[e] = __double_as_longlong(rs.row_k[r]);
+      }
+      __syncthreads();
+      ranks(S.one.k, S.one.r, n, t, 256);
+      continue;
+    }
+    for (int e = t; e < n; e += 256) spare[start + e] = rs.perm[start + e];
+    auto bits = [&](int word) -> unsigned& { return S.bits[word + (word >> 5)]; };
+    long long out = start;
+    for (long long w0 = r0; w0 < r0 + nrows && out < start + n; w0 += kOrderWindow) {
+      const long long left = r0 + nrows - w0;
+      const int rows = left < kOrderWindow ? (int)left : kOrderWindow;
+      const int own = ((rows + 31) / 32 + 255) / 256, first = t * own;  // the thread's words
+      for (int j = 0; j < own; ++j) bits(first + j) = 0;
+      __syncthreads();
+      for (int e = t; e < n; e += 256) {
+        const long long x = spare[start + e] - w0;
+        if (x >= 0 && x < rows) atomicOr(&bits((int)(x >> 5)), 1u << (x & 31));
+      }
+      __syncthreads();
+      int c = 0;
+      for (int j = 0; j < own; ++j) c += __popc(bits(first + j));
+      int inc = c;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int u = __shfl_up(inc, o);
+        if (lane >= o) inc += u;
+      }
+      if (lane == 63) wsum[wv] = inc;
+      __syncthreads();
+      long long at = out + inc - c;
+      for (int w = 0; w < wv; ++w) at += wsum[w];
+      for (int j = 0; j < own; ++j)
+        for (unsigned m = bits(first + j); m; m &= m - 1) rs.perm[at++] = (int)(w0 + 32 * (first + j) + __ffs(m) - 1);
+      out += wsum[0] + wsum[1] + wsum[2] + wsum[3];
+      __syncthreads();  // wsum is read
+    }
   }
 }
 

@@ -183,7 +183,7 @@ static int ensure_work(upc_ctx* c, size_t npts, size_t rows, size_t points_ff = 
   UPC_HIP(hipMalloc(&w.d_row_k, sizeof(double) * rows));
   UPC_HIP(hipMalloc(&w.d_row_logd, sizeof(double) * rows));
   UPC_HIP(hipMalloc(&w.d_row_cnt, sizeof(int) * rows));
-  UPC_HIP(hipMalloc(&w.d_perm, sizeof(int) * rows));
+  UPC_HIP(hipMalloc(&w.d_perm, sizeof(int) * 2 * rows));
   UPC_HIP(hipMalloc(&w.d_flux, sizeof(double) * rows * kNB1));
   UPC_HIP(hipMalloc(&w.d_idx, sizeof(int) * nidx));
   UPC_HIP(hipMalloc(&w.d_overflow, sizeof(long long) * nover));
@@ -254,7 +254,7 @@ static int run_flux(upc_ctx* c, int npts, int mirror_ny, hipStream_t s, const un
                      w.d_row_k, w.d_row_logd, w.d_row_cnt, w.d_flux, w.d_hist, sorted ? w.d_perm : nullptr, row_need);
   if (share)
     hipLaunchKernelGGL(k_row_order<GridRows>, dim3(nblk(kRowBuckets, 4)), dim3(256), 0, s, rs, w.d_hist,
-                       (long long)kRowBuckets);
+                       (long long)kRowBuckets, w.d_perm + w.rows_cap);
   if (share && row_need)
     hipLaunchKernelGGL(k_need_rows, dim3(nblk(nrows, 1024)), dim3(1024), 0, s, w.d_perm, w.d_counters + 6, row_need,
                        need_perm, w.d_counters + 7);

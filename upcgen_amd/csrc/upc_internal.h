@@ -49,7 +49,7 @@ struct LumiWork {
   double* d_row_k = nullptr;      // photon energy of each flux row
   double* d_row_logd = nullptr;   // log step of the row's b grid
   int* d_row_cnt = nullptr;       // number of QAGS nodes in the row
-  int* d_perm = nullptr;          // rows with QAGS nodes, ordered by photon energy
+  int* d_perm = nullptr;          // rows with QAGS nodes, ordered by photon energy; as many again for the ordering
   double* d_flux = nullptr;       // [rows][120]
   size_t idx_cap = 0, over_cap = 0;
   int* d_idx = nullptr;           // per-point calls: point indices
