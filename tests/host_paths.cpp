@@ -212,6 +212,17 @@ size_t largest_block()
   return n;
 }
 
+// Whether n draws from tables of these sizes take guides.
+void guided(int nm, int ny, int nz, int pol, long long n, int want)
+{
+  upc_config cf = config_of(1, nm, ny, nz);
+  cf.use_polarized = pol;
+  upc_ctx* ctx = context(cf);
+  CHECK(upc_sample_events(ctx, cell, cell, cell, cell, cell, 1, 0, n, cell, cell, cell, nullptr) == 0);
+  CHECK(launched("k_pdf_guides") == want);
+  upc_ctx_destroy(ctx);
+}
+
 // Whole form-factor grids on a device with `left` bytes beside the context's
 // tables: the integrand factors take what is there, and where they do not fit,
 // the kernel that needs none.
@@ -294,6 +305,8 @@ int main(int argc, char** argv)
   else if (what == "batch_full") batch(30000000, 0, 1);
   else if (what == "tune_shared") tune(1, 2, 0);
   else if (what == "tune_mixed") tune(2, 3, 4);
+  else if (what == "guided" && argc == 8)
+    guided(atoi(argv[2]), atoi(argv[3]), atoi(argv[4]), atoi(argv[5]), atoll(argv[6]), atoi(argv[7]));
   else return printf("no case %s\n", what.c_str()), 2;
   printf("ok\n");
   return 0;

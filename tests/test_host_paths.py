@@ -27,3 +27,12 @@ def host_paths(tmp_path_factory):
 def test_host_path(host_paths, case):
     r = subprocess.run([host_paths, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_large_draw_cases_take_the_guides(host_paths):
+    from test_gpu_draw_guides_large import CASES, PART
+    for nm, ny, nz, pol, n in CASES:
+        for draws, want in ((n, 1), (PART, 0)):
+            r = subprocess.run([host_paths, "guided"] + [str(v) for v in (nm, ny, nz, pol, draws, want)],
+                               capture_output=True, text=True, timeout=60)
+            assert r.returncode == 0, r.stdout + r.stderr
