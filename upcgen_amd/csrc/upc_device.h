@@ -363,21 +363,6 @@ __device__ __forceinline__ double spline_eval(const double4* __restrict__ coef, 
   return c.x + d * (c.y + d * (c.z + d * c.w));
 }
 
-// The same cubic on the estimated interval alone (no one-knot correction).
-// When v lies within rounding of a knot the estimate may name the
-// neighbouring interval; the spline is C2, so that cubic agrees at v to a
-// few ulp.  For sums of many spline values, where the exact interval choice
-// does not matter.
-__device__ __forceinline__ double spline_eval_near(const double4* __restrict__ coef, double x0, double dx,
-                                                   double inv_dx, int n, double v)
-{
-  int i = (int)((v - x0) * inv_dx);
-  i = i < 0 ? 0 : (i > n - 2 ? n - 2 : i);
-  const double4 c = coef[i];
-  const double d = v - knot(x0, dx, i);
-  return c.x + d * (c.y + d * (c.z + d * c.w));
-}
-
 __device__ __forceinline__ double spline_deriv(const double4* __restrict__ coef, double x0, double dx,
                                                double inv_dx, int n, double v)
 {
@@ -414,68 +399,6 @@ struct QK21Out {
   double result, abserr, resabs, resasc;
 };
 
-// dqk21 with the dqagse error rescaling; same summation order as QUADPACK.
-template <class F>
-__device__ __forceinline__ QK21Out qk21(const F& f, double a, double b)
-{
-  constexpr double epmach = DBL_EPSILON, uflow = DBL_MIN;
-  double fv1[10], fv2[10];
-  const double centr = 0.5 * (a + b);
-  const double hlgth = 0.5 * (b - a);
-  const double dhlgth = fabs(hlgth);
-  double resg = 0.0;
-  const double fc = f(centr);
-  double resk = kWgk[10] * fc;
-  double rabs = fabs(resk);
-#pragma unroll
-  for (int j = 1; j <= 5; ++j) {
-    const int jtw = 2 * j - 1; // 0-based index of the Fortran xgk(2j)
-    const double absc = hlgth * kXgk[jtw];
-    const double f1 = f(centr - absc);
-    const double f2 = f(centr + absc);
-    fv1[jtw] = f1;
-    fv2[jtw] = f2;
-    const double fsum = f1 + f2;
-    resg = resg + kWg[j - 1] * fsum;
-    resk = resk + kWgk[jtw] * fsum;
-    rabs = rabs + kWgk[jtw] * (fabs(f1) + fabs(f2));
-  }
-#pragma unroll
-  for (int j = 1; j <= 5; ++j) {
-    const int jtwm1 = 2 * j - 2; // xgk(2j-1)
-    const double absc = hlgth * kXgk[jtwm1];
-    const double f1 = f(centr - absc);
-    const double f2 = f(centr + absc);
-    fv1[jtwm1] = f1;
-    fv2[jtwm1] = f2;
-    const double fsum = f1 + f2;
-    resk = resk + kWgk[jtwm1] * fsum;
-    rabs = rabs + kWgk[jtwm1] * (fabs(f1) + fabs(f2));
-  }
-  const double reskh = resk * 0.5;
-  double rasc = kWgk[10] * fabs(fc - reskh);
-#pragma unroll
-  for (int j = 0; j < 10; ++j) rasc = rasc + kWgk[j] * (fabs(fv1[j] - reskh) + fabs(fv2[j] - reskh));
-  QK21Out o;
-  o.result = resk * hlgth;
-  rabs = rabs * dhlgth;
-  rasc = rasc * dhlgth;
-  double err = fabs((resk - resg) * hlgth);
-  if (rasc != 0.0 && err != 0.0) {
-    const double t15 = 200.0 * err / rasc;
-    const double sc = t15 * sqrt(t15);
-    err = rasc * (sc < 1.0 ? sc : 1.0);
-  }
-  if (rabs > uflow / (50.0 * epmach)) {
-    const double m = (epmach * 50.0) * rabs;
-    if (m > err) err = m;
-  }
-  o.abserr = err;
-  o.resabs = rabs;
-  o.resasc = rasc;
-  return o;
-}
-
 // The 21 nodes of a QK21 pass in the order the passes below visit them:
 // e = 0 the centre, e = 1..10 the Gauss abscissae xgk(2j) in (left, right)
 // pairs, e = 11..20 the Kronrod-only abscissae xgk(2j - 1) in pairs.
@@ -490,48 +413,9 @@ __device__ __forceinline__ double qk21_abscissa(int e, double centr, double hlgt
   return e == 0 ? centr : (side ? centr + absc : centr - absc);
 }
 
-// dqk21 as a rolled loop over the 21 nodes (e = 0 the centre, e = 1..10
-// the Gauss pairs, e = 11..20 the Kronrod-only pairs; qk21_abscissa): the
-// same operations in the same order as qk21() above.  fx(e, x) gives the
-// integrand at node e, abscissa x; gx(j, side) gives back the value of
-// pair j (kXgk index), side 0 (centr - absc) or 1 (centr + absc), for the
-// mean deviation once the Kronrod mean is known.
-template <class GX>
-__device__ __forceinline__ QK21Out qk21_tail(const GX& gx, double resg, double resk, double rabs, double fc,
-                                             double hlgth);
-
-template <class FX, class GX>
-__device__ __forceinline__ QK21Out qk21_core(const FX& fx, const GX& gx, double a, double b)
-{
-  const double centr = 0.5 * (a + b);
-  const double hlgth = 0.5 * (b - a);
-  double resg = 0.0, resk = 0.0, rabs = 0.0, fc = 0.0, f1 = 0.0;
-#pragma unroll 1
-  for (int e = 0; e < 21; ++e) {
-    const bool gauss = e <= 10;
-    const int p = gauss ? (e - 1) >> 1 : (e - 11) >> 1;
-    const int side = gauss ? (e - 1) & 1 : (e - 11) & 1;
-    const int xi = e == 0 ? 10 : (gauss ? 2 * p + 1 : 2 * p);
-    const double fx_e = fx(e, qk21_abscissa(e, centr, hlgth));
-    if (e == 0) {
-      fc = fx_e;
-      resk = kWgk[10] * fc;
-      rabs = fabs(resk);
-    } else if (side == 0) {
-      f1 = fx_e;
-    } else {
-      const double f2 = fx_e;
-      const double fsum = f1 + f2;
-      if (gauss) resg = resg + kWg[p] * fsum;
-      resk = resk + kWgk[xi] * fsum;
-      rabs = rabs + kWgk[xi] * (fabs(f1) + fabs(f2));
-    }
-  }
-  return qk21_tail(gx, resg, resk, rabs, fc, hlgth);
-}
-
-// The end of dqk21 once the node sums are known: the mean deviation (gx as
-// in qk21_core) and the error estimate.
+// The end of dqk21 once the node sums are known: the mean deviation, from the
+// values gx(j, side) of pair j (kXgk index) at centr - absc (side 0) and centr +
+// absc (1), and the error estimate with the dqagse rescaling.
 template <class GX>
 __device__ __forceinline__ QK21Out qk21_tail(const GX& gx, double resg, double resk, double rabs, double fc,
                                              double hlgth)
@@ -567,36 +451,15 @@ __device__ __forceinline__ QK21Out qk21_tail(const GX& gx, double resg, double r
   return o;
 }
 
-// Node e of pair j (kXgk index), side 0 or 1 (the inverse of the mapping in
-// qk21_core).
+// Node e of pair j (kXgk index), side 0 or 1 (the inverse of qk21_abscissa's mapping).
 __device__ __forceinline__ int qk21_node(int j, int side) { return (j & 1) ? j + side : 11 + j + side; }
 
-// qk21_core evaluating the integrand: the 20 off-centre values are parked
-// at fv[(2 j + side) * stride] until the mean deviation needs them.
-template <class FX>
-__device__ __forceinline__ QK21Out qk21_sum(const FX& fx, double a, double b, double* fv, int stride)
-{
-  return qk21_core(
-      [&](int e, double x) {
-        const double v = fx(e, x);
-        if (e != 0) {
-          const int gauss = e <= 10;
-          const int p = gauss ? (e - 1) >> 1 : (e - 11) >> 1;
-          const int side = gauss ? (e - 1) & 1 : (e - 11) & 1;
-          const int xi = gauss ? 2 * p + 1 : 2 * p;
-          fv[(2 * xi + side) * stride] = v;
-        }
-        return v;
-      },
-      [&](int j, int side) { return fv[(2 * j + side) * stride]; }, a, b);
-}
-
-// qk21_core over values already evaluated (node e's value at v[e * stride]),
-// as two loops over pairs: the Gauss pairs (nodes 1..10), then the
-// Kronrod-only pairs (11..20), summed in qk21_core's order.  (qk21_core's
-// loop over the 21 nodes branches on each node's kind and waits for a scalar
-// load of its weights on every trip.)  The Gauss loop is unrolled (its ten
-// loads issued together); unrolling the second as well costs the QAGS kernel
+// dqk21 over values already evaluated (node e's value at v[e * stride]), in
+// QUADPACK's summation order, as two loops over pairs: the Gauss pairs (nodes
+// 1..10), then the Kronrod-only pairs (11..20).  (One loop over the 21 nodes
+// branches on each node's kind and waits for a scalar load of its weights on
+// every trip.)  The Gauss loop is unrolled (its ten loads issued together);
+// unrolling the second as well costs the QAGS kernel
 // a spilled VGPR.
 __device__ __forceinline__ QK21Out qk21_stored(const double* v, int stride, double a, double b)
 {
@@ -620,13 +483,6 @@ __device__ __forceinline__ QK21Out qk21_stored(const double* v, int stride, doub
     rabs = rabs + kWgk[2 * p] * (fabs(f1) + fabs(f2));
   }
   return qk21_tail([&](int j, int side) { return v[qk21_node(j, side) * stride]; }, resg, resk, rabs, fc, hlgth);
-}
-
-// dqk21 of f on [a, b] through qk21_sum.
-template <class F>
-__device__ __forceinline__ QK21Out qk21_lds(const F& f, double a, double b, double* fv, int stride)
-{
-  return qk21_sum([&](int, double x) { return f(x); }, a, b, fv, stride);
 }
 
 // dqelg (Wynn epsilon) on the 1-based table of a store (ep, set_ep) and its

@@ -138,7 +138,7 @@ __device__ __forceinline__ int row_bucket(double k)
 //
 // The spline record is a dependent load from a 32 MB table: it is issued
 // first and J1 (independent ALU work) runs while it is in flight.  The
-// interval is the rounded estimate alone, as in spline_eval_near: within
+// interval is the rounded estimate alone: within
 // rounding of a knot the neighbouring cubic agrees to a few ulp.
 //
 // BR fixes J1's branch: 0 lets J1 choose (x <= 8 or not), 1 and 2 take the
@@ -327,7 +327,6 @@ struct GridRows {
     get(overflow_id(id), ft);
     return true;
   }
-  __device__ int job_of(int) const { return 0; }
   __device__ RowJob params(int) const { return job; }
   __device__ void failed(int) const {}
   __device__ void get(long long t, FluxTask* ft) const
@@ -1254,7 +1253,7 @@ __global__ __launch_bounds__(kQagsBlock) void k_flux_qags_team(TS ts, double* __
 // rerun from the start here, one wavefront per integral, with the reference's
 // 1000-interval workspace in LDS.  Lanes 0..41 evaluate the 42 nodes of a
 // step (both halves) at once; lane 0 sums each pass in QK21's order (the same
-// qk21_core as the fast kernel) and runs the dqagse state machine, so the
+// qk21_stored as the fast kernel) and runs the dqagse state machine, so the
 // serial part of a step is LDS work and one sum per pass.
 constexpr int kQagsWaveBlocks = 1024;  // workgroups of the overflow kernel (36.5 KB LDS each)
 
