@@ -25,7 +25,7 @@ namespace upc {
 // that need no spline.  1001 x 121 Pb-Pb: 0.85 ms
 // (mode 1), 1.29 (mode 2), 1.09 (mode 4, polarised); 1.29, 1.62 and 1.45 with
 // two exponentials per node, scaled square roots and interval clamps of 64 bits
-// at 96 VGPRs (now 68).
+// at 96 VGPRs (now 74).
 // The pairs of a point are cut into kLumiParts runs that are summed apart and
 // then in order, so one wavefront, four and eight give the same bits.
 // ---------------------------------------------------------------------------
@@ -108,7 +108,6 @@ __device__ __forceinline__ void node_k(double tb, double ss, bool breakup, doubl
 
 // Job resolvers: the job and first point of a block of `points` points.
 struct SingleLumi {
-  static constexpr int kWavesPerEu = 5;  // register budget of k_lumi_fp64 (waves per SIMD)
   LumiView v;
   __device__ void get(int blk, int points, LumiView* out, int* p0) const
   {
@@ -119,7 +118,6 @@ struct SingleLumi {
 
 // Contraction job resolver: blk0[j] = first block of job j for this wave count.
 struct BatchLumi {
-  static constexpr int kWavesPerEu = 4;  // register budget of k_lumi_fp64 (waves per SIMD)
   const BatchJob* __restrict__ jobs;
   const int* __restrict__ blk0;
   int njobs;
@@ -392,11 +390,13 @@ __device__ __forceinline__ void lumi_fp64_body(const LumiView& v, int p0, LumiSm
 
 // WAVES / WPP points per block; the resolver maps the block to its job (all
 // threads of a block take the same branch, so the barriers are uniform).
-// JR::kWavesPerEu budgets the registers: for one grid a fifth wave per SIMD
-// hides more of the gathers' latency, while the batch's mostly polarised jobs
-// spill at that budget and keep 4.
+// 74 to 76 VGPRs without spills with one wavefront per point (52 to 56 with a
+// workgroup per point), alike for budgets of 4 to 6 waves per SIMD; LDS admits 5
+// of four-wave workgroups.
+constexpr int kLumiWavesPerEu = 5;
+
 template <int WAVES, int WPP, class JR>
-__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(JR::kWavesPerEu))) void k_lumi_fp64(
+__global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(kLumiWavesPerEu))) void k_lumi_fp64(
     JR jr)
 {
   __shared__ LumiSmem<WAVES, WPP> sm;
