@@ -12,12 +12,12 @@ ROOT = os.path.dirname(HERE)
 @pytest.fixture(scope="module")
 def host_paths(tmp_path_factory):
     from upcgen_amd import LIB_PATH
+    from upcgen_amd.build import HIPCC
     exe = str(tmp_path_factory.mktemp("host_paths") / "host_paths")
-    rocm = os.path.dirname(os.path.dirname(os.path.realpath("/opt/rocm/bin/hipcc")))
-    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include", "-I/opt/rocm/include",
-                    f"-I{ROOT}/include", os.path.join(HERE, "host_paths.cpp"), "-o", exe, LIB_PATH, "-rdynamic",
-                    "-L/opt/rocm/lib", f"-Wl,-rpath,{os.path.dirname(LIB_PATH)}:/opt/rocm/lib",
-                    "-Wl,--allow-shlib-undefined"], check=True)
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include", f"-I{ROOT}/include",
+                    os.path.join(HERE, "host_paths.cpp"), "-o", exe, LIB_PATH, "-rdynamic", f"-L{rocm}/lib",
+                    f"-Wl,-rpath,{os.path.dirname(LIB_PATH)}:{rocm}/lib", "-Wl,--allow-shlib-undefined"], check=True)
     return exe
 
 

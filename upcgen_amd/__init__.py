@@ -503,8 +503,8 @@ def mixed_systems_jobs(seed=2024, n=64, polarized=1, flux_point=0):
 
 class Batch:
     """Many configurations whose luminosity grids run as one launch sequence
-    (one persistent QAGS launch, one contraction launch), optionally replayed
-    from a captured hipGraph."""
+    (the QAGS launches and the contraction shared by all jobs), optionally
+    replayed from a captured hipGraph."""
 
     def __init__(self, configs, stream=None):
         import torch

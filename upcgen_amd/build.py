@@ -34,7 +34,8 @@ HIPFLAGS = COMMON + [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-X
                      "-munsafe-fp-atomics", "-Wno-unused-command-line-argument"]
 # The QAGS kernels run at their register budget: without this the compiler lifts
 # address and constant computations out of their long loops and spills them
-# (k_flux_qags_team 164 -> 122 VGPRs, k_flux_qags_table 60 -> 0 spilled).
+# (k_flux_qags_team 155 -> 122 VGPRs, k_flux_qags 157 -> 127; k_flux_qags_table 47
+# -> 0 spilled for a grid's rows, 63 -> 12 for a batch's).
 QAGS_FLAGS = ["-mllvm", "-disable-machine-licm"]
 QAGS_SOURCES = {"upc_flux_lumi.hip", "upc_batch.hip", "upc_noalloc.hip"}
 

@@ -367,7 +367,7 @@ struct GridRows {
 // same bits as a lane evaluating its own nodes.
 //
 // The LDS table (13,440 B per wavefront) sets the occupancy: 3 workgroups
-// of 4 wavefronts per CU, 168 VGPRs per lane.
+// of 4 wavefronts per CU (127 VGPRs would admit 4).
 //
 // stats: [0] integrand evaluations, [1] integrals with ier != 0, [2]
 // overflow count.

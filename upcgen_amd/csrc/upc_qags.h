@@ -11,7 +11,8 @@
 // table) go through a store policy:
 //  - QagsSmallStore<CAP> (fast path): per-lane private arrays, intervals
 //    packed into 32 bits, the order list in 4-bit fields of one register;
-//  - QagsBigStore (the reference's 1000-interval workspace, global memory).
+//  - QagsLdsStore<CAP>: its first entries in LDS, a column per lane;
+//  - QagsBigStore (the reference's 1000-interval workspace, in LDS).
 // Every flux integral runs over q in [0, 10]; bisection keeps each interval a
 // dyadic piece [10 m 2^-L, 10 (m + 1) 2^-L] of it, and those end points (and
 // the midpoints 0.5 (a + b) that dqagse computes) are exact in FP64, so the
@@ -149,8 +150,8 @@ struct QagsLdsStore : QagsSmallStore<CAP> {
   }
 };
 
-// The reference's workspace: limit 1000, FP64 end points, one per lane in
-// global memory.
+// The reference's workspace: limit 1000, FP64 end points (k_flux_qags_wave: one
+// per workgroup, in LDS).
 struct QagsBigArrays {
   double alist[kQagsLimit], blist[kQagsLimit], rlist[kQagsLimit], elist[kQagsLimit];
   int iord[kQagsLimit];

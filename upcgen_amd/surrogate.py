@@ -1,6 +1,9 @@
 """Learned surrogate of log L(M, Y; system): data generation by the FP64 GPU
 quadrature, training by the library's own HIP kernels, and serving as the
-UPC_FORM_SURROGATE luminosity form (with quadrature fallback).
+UPC_FORM_SURROGATE luminosity form (with quadrature fallback).  A whole
+form-factor grid is faster by FORM_FP64 (1001 x 121: 6.1 against 8.4 ms): its rows
+share their integrand factors, and the bins the network leaves to the quadrature
+take most of that work again.
 
 Training distribution (one system per context, points drawn per system):
 Z ~ U[8, 92], A = round(2.5 Z), sqrt(s_NN) log-uniform in [0.2, 40] TeV,
