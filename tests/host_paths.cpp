@@ -18,6 +18,7 @@ namespace {
 
 size_t capacity = ~size_t(0), live = 0;  // bytes of the device
 bool pool_fails = false;                 // hipMallocAsync finds no memory
+long clear_threads = 0, clear_counters = 0;  // of the last k_batch_clear, a thread per counter
 hipError_t last_error = hipSuccess;
 std::map<void*, size_t> blocks;
 std::vector<std::string> launches;
@@ -80,9 +81,13 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shmem, hip
   *grid = config.grid, *block = config.block, *shmem = config.shmem, *stream = config.stream;
   return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, hipStream_t)
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3 block, void** args, size_t, hipStream_t)
 {
   launches.push_back(kernels()[f]);
+  if (launches.back().find("k_batch_clear") != std::string::npos) {
+    clear_threads = (long)grid.x * block.x;
+    clear_counters = *(const int*)args[1];
+  }
   return hipSuccess;
 }
 
@@ -269,6 +274,16 @@ void batch(size_t left, int table_launches, int direct_launches)
   CHECK(live == 0);
 }
 
+// The largest job: more work cursors than row buckets, all of them cleared.
+void batch_large()
+{
+  const upc_config job = config_of(0, 4000, 4000, 50);
+  upc_batch* b = nullptr;
+  CHECK(upc_batch_create(&job, 1, nullptr, &b) == 0);
+  CHECK(clear_counters > 10240 && clear_threads >= clear_counters);
+  CHECK(upc_batch_destroy(b) == 0);
+}
+
 // Tuning times the launch shapes that differ: three for the kernel without
 // factors, two for the one with them (two workgroups fill a CU).
 void tune(int njobs, int table_launches, int direct_launches)
@@ -303,6 +318,7 @@ int main(int argc, char** argv)
   else if (what == "batch") batch(0, 1, 1);
   else if (what == "batch_short") batch(240000000, 4, 1);  // a quarter
   else if (what == "batch_full") batch(30000000, 0, 1);
+  else if (what == "batch_large") batch_large();
   else if (what == "tune_shared") tune(1, 2, 0);
   else if (what == "tune_mixed") tune(2, 3, 4);
   else if (what == "guided" && argc == 8)

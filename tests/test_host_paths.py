@@ -14,7 +14,7 @@ def host_paths(tmp_path_factory):
     from upcgen_amd import LIB_PATH
     from upcgen_amd.build import HIPCC
     exe = str(tmp_path_factory.mktemp("host_paths") / "host_paths")
-    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    rocm = os.path.dirname(os.path.dirname(os.path.realpath(HIPCC)))
     subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", f"-I{rocm}/include", f"-I{ROOT}/include",
                     os.path.join(HERE, "host_paths.cpp"), "-o", exe, LIB_PATH, "-rdynamic", f"-L{rocm}/lib",
                     f"-Wl,-rpath,{os.path.dirname(LIB_PATH)}:{rocm}/lib", "-Wl,--allow-shlib-undefined"], check=True)
@@ -22,7 +22,7 @@ def host_paths(tmp_path_factory):
 
 
 @pytest.mark.parametrize("case", ["draws", "draws_full", "pairs", "pairs_full",
-                                  "grid", "grid_short", "grid_full", "batch", "batch_short", "batch_full",
+                                  "grid", "grid_short", "grid_full", "batch", "batch_short", "batch_full", "batch_large",
                                   "tune_shared", "tune_mixed"])
 def test_host_path(host_paths, case):
     r = subprocess.run([host_paths, case], capture_output=True, text=True, timeout=60)

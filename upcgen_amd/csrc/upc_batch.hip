@@ -200,8 +200,8 @@ void enqueue_rows(upc_batch* b, hipStream_t s)
 {
   const int nj = (int)b->jobs.size();
   const long nhist = (long)nj * kRowBuckets;
-  hipLaunchKernelGGL(k_batch_clear, dim3(nblk(nhist, 256)), dim3(256), 0, s, b->d_counters, 8 + b->ncursors,
-                     b->d_job_failed, nj, b->d_hist, nhist);
+  hipLaunchKernelGGL(k_batch_clear, dim3(nblk(std::max(nhist, 8L + b->ncursors), 256)), dim3(256), 0, s, b->d_counters,
+                     8 + b->ncursors, b->d_job_failed, nj, b->d_hist, nhist);
   hipLaunchKernelGGL(k_batch_points, dim3(nblk(b->npts, 256)), dim3(256), 0, s, b->d_jobs, b->d_pt0, nj,
                      b->npts, b->d_pts);
   hipLaunchKernelGGL(k_batch_rows, dim3(nblk(b->nrows, 256)), dim3(256), 0, s, b->d_jobs, b->d_row0, nj,
